@@ -55,9 +55,10 @@ struct ActQ8 {
     float* xs32;     // [p][cols/32]   per-32 sums (amd64 order)
     float* xs16;     // [p][cols/16]   per-16 sums (amd64 order; Q6_K scales them by 32)
     // Batches of more than kTiledMinP rows also get the q8 values as f16 in
-    // the matrix-core operand layout of the batched Q4_K kernel:
+    // the matrix-core operand layout of the batched kernels:
     // [block][16-token tile][lane k][group g][token c][8 halves], the eight
-    // halves being q8perm's bytes 32 k + 8 g .. + 7 of token 16 tile + c.
+    // halves being q8perm's bytes 32 k + 8 g .. + 7 of token 16 tile + c, in
+    // the order b16_slot gives them.
     // Tokens p .. 16 tiles - 1 hold zeros.  Null for smaller batches.
     uint16_t* b16t;
     float* xs32t;    // xs32 of the same batches as [block][tile][lane k][token c]
@@ -65,6 +66,11 @@ struct ActQ8 {
     int cols, p;
 };
 constexpr int kTiledMinP = 16;
+// Place, among the eight halves, of byte kappa % 8: bytes 0, 2, 1, 3 of each
+// weight dword, the order in which two masks of the dword give the pairs.
+__host__ __device__ __forceinline__ int b16_slot(int kappa) {
+    return (kappa & 4) | ((kappa & 1) << 1) | ((kappa >> 1) & 1);
+}
 size_t act_bytes(int cols, int p);
 void act_carve(void* base, int cols, int p, ActQ8* a);
 int launch_q8k_prep(const float* d_x, int cols, int p, const ActQ8& a, hipStream_t s);

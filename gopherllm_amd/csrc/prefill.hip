@@ -336,39 +336,45 @@ __device__ __forceinline__ void sb_scale_min(const u4v h, int j, uint32_t& sc, u
     }
 }
 
-// --- more than 16 activation rows: operands staged once per workgroup -----
-// A workgroup of eight waves covers 64 weight rows x 64 tokens.  Per block it
-// stages in LDS, double-buffered:
-//   * the 64 rows' A operands, sc_j * q4 as f16, dequantised once for the
-//     whole workgroup: wave w copies the nibbles of AVX2 lanes 4 (w % 2) ..
-//     + 3 of rows 16 (w / 2) .. + 15, and those rows' headers, into LDS two
-//     blocks ahead and dequantises them itself, lane (row, k) the 16 nibble
-//     bytes of AVX2 lane k (16 rows per wave keep its LDS writes on distinct
-//     banks);
-//   * the four 16-token tiles' B operands, q8 as f16 written by the quantiser
-//     in this operand layout, copied global -> LDS one block ahead;
-//   * the rows' d, dmin and mins and the tokens' xscale and xsums.
-// Every global read is a direct global -> LDS copy, so the waits are exact
-// vmcnt counts of this wave's own copies.  Both operand tiles are laid out
-// [tile][lane k][group g][row or token c][8 halves], so each MFMA operand
-// read of a wave is 1 KB of consecutive LDS.  Wave w owns rows 16 (w % 4) ..
-// + 15 and the two token tiles 2 (w / 4), 2 (w / 4) + 1, sharing its A
-// operand between them; per lane k and tile it runs q4kDotQ8KRow's two chains
-// on the exact MFMA lane sums, in block order:
+// --- more than 16 activation rows: one pair of AVX2 lanes per wave ---------
+// A workgroup of sixteen waves covers 64 weight rows x 64 tokens.  The eight
+// AVX2 lanes k of a row never meet before the final tree, so the waves split
+// by lane: wave (rq, kp) = (w >> 2, w & 3) owns rows 16 rq .. + 15, all 64
+// tokens and the lanes kp and kp + 4, the first pair the tree adds.  A weight
+// nibble then belongs to one wave: it is dequantised once, in that wave's
+// registers, straight into the MFMA operand, with no f16 copy of the weights
+// in LDS, and 64 accumulator registers leave room for four waves per SIMD.
+// The products take the activations as the A operand and the weights as B,
+// so D has token 16 tt + 4g + i in register i and weight row 16 rq + c in
+// lane (g, c): a row's factors are one register per lane, and the stores run
+// along the rows.  The two outer products of a block, m * xsum and
+// d * xscale, come from v_mfma_f32_16x16x1 with K = 1: one exact float32
+// product per output, rounded once, as the VALU's (a zero product may lose
+// its sign, which a chain that starts at +0 does not show).  Four 16-token
+// tiles are its four blocks, so an operand is one register and one dword of
+// LDS per lane.  Left to the VALU are the two chain steps per output:
 //   accF = fma(I, d * xscale, accF); accM = fma(dmin, m * xsum, accM).
+// Per block the workgroup stages the token tiles' B16 operands, xsums and
+// xscales in LDS one block ahead, and each wave its own nibbles and headers
+// two blocks ahead (they come from HBM), all by direct copies; one barrier
+// per block.  The block loop is unrolled by two, so every LDS address is a
+// lane constant plus an immediate.
+// Measured at 14336 x 4096 x 512 (with the 9.5 us quantiser launch): 261 us
+// for the kernel before it, which staged the dequantised f16 weights in LDS
+// and ran all eight lanes of a 16 x 32 tile in a wave (two waves per SIMD,
+// LDS traffic 370 KB per block), 195 us with eight waves of 32 rows x 64
+// tokens (two per SIMD), 202 us with eight waves of 16 rows x 128 tokens, 183
+// us like this.  What is left is issue: per wave and block 64 chain steps, 37
+// VALU operations of dequantisation and 11 matrix instructions, which hardly
+// overlap the VALU on this part (a 16x16x32 f16 MFMA and four fmas take 30
+// cycles at four waves per SIMD, the MFMA alone 20).
 constexpr int kTlRows = 64, kTlTok = 64;
 
-constexpr int kTlMStride = 80;     // floats per sub-block row of m: writes on distinct banks
-struct TlStage {
-    uint8_t a16[4 * 8 * 4 * 256];  // [row group][lane k][group g][row c][8 halves]
+struct LnStage {
     uint8_t b16[4 * 8 * 4 * 256];  // [token tile][lane k][group g][token c][8 halves]
-    float m[8][kTlMStride];        // [sub-block k][row] 6-bit min
     float xsum[4][8][16];          // [token tile][lane k][token c]
-    float d[kTlRows], dmin[kTlRows], xs[kTlTok];
-};
-struct TlRaw {                     // one block of the 64 rows as stored, per wave
-    uint8_t nib[8][64][16];        // [wave][lane: row 16 (w / 2) + lane / 4, lane k 4 (w % 2) + lane % 4]
-    uint8_t hdr[8][16][16];        // [wave][row 16 (w / 2) + r]: d, dmin, 12 scale bytes
+    float xs[kTlTok];
+    uint8_t raw[16][48][16];       // [wave]: nibbles [lane kp, kp + 4][row c], headers [row c]
 };
 
 // Direct global -> LDS copies addressed by a wave-uniform base and a 32-bit
@@ -384,94 +390,6 @@ __device__ __forceinline__ void lds_copy4_s(const void* sbase, uint32_t voff, ui
                  :
                  : "v"(voff), "s"(sbase), "s"(lds_dst)
                  : "memory", "m0");
-}
-
-// Block b's token operands into S: 32 one-KB pieces of B (four per wave),
-// the four tiles' xsums (waves 0, 1) and the 64 xscales (wave 2).  Issues 5
-// copies on waves 0-2 and 4 on the others.
-__device__ __forceinline__ void tl_copy_tokens(const PfArgs& a, int w, int lane, int tile0, int tok0,
-                                               int b, TlStage& S) {
-    const int cols = a.blocks * 256;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int ch = 4 * w + i, tt = ch >> 3, piece = ch & 7;
-        const int gt = min(tile0 + tt, a.act.tiles - 1);
-        const uint8_t* base = (const uint8_t*)a.act.b16t + ((size_t)b * a.act.tiles + gt) * 8192 + piece * 1024;
-        lds_copy16_s(base, 16 * lane, lds_addr(S.b16 + tt * 8192 + piece * 1024));
-    }
-    if (w < 2) {
-        const int gt = min(tile0 + 2 * w + (lane >> 5), a.act.tiles - 1);
-        lds_copy16_s(a.act.xs32t, (uint32_t)(((size_t)b * a.act.tiles + gt) * 512 + 16 * (lane & 31)),
-                     lds_addr(&S.xsum[2 * w][0][0]));
-    } else if (w == 2) {
-        lds_copy4_s(a.act.xscale + b, (uint32_t)min(tok0 + lane, a.p - 1) * a.blocks * 4,
-                    lds_addr(&S.xs[0]));
-    }
-}
-
-// Block b of this wave's rows into R: lane (row 16 (w / 2) + lane / 4, lane
-// k = 4 (w % 2) + lane % 4) copies 16 nibble bytes, lanes 0-15 the rows'
-// headers.  Two copies.  noff / hoff: this lane's 32-bit offsets of its
-// nibble chunk and header row (the launcher checks that rows * rb < 2^32).
-__device__ __forceinline__ void tl_copy_raw(const PfArgs& a, int w, int lane, uint32_t noff,
-                                            uint32_t hoff, int b, TlRaw& R) {
-    lds_copy16_s(a.w + q4k_nib_off(a.blocks, b), noff, lds_addr(&R.nib[w][0][0]));
-    if (lane < 16) lds_copy16_s(a.w + q4k_hdr_off(b), hoff, lds_addr(&R.hdr[w][0][0]));
-}
-
-// Dequantisation of this wave's part of one block from R into S, in parts
-// that the kernel interleaves with the MFMA chains: A operands sc_j * q4
-// (f16), the rows' mins (lane k: sub-block k), d and dmin.
-struct TlDq {
-    u4v nib;
-    uint32_t sc03, sc47;
-};
-
-__device__ __forceinline__ void tl_dq_begin(int w, int lane, const TlRaw& R, TlDq& q) {
-    q.nib = *(const u4v*)&R.nib[w][lane][0];
-    const u4v h = *(const u4v*)&R.hdr[w][lane >> 2][0];
-    // getScaleMinK4 (simd.go:1672-1677) for all eight sub-blocks at once, one
-    // byte each: j < 4 from s03 / s47, j >= 4 from s811 and their top bits
-    q.sc03 = h.y & 0x3f3f3f3fu;
-    q.sc47 = (h.w & 0x0f0f0f0fu) | ((h.y >> 2) & 0x30303030u);
-}
-
-// nibble dword sg: sub-blocks 2 sg (low nibbles) and 2 sg + 1 (high nibbles)
-__device__ __forceinline__ void tl_dq_part(int w, int lane, int sg, const TlDq& q, TlStage& S) {
-    const int c = lane >> 2, k = 4 * (w & 1) + (lane & 3), rg = w >> 1;
-    typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-    const h2v m1024 = {(_Float16)-1024.0f, (_Float16)-1024.0f};
-    // scale bytes 2 (sg & 1) and 2 (sg & 1) + 1 of sc03 / sc47 as (1024 + sc)
-    const uint32_t src = sg < 2 ? q.sc03 : q.sc47;
-    const uint32_t sel_lo = (sg & 1) ? 0x04020402u : 0x04000400u;
-    const uint32_t sel_hi = (sg & 1) ? 0x04030403u : 0x04010401u;
-    const h2v pl = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x64646464u, src, sel_lo));
-    const h2v ph = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x64646464u, src, sel_hi));
-    const h2v sl = pl + m1024, sh = ph + m1024;  // exact small integers
-    const h2v nl = sl * m1024, nh = sh * m1024;  // exact: at most 64512
-    const h8v av = dequant_a(q.nib[sg], __builtin_bit_cast(uint32_t, sl), __builtin_bit_cast(uint32_t, nl),
-                             __builtin_bit_cast(uint32_t, sh), __builtin_bit_cast(uint32_t, nh));
-    *(h8v*)(S.a16 + ((rg * 8 + k) * 4 + sg) * 256 + c * 16) = av;
-}
-
-// the rows' mins (lane k: sub-block k, same packing as the scales), d, dmin;
-// the header is read again from R, which the next copies overwrite only
-// after the workgroup barrier
-__device__ __forceinline__ void tl_dq_end(int w, int lane, const TlRaw& R, TlStage& S) {
-    const int c = lane >> 2, k = 4 * (w & 1) + (lane & 3), lr = 16 * (w >> 1) + c;
-    const u4v h = *(const u4v*)&R.hdr[w][c][0];
-    const uint32_t msrc = k < 4 ? h.z & 0x3f3f3f3fu : ((h.w >> 4) & 0x0f0f0f0fu) | ((h.z >> 2) & 0x30303030u);
-    S.m[k][lr] = (float)((msrc >> (8 * (k & 3))) & 63u);
-    if (k == 0) S.d[lr] = f16_bits_to_f32(h.x & 0xffffu);
-    if (k == 1) S.dmin[lr] = f16_bits_to_f32(h.x >> 16);
-}
-
-__device__ __forceinline__ void tl_dequant(int w, int lane, const TlRaw& R, TlStage& S) {
-    TlDq q;
-    tl_dq_begin(w, lane, R, q);
-#pragma unroll
-    for (int sg = 0; sg < 4; sg++) tl_dq_part(w, lane, sg, q, S);
-    tl_dq_end(w, lane, R, S);
 }
 
 // Workgroup -> tile map.  Workgroup i runs on XCD i % 8 (round robin); the
@@ -498,9 +416,39 @@ static TlMap tl_map(int rows, int p) {
     return m;
 }
 
-__global__ __launch_bounds__(512) void prefill_q4k_tiled_kernel(PfArgs a, TlMap mp) {
-    __shared__ __align__(16) TlStage st[2];
-    __shared__ __align__(16) TlRaw raw[2];
+typedef _Float16 h2v __attribute__((ext_vector_type(2)));
+typedef float f16v __attribute__((ext_vector_type(16)));
+
+// One nibble dword as eight f16 values sc_lo * low, sc_hi * high in the
+// element order of B16 (bytes 0, 2, 1, 3).  A masked nibble pair under f16
+// exponent bits is 1024 + q (bits 0-3) or 1024 + 16 q (bits 4-7), so with
+// s = {sc_lo, sc_hi / 16} and n = -1024 s the fma is exact.
+struct NibMasks {  // held in registers: a v_and_or_b32 takes no two literals
+    uint32_t lo, hi, exp;
+};
+__device__ __forceinline__ NibMasks nib_masks() {
+    NibMasks m{0x000f000fu, 0x00f000f0u, 0x64006400u};
+    asm("" : "+s"(m.lo), "+s"(m.hi), "+v"(m.exp));
+    return m;
+}
+__device__ __forceinline__ h8v dequant_nib(uint32_t w, h2v s, h2v n, const NibMasks& m) {
+    const uint32_t v = w >> 8;
+    const h2v p0 = __builtin_bit_cast(h2v, (w & m.lo) | m.exp), p1 = __builtin_bit_cast(h2v, (v & m.lo) | m.exp);
+    const h2v p2 = __builtin_bit_cast(h2v, (w & m.hi) | m.exp), p3 = __builtin_bit_cast(h2v, (v & m.hi) | m.exp);
+    const h2v sl = {s[0], s[0]}, nl = {n[0], n[0]}, sh = {s[1], s[1]}, nh = {n[1], n[1]};
+    const h2v a0 = __builtin_elementwise_fma(p0, sl, nl), a1 = __builtin_elementwise_fma(p1, sl, nl);
+    const h2v a2 = __builtin_elementwise_fma(p2, sh, nh), a3 = __builtin_elementwise_fma(p3, sh, nh);
+    return h8v{a0[0], a0[1], a1[0], a1[1], a2[0], a2[1], a3[0], a3[1]};
+}
+
+// A chain step ends here: the compiler may not sink it past this point.
+__device__ __forceinline__ void pin4(float (&v)[4]) {
+    asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+}
+
+__global__ __launch_bounds__(1024) void prefill_q4k_lanes_kernel(PfArgs a, TlMap mp) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t dyn[];
+    LnStage* const st = (LnStage*)dyn;
     const int id = blockIdx.x, xcd = id & 7, local = id >> 3;
     const int lt = local % mp.tg_size, lrow = local / mp.tg_size;
     const int ttile = (xcd % mp.h) * mp.tg_size + lt, rtile = (xcd / mp.h) * mp.rg_size + lrow;
@@ -508,137 +456,182 @@ __global__ __launch_bounds__(512) void prefill_q4k_tiled_kernel(PfArgs a, TlMap 
     const int row0 = rtile * kTlRows, tok0 = ttile * kTlTok, tile0 = tok0 / 16;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 4, c = lane & 15;
-    const int rg = w & 3, tg = w >> 2;
+    const int kp = w & 3, rq = w >> 2;
     const int nb = a.blocks;
-    const uint32_t noff = (uint32_t)min(row0 + 16 * (w >> 1) + (lane >> 2), a.rows - 1) * (uint32_t)a.rb +
-                          16 * (4 * (w & 1) + (lane & 3));
-    const uint32_t hoff = (uint32_t)min(row0 + 16 * (w >> 1) + (lane & 15), a.rows - 1) * (uint32_t)a.rb;
 
-    float accF[2][8][4], accM[2][8][4];
-#pragma unroll
-    for (int n = 0; n < 2; n++)
-#pragma unroll
-        for (int k = 0; k < 8; k++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) accF[n][k][i] = accM[n][k][i] = 0.0f;
+    // Copies of one block's tokens: two 1 KB pieces of B16 (wave w: tile w / 4,
+    // lanes k 2 (w % 4), + 1), the tiles' xsums (waves 0, 1) and xscales
+    // (wave 2).  Past the end they stay on the last block, so that the counts
+    // of copies in flight are constants.
+    const int last = a.act.tiles - 1;
+    const size_t bstep = (size_t)a.act.tiles * 8192;
+    const uint8_t* bsrc = (const uint8_t*)a.act.b16t + (size_t)min(tile0 + rq, last) * 8192 + 2048 * kp;
+    const uint32_t xoff = w < 2 ? (uint32_t)(min(tile0 + 2 * w + (lane >> 5), last) * 512 + 16 * (lane & 31))
+                                : (uint32_t)min(tok0 + lane, a.p - 1) * nb * 4;
+    auto copy_tokens = [&](int b, LnStage& S) __attribute__((always_inline)) {
+        b = min(b, nb - 1);
+        const uint8_t* src = bsrc + b * bstep;
+        const uint32_t dst = lds_addr(S.b16 + rq * 8192 + 2048 * kp);
+        lds_copy16_s(src, 16 * lane, dst);
+        lds_copy16_s(src + 1024, 16 * lane, dst + 1024);
+        if (w < 2) lds_copy16_s(a.act.xs32t + (size_t)b * a.act.tiles * 128, xoff, lds_addr(&S.xsum[2 * w][0][0]));
+        else if (w == 2) lds_copy4_s(a.act.xscale + b, xoff, lds_addr(&S.xs[0]));
+    };
+    // The wave's nibbles, lane k = kp + 4 kc of row 16 rq + c in lanes 0-31
+    // (kc = 0, 1), and headers, row c in lanes 32-47, of one block after the
+    // other (roff: this lane's source offset of the next one)
+    const int kc = min(lane >> 4, 2);
+    uint32_t roff = (uint32_t)min(row0 + 16 * rq + c, a.rows - 1) * (uint32_t)a.rb +
+                    (kc < 2 ? 16 * nb + 16 * (kp + 4 * kc) : 0);
+    const uint32_t rstep = kc < 2 ? 128 : 16;
+    auto copy_raw = [&](int b, LnStage& S) __attribute__((always_inline)) {
+        if (lane < 48) lds_copy16_s(a.w, roff, lds_addr(&S.raw[w][0][0]));
+        if (b < nb - 1) roff += rstep;
+    };
+    // This lane's weight row 16 rq + c in one block: factors, mins of the two
+    // lanes k, f16 scales of sub-blocks 2g, 2g + 1 (getScaleMinK4,
+    // simd.go:1672-1677: six bits of byte 4 + j, or four bits of byte 12 + j
+    // - 4 under the top two of byte 4 + j - 4) and the nibble dwords.  The
+    // wave copied them itself, so they are read as soon as its own copies
+    // have landed.
+    struct Row {
+        float d, dm, mn[2];
+        h2v s, n;  // {sc_2g, sc_(2g + 1) / 16} and -1024 times them
+        uint32_t nd[2];
+    };
+    const uint32_t sel = g < 2 ? 4 : 12, sh0 = 16 * (g & 1), low = g < 2 ? 0x3f3fu : 0x0f0fu;
+    const h2v one16 = {(_Float16)1.0f, (_Float16)0.0625f}, off16 = {(_Float16)-1024.0f, (_Float16)-64.0f};
+    const h2v m1024 = {(_Float16)-1024.0f, (_Float16)-1024.0f};
+    auto row_of = [&](const LnStage& S) __attribute__((always_inline)) {
+        Row r;
+        const u4v h = *(const u4v*)&S.raw[w][32 + c][0];
+        const uint32_t hs = *(const uint32_t*)&S.raw[w][32 + c][sel];
+        r.nd[0] = *(const uint32_t*)&S.raw[w][c][4 * g];
+        r.nd[1] = *(const uint32_t*)&S.raw[w][16 + c][4 * g];
+        r.d = f16_bits_to_f32(h.x & 0xffffu);
+        r.dm = f16_bits_to_f32(h.x >> 16);
+        r.mn[0] = (float)__builtin_amdgcn_ubfe(h.z, 8 * kp, 6);
+        r.mn[1] = (float)((__builtin_amdgcn_ubfe(h.z, 8 * kp + 6, 2) << 4) | __builtin_amdgcn_ubfe(h.w, 8 * kp + 4, 4));
+        const uint32_t sb = (((hs >> sh0) & low) | ((h.y >> (sh0 + 2)) & ~low)) & 0x3f3fu;
+        const h2v x = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x64646464u, sb, 0x04010400u));  // 1024 + sc
+        r.s = __builtin_elementwise_fma(x, one16, off16);
+        r.n = r.s * m1024;
+        return r;
+    };
 
-    // prologue: raw blocks 0 and 1, token operands of block 0
-    tl_copy_raw(a, w, lane, noff, hoff, 0, raw[0]);
-    tl_copy_raw(a, w, lane, noff, hoff, min(1, nb - 1), raw[1]);
-    tl_copy_tokens(a, w, lane, tile0, tok0, 0, st[0]);
-    wait_vmem_le<0>();
-    tl_dequant(w, lane, raw[0], st[0]);
+    // [lane k = kp + 4 kk][token tile tt][i]
+    float accF[2][4][4], accM[2][4][4];
+#pragma unroll
+    for (int kk = 0; kk < 2; kk++)
+#pragma unroll
+        for (int tt = 0; tt < 4; tt++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) accF[kk][tt][i] = accM[kk][tt][i] = 0.0f;
+
+    copy_raw(0, st[0]);
+    copy_tokens(0, st[0]);
+    copy_raw(1, st[1]);
+    wait_vmem_le<1>();
+    asm volatile("" ::: "memory");
+    Row row = row_of(st[0]);
     wait_lgkm0();
     lds_barrier();
-#pragma unroll 1
-    for (int b = 0; b < nb; b++) {
-        // copies stay unconditional (clamped to the last block; the buffers
-        // they fill are not read this iteration) so the vmcnt counts below
-        // are constants: tokens of b + 1 (5 / 4 copies), raw of b + 2 (2)
-        tl_copy_tokens(a, w, lane, tile0, tok0, min(b + 1, nb - 1), st[(b + 1) & 1]);
-        tl_copy_raw(a, w, lane, noff, hoff, min(b + 2, nb - 1), raw[b & 1]);
-        const TlStage& S = st[b & 1];
-        const f4v dv = *(const f4v*)&S.d[16 * rg + 4 * g];
-        const f4v dm = *(const f4v*)&S.dmin[16 * rg + 4 * g];
-        float dxs[2][4];
+    const NibMasks nm = nib_masks();
+    // Block b from stage S, N the other one.  The pins and scheduling barriers
+    // hold the order (the compiler would keep more operands at once than four
+    // waves per SIMD have registers for).  Register 4 tt + i of an outer
+    // product is token 16 tt + 4g + i.
+    auto block = [&](int b, LnStage& S, LnStage& N) __attribute__((always_inline)) {
+        copy_tokens(b + 1, N);
+        copy_raw(b + 2, S);  // row b is in registers
+        const f16v z16 = {0.0f};
 #pragma unroll
-        for (int n = 0; n < 2; n++) {
-            const float xc = S.xs[32 * tg + 16 * n + c];
+        for (int kk = 0; kk < 2; kk++) {
+            const f16v P = __builtin_amdgcn_mfma_f32_16x16x1f32(S.xsum[g][kp + 4 * kk][c], row.mn[kk], z16, 0, 0, 0);
 #pragma unroll
-            for (int i = 0; i < 4; i++) dxs[n][i] = dv[i] * xc;
-        }
-        // raw block b + 1 (copied last iteration) has landed once at most this
-        // iteration's copies are outstanding; its dequantisation into the
-        // other stage runs in parts between the chain steps below
-        if (w < 3) wait_vmem_le<7>();
-        else wait_vmem_le<6>();
-        asm volatile("" ::: "memory");
-        TlDq dq;
-        tl_dq_begin(w, lane, raw[(b + 1) & 1], dq);
-        // Software pipeline over the lanes k: step k reads lane k + 2's
-        // operands, issues lane k + 1's MFMAs and runs lane k's chains on the
-        // products issued one step earlier, so neither the LDS latency nor the
-        // MFMA latency sits in front of the chains.  The empty asm statements
-        // pin that order (lane k's accumulators final and lane k + 2's
-        // operands arrived when step k ends); without them the compiler
-        // hoists more lanes' operands than two waves per SIMD have registers for.
-        struct Ops {
-            h8v av, bv[2];
-            f4v mk;
-            float xk[2];
-        };
-        auto ops = [&](int k, Ops& o) __attribute__((always_inline)) {
-            o.av = *(const h8v*)(S.a16 + ((rg * 8 + k) * 4 + g) * 256 + c * 16);
-            o.mk = *(const f4v*)&S.m[k][16 * rg + 4 * g];
+            for (int tt = 0; tt < 4; tt++) {
 #pragma unroll
-            for (int n = 0; n < 2; n++) {
-                o.bv[n] = *(const h8v*)(S.b16 + (((2 * tg + n) * 8 + k) * 4 + g) * 256 + c * 16);
-                o.xk[n] = S.xsum[2 * tg + n][k][c];
+                for (int i = 0; i < 4; i++) accM[kk][tt][i] = fmaf(row.dm, P[4 * tt + i], accM[kk][tt][i]);
+                pin4(accM[kk][tt]);
             }
-        };
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        const f16v dxs = __builtin_amdgcn_mfma_f32_16x16x1f32(S.xs[lane], row.d, z16, 0, 0, 0);
+        // step u = (kk, tt): reads step u + 2's activations, issues its own
+        // product and runs the chains of step u - 1
         const f4v z = {0.0f, 0.0f, 0.0f, 0.0f};
-        Ops o[3];
-        f4v dI[2][2];  // [lane k parity][token tile]
-        ops(0, o[0]);
-        ops(1, o[1]);
-        asm volatile("" : "+v"(o[0].av), "+v"(o[0].bv[0]), "+v"(o[0].bv[1]));
+        auto acts = [&](int u) __attribute__((always_inline)) {
+            return *(const h8v*)(S.b16 + (((u & 3) * 8 + kp + 4 * (u >> 2)) * 4 + g) * 256 + c * 16);
+        };
+        h8v bv[3], wv;
+        f4v D[2];
+        bv[0] = acts(0);
+        bv[1] = acts(1);
 #pragma unroll
-        for (int n = 0; n < 2; n++) dI[0][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(o[0].av, o[0].bv[n], z, 0, 0, 0);
-        asm volatile("" : "+v"(o[1].av), "+v"(o[1].bv[0]), "+v"(o[1].bv[1]), "+v"(o[1].mk), "+v"(o[1].xk[0]),
-                     "+v"(o[1].xk[1]));
+        for (int u = 0; u <= 8; u++) {
+            if (u < 6) bv[(u + 2) % 3] = acts(u + 2);
+            if (u == 0 || u == 4) wv = dequant_nib(row.nd[u >> 2], row.s, row.n, nm);
+            if (u < 8) D[u & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bv[u % 3], wv, z, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (u > 0) {
+                const int kk = (u - 1) >> 2, tt = (u - 1) & 3;
 #pragma unroll
-        for (int k = 0; k < 8; k++) {
-            if (k < 6) ops(k + 2, o[(k + 2) % 3]);
-            if (k < 7) {
-                const Ops& nx = o[(k + 1) % 3];
-#pragma unroll
-                for (int n = 0; n < 2; n++)
-                    dI[(k + 1) & 1][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(nx.av, nx.bv[n], z, 0, 0, 0);
+                for (int i = 0; i < 4; i++)
+                    accF[kk][tt][i] = fmaf(D[(u - 1) & 1][i], dxs[4 * tt + i], accF[kk][tt][i]);
+                pin4(accF[kk][tt]);
             }
-            const Ops& cur = o[k % 3];
-#pragma unroll
-            for (int n = 0; n < 2; n++) {
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    accF[n][k][i] = fmaf(dI[k & 1][n][i], dxs[n][i], accF[n][k][i]);
-                    const float mx = cur.mk[i] * cur.xk[n];
-                    accM[n][k][i] = fmaf(dm[i], mx, accM[n][k][i]);
-                }
-            }
-            if (k & 1) tl_dq_part(w, lane, k >> 1, dq, st[(b + 1) & 1]);
-#pragma unroll
-            for (int n = 0; n < 2; n++)
-                asm volatile("" : "+v"(accF[n][k][0]), "+v"(accF[n][k][1]), "+v"(accF[n][k][2]),
-                             "+v"(accF[n][k][3]), "+v"(accM[n][k][0]), "+v"(accM[n][k][1]),
-                             "+v"(accM[n][k][2]), "+v"(accM[n][k][3]));
-            if (k < 6) {
-                Ops& nx = o[(k + 2) % 3];
-                asm volatile("" : "+v"(nx.av), "+v"(nx.bv[0]), "+v"(nx.bv[1]), "+v"(nx.mk),
-                             "+v"(nx.xk[0]), "+v"(nx.xk[1]));
-            }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        tl_dq_end(w, lane, raw[(b + 1) & 1], st[(b + 1) & 1]);
-        wait_vmem_le<2>();  // token operands of b + 1
+        // block b + 1 has landed (all but the raw copy of b + 2)
+        wait_vmem_le<1>();
+        asm volatile("" ::: "memory");
+        row = row_of(N);
         wait_lgkm0();
         lds_barrier();
+    };
+#pragma unroll 1
+    for (int b = 0;;) {
+        block(b, st[0], st[1]);
+        if (++b == nb) break;
+        block(b, st[1], st[0]);
+        if (++b == nb) break;
     }
-    wait_vmem_le<0>();  // the clamped copies of the last iterations
-    // tree8 of the reference's horizontal sum, then the (row, token) stores
+    wait_vmem_le<0>();  // the last copies, never read
+    lds_barrier();
+    // the reference's tree: s_kp = v_kp + v_(kp + 4) here, then (s0 + s1) +
+    // (s2 + s3) across the four waves of a row group, through LDS
+    float* ex = (float*)dyn;  // [rq][kp][tt][i][lane]
 #pragma unroll
-    for (int n = 0; n < 2; n++) {
-        const int t = tok0 + 32 * tg + 16 * n + c;
-        if (t >= a.p) continue;
+    for (int tt = 0; tt < 4; tt++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const int rr = row0 + 16 * rg + 4 * g + i;
-            if (rr >= a.rows) continue;
-            float v[8];
-#pragma unroll
-            for (int k = 0; k < 8; k++) v[k] = accF[n][k][i] - accM[n][k][i];
-            const float s0 = v[0] + v[4], s1 = v[1] + v[5], s2 = v[2] + v[6], s3 = v[3] + v[7];
-            a.out[(size_t)t * a.out_stride + rr] = (s0 + s1) + (s2 + s3);
+            const float v0 = accF[0][tt][i] - accM[0][tt][i], v1 = accF[1][tt][i] - accM[1][tt][i];
+            ex[((w * 4 + tt) * 4 + i) * 64 + lane] = v0 + v1;
         }
+    wait_lgkm0();
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        float v[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) v[q] = ex[(((rq * 4 + q) * 4 + kp) * 4 + i) * 64 + lane];
+        const int t = tok0 + 16 * kp + 4 * g + i, rr = row0 + 16 * rq + c;
+        if (t < a.p && rr < a.rows) a.out[(size_t)t * a.out_stride + rr] = (v[0] + v[1]) + (v[2] + v[3]);
     }
+}
+
+static int launch_q4k_lanes(const PfArgs& a, hipStream_t s) {
+    constexpr size_t lds = 2 * sizeof(LnStage);
+    static_assert(lds >= 65536 && lds <= 160 * 1024, "the stages, and the exchange over them");
+    static const bool ok = hipFuncSetAttribute((const void*)prefill_q4k_lanes_kernel,
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+    if (!ok) {
+        (void)hipGetLastError();
+        return fail(GLLM_EDEVICE, "prefill: %zu bytes of LDS were refused", lds);
+    }
+    const TlMap mp = tl_map(a.rows, a.p);
+    hipLaunchKernelGGL(prefill_q4k_lanes_kernel, dim3(8 * mp.tg_size * mp.rg_size), dim3(1024), lds, s, a, mp);
+    return GLLM_OK;
 }
 
 // --- Q6_K, more than 16 activation rows: 64 x 64 staged tiles --------------
@@ -726,8 +719,8 @@ __device__ __forceinline__ void q6_prep(int tid, int b, Q6Stage& S) {
 __device__ __forceinline__ void u8x4_to_h(uint32_t v, uint32_t& lo, uint32_t& hi) {
     typedef _Float16 h2v __attribute__((ext_vector_type(2)));
     const h2v bias = {(_Float16)-1024.0f, (_Float16)-1024.0f};
-    const h2v a = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x64646464u, v, 0x05010400u)) + bias;
-    const h2v c = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x64646464u, v, 0x05030402u)) + bias;
+    const h2v a = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x64646464u, v, 0x05020400u)) + bias;
+    const h2v c = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x64646464u, v, 0x05030401u)) + bias;
     lo = __builtin_bit_cast(uint32_t, a);
     hi = __builtin_bit_cast(uint32_t, c);
 }
@@ -1399,8 +1392,8 @@ static bool launch_b16s(const PfArgs& a, hipStream_t s) {
 }
 
 
-// Kernel choice.  More than 16 activation rows: the 64 x 64 staged tile
-// (prefill_q4k_tiled_kernel).  At most 16 rows (a decode batch): 64 rows x
+// Kernel choice.  More than 16 activation rows: 64 x 64 tiles split by AVX2
+// lane (prefill_q4k_lanes_kernel).  At most 16 rows (a decode batch): 64 rows x
 // 16 tokens (prefill_q4k_mfma_kernel); the per-block staging (q8 to f16,
 // scale decoding) is a fixed cost per workgroup, so 64 rows per workgroup
 // beat smaller tiles that would fill more CUs (measured at batch 8: 22.8 vs
@@ -1417,9 +1410,7 @@ int launch_q4k_mfma(const uint8_t* d_w, size_t rb, int rows, int blocks, const A
     if (p > kTiledMinP) {
         if (!act.b16t || !fits)
             return fail(GLLM_EINVAL, "prefill: %d rows of %zu B need f16 tiles and < 4 GiB", rows, rb);
-        const TlMap mp = tl_map(rows, p);
-        const int grid = 8 * mp.tg_size * mp.rg_size;
-        hipLaunchKernelGGL(prefill_q4k_tiled_kernel, dim3(grid), dim3(512), 0, s, a, mp);
+        GLLM_TRY(launch_q4k_lanes(a, s));
     } else if ((rows + 63) / 64 < 2 * device_cus() / 3) {
         if (!fits) return fail(GLLM_EINVAL, "prefill: weights of %zu B past 4 GiB", (size_t)rows * rb);
         const bool done = p > 8 ? launch_b16s<4, 3, 16>(a, s) : launch_b16p<2>(a, s);

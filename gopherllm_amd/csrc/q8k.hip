@@ -63,7 +63,7 @@ __global__ __launch_bounds__(256) void q8k_prep_kernel(const float* __restrict__
     if (a.b16t && t >= a.p) {  // padding tokens of the last f16 tile (uniform per workgroup)
         const int kappa = q8perm_offset(e);
         a.b16t[((size_t)b * a.tiles + (t >> 4)) * 4096 + ((kappa >> 3) * 16 + (t & 15)) * 8 +
-               (kappa & 7)] = 0;
+               b16_slot(kappa)] = 0;
         if (e < 8) a.xs32t[(((size_t)b * a.tiles + (t >> 4)) * 8 + e) * 16 + (t & 15)] = 0.0f;
         return;
     }
@@ -93,9 +93,9 @@ __global__ __launch_bounds__(256) void q8k_prep_kernel(const float* __restrict__
     const int kappa = q8perm_offset(e);
     a.q8perm[(size_t)t * cols + (size_t)b * 256 + kappa] = (int8_t)q;
     if (a.b16t) {
-        // kappa = 32 k + 8 g + i -> ((k 4 + g) 16 + c) 8 + i of the tile block
+        // kappa = 32 k + 8 g + i -> ((k 4 + g) 16 + c) 8 + b16_slot(i) of the tile block
         a.b16t[((size_t)b * a.tiles + (t >> 4)) * 4096 + ((kappa >> 3) * 16 + (t & 15)) * 8 +
-               (kappa & 7)] = __builtin_bit_cast(uint16_t, (_Float16)(float)q);
+               b16_slot(kappa)] = __builtin_bit_cast(uint16_t, (_Float16)(float)q);
     }
     if (e == 0) a.xscale[(size_t)t * nb + b] = scale;
     if (e < 8) {

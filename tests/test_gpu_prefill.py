@@ -45,6 +45,17 @@ def test_prefill_bit_exact_small(hip, rows, cols, p):
     assert_bits(got, amd64(data, xs, rows, cols), "vs amd64 oracle")
 
 
+@pytest.mark.parametrize("rows,cols,p", [(1, 768, 17), (65, 256, 65), (64, 512, 128), (130, 1280, 129),
+                                         (63, 768, 64)])
+def test_prefill_tile_edges(hip, rows, cols, p):
+    """One row or token past a 64 x 64 tile, one to five blocks (the block
+    loop's two halves), the last wave's rows and tokens past the end."""
+    data, _ = quant_matrix(ref.Q4_K, rows, cols, 900 + rows)
+    w = hip.Weight.from_host(data, ref.Q4_K, rows, cols)
+    xs = normal(901 + p, (p, cols))
+    assert_bits(w.matvec_batch(xs), amd64(data, xs, rows, cols), f"{rows}x{cols} p={p}")
+
+
 def test_prefill_degenerate_blocks(hip):
     """All-zero tokens, zero 256-blocks inside a token, a lone large value and
     NaN-free extremes (q8kQuantize's scale-0 blocks, quant_q8k_portable.go:36-62)."""
