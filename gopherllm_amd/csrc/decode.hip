@@ -259,7 +259,8 @@ static int ensure_buffers(gllm_hip_model* m, int p) {
     if (m->h_tokens) (void)hipHostFree(m->h_tokens);
     GLLM_HIP(hipMalloc(&m->d_tokens, (size_t)(p + 4) * 4));
     GLLM_HIP(hipHostMalloc(&m->h_tokens, (size_t)(p + 4) * 4, hipHostMallocDefault));
-    const size_t an = act_bytes(std::max(c.dim, c.hidden), p);
+    // the widest projection input: the attention output may be wider than the FFN's
+    const size_t an = act_bytes(std::max({c.dim, c.hidden, c.n_heads * c.head_dim}), p);
     if (m->act) (void)hipFree(m->act);
     GLLM_HIP(hipMalloc(&m->act, an));
     m->act_n = an;

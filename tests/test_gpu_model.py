@@ -281,6 +281,21 @@ def test_decode_attention_head_dim_128_matches_oracle(hip, n_heads, n_kv):
         assert np.array_equal(v, cpu.vcache(l, max_len)[:used])
 
 
+def test_attention_wider_than_ffn(hip):
+    """n_heads * head_dim = 1024 with dim and hidden 512: the attention output
+    projection quantises rows wider than either, for a prompt and a decode
+    step."""
+    from gopherllm_amd.decoder import LlamaDecoder
+    m = tiny_llama(seed=51, n_layers=1, dim=512, hidden=512, n_heads=8, n_kv_heads=2, head_dim=128, vocab=500)
+    prompt = np.random.default_rng(52).integers(0, 500, 40)
+    gpu, cpu = LlamaDecoder.from_host_model(m, 64), ref.Llama(m, 64)
+    gt, gl = gpu.prefill(prompt, want_logits=True)
+    ct, cl = cpu.prefill(prompt)
+    assert gt == ct and np.array_equal(bits(gl), bits(cl))
+    want, hid = cpu.decode(ct, 40)
+    assert gpu.decode(gt, 40) == want and np.array_equal(bits(gpu.hidden()), bits(hid))
+
+
 def test_swiglu_epilogue_decode_matches_oracle(hip):
     """dim 1024, hidden 8192: the gate/up launch takes the RMSNorm prologue
     and the SwiGLU + Q8K epilogue (the last workgroup of each 256-row block
