@@ -16,58 +16,15 @@
 #include <algorithm>
 #include <cstdlib>
 
-#include "gllm_common.h"
+#include "attn_exp.h"
 
 namespace gllm {
+size_t attend_prefill_floats(int p, int n_heads, int n_kv, int span_max);
+bool attend_prefill_fits(int hd, int kv_dim_k, int kv_dim_v);
+int attend_prefill(const float* d_q, const uint16_t* K, const uint16_t* V, int kv_dim, int n_heads, int n_kv, int hd,
+                   int span0, int p, float scale, float* scratch, float* d_out, hipStream_t s);
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-// fastExpF32 (fastmath.go:47-77), operation for operation, without
-// branches: the two range checks select the result, so a thread's several
-// exps interleave instead of running one exec-masked block after another.
-// Inside the range |t| < 128, so the clamp only keeps the int conversion
-// defined for inputs the selects discard (a NaN still gives NaN).  The
-// empty asm keeps the compiler from turning the first select back into a
-// branch around the polynomial.
-__device__ __forceinline__ float fast_exp(float x) {
-    const float t = x * 1.44269502f;  // float32(1.4426950408889634)
-    const float tc = fminf(fmaxf(t, -256.0f), 256.0f);
-    const int k = (int)(tc + (tc >= 0.0f ? 0.5f : -0.5f));
-    const float r = (float)((double)x - (double)k * 0.6931471805599453);
-    const float p = 1.0f + r * (1.0f + r * (0.5f + r * ((float)(1.0 / 6) +
-                    r * ((float)(1.0 / 24) + r * ((float)(1.0 / 120) + r * (float)(1.0 / 720))))));
-    float v = p * __uint_as_float((uint32_t)(127 + k) << 23);
-    asm volatile("" : "+v"(v));  // computed unconditionally: the selects stay selects
-    return x > 88.02969f ? __int_as_float(0x7f800000) : x < -87.33654f ? 0.0f : v;
-}
-
-// fast_exp of N independent values, step by step across all of them so
-// their dependent chains interleave (one wave per SIMD hides no latency
-// otherwise); each value sees exactly fast_exp's operations.
-template <int N>
-__device__ __forceinline__ void fast_exp_n(const float (&x)[N], float (&y)[N]) {
-    int k[N];
-    float r[N];
-#pragma unroll
-    for (int i = 0; i < N; i++) {
-        const float t = x[i] * 1.44269502f;
-        const float tc = fminf(fmaxf(t, -256.0f), 256.0f);
-        k[i] = (int)(tc + (tc >= 0.0f ? 0.5f : -0.5f));
-    }
-#pragma unroll
-    for (int i = 0; i < N; i++) r[i] = (float)((double)x[i] - (double)k[i] * 0.6931471805599453);
-#pragma unroll
-    for (int i = 0; i < N; i++) {
-        const float p = 1.0f + r[i] * (1.0f + r[i] * (0.5f + r[i] * ((float)(1.0 / 6) +
-                        r[i] * ((float)(1.0 / 24) + r[i] * ((float)(1.0 / 120) + r[i] * (float)(1.0 / 720))))));
-        y[i] = p * __uint_as_float((uint32_t)(127 + k[i]) << 23);
-    }
-#pragma unroll
-    for (int i = 0; i < N; i++) asm volatile("" : "+v"(y[i]));
-#pragma unroll
-    for (int i = 0; i < N; i++)
-        y[i] = x[i] > 88.02969f ? __int_as_float(0x7f800000) : x[i] < -87.33654f ? 0.0f : y[i];
-}
 
 // row[t] = fast_exp(row[t] - mx) for t = first, first + stride, ... < span,
 // N positions at a time so that their chains interleave.
@@ -1489,6 +1446,29 @@ static bool vdec_usable(int kvmul, int span_max) {
     return big_ok && bytes <= 160 * 1024;
 }
 
+// Several tokens on the matrix cores (attn_prefill.hip) instead of a
+// workgroup per (head, token).  At head_dim 128 the line is sixteen tokens:
+// a query tile is one workgroup, and fewer tokens leave most CUs idle while
+// each step's exponentials, barrier and products follow one another.  Per
+// layer of the 8B shape at position 4000, with everything else of the layer:
+// 2 / 8 / 17 / 64 / 512 tokens 210 / 256 / 494 / 742 / 3717 us without,
+// 279 / 316 / 485 / 512 / 1438 us with.  Spans past what the other kernel
+// keeps in LDS, and head_dim 64, would take the three-kernel path below,
+// which is slower at any count.
+static bool prefill_path(const gllm_hip_kv* kv, int p, int kvmul, int hd, int span_max) {
+    if (p <= 1 || !attend_prefill_fits(hd, kv->kv_dim_k, kv->kv_dim_v)) return false;
+    return p >= 16 || hd != kFusedHD || kvmul > 4 || span_max > kSmaxSpan;
+}
+
+// Device floats that attend_exact works in for at most p tokens over spans of
+// at most span_max.
+size_t attend_exact_floats(const gllm_hip_kv* kv, int p, int n_heads, int n_kv, int hd, int span_max) {
+    const bool tiles = attend_prefill_fits(hd, kv->kv_dim_k, kv->kv_dim_v);
+    const size_t rows = tiles ? std::min(p, 15) : p;  // tokens that may take the other kernels
+    const size_t n = rows * n_heads * (span_max + 1) + (size_t)n_heads * ((span_max + 31) / 32) + 64;
+    return tiles ? std::max(n, attend_prefill_floats(p, n_heads, n_kv, span_max)) : n;
+}
+
 // Exact attention for p consecutive query tokens: token t attends
 // start .. end0 + t.  d_q / d_out: [p][n_heads][hd].
 bool attend_exact_graphable(const gllm_hip_kv* kv, int n_heads, int n_kv, int hd, int span_cap) {
@@ -1496,8 +1476,8 @@ bool attend_exact_graphable(const gllm_hip_kv* kv, int n_heads, int n_kv, int hd
            span_cap <= kSmaxSpan1;
 }
 
-// scratch: p * n_heads * (span_max + 1) + n_heads * ceil(span_max / 32) + 64
-// floats of device memory, or null for the calling thread's scratch.  d_end (with p == 1): the end position is read
+// scratch: attend_exact_floats(p, ...) floats of device memory, or null for
+// the calling thread's scratch.  d_end (with p == 1): the end position is read
 // on the device and span_cap bounds the span, so the launches do not depend
 // on the position (a captured decode step replays for every position).
 int attend_exact(const gllm_hip_kv* kv, int l, const float* d_q, int n_heads, int n_kv, int hd,
@@ -1517,6 +1497,13 @@ int attend_exact(const gllm_hip_kv* kv, int l, const float* d_q, int n_heads, in
     if (rope_sin && (!d_end || !d_knew || !d_vnew))
         return fail(GLLM_EINVAL, "attend: RoPE folding needs one token and its raw k / v rows");
     const AttnRope rope{rope_sin, rope_cos, d_knew, d_vnew, kv->k[l], kv->v[l], rope_cur};
+    if (prefill_path(kv, p, kvmul, hd, span_max)) {
+        float* sc = scratch ? scratch
+                            : (float*)thread_scratch(5, attend_prefill_floats(p, n_heads, n_kv, span_max) * 4, s);
+        if (!sc) return scratch_error();
+        return attend_prefill(d_q, kv->k[l] + (size_t)start * kv->kv_dim_k, kv->v[l] + (size_t)start * kv->kv_dim_v,
+                              kv->kv_dim_k, n_heads, n_kv, hd, span0, p, scale, sc, d_out, s);
+    }
     if (hd == kFusedHD && kvmul <= 4 && kv->kv_dim_k == kv->kv_dim_v &&
         span_max <= (p == 1 ? kSmaxSpan1 : kSmaxSpan)) {
         const int nchunk = (span_max + kScoreChunk - 1) / kScoreChunk;

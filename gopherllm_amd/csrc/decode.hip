@@ -47,6 +47,7 @@ int attend_exact(const gllm_hip_kv* kv, int l, const float* d_q, int n_heads, in
                  float* scratch, const int* d_end, int span_cap, const float* rope_sin,
                  const float* rope_cos, const float* d_knew, const float* d_vnew,
                  const float* rope_cur = nullptr);
+size_t attend_exact_floats(const gllm_hip_kv* kv, int p, int n_heads, int n_kv, int hd, int span_max);
 bool attend_exact_graphable(const gllm_hip_kv* kv, int n_heads, int n_kv, int hd, int span_cap);
 int attend_splitk(const gllm_hip_kv* kv, int l, const float* d_q, int n_heads, int n_kv, int hd,
                   int start, int end, float scale, float* d_out, hipStream_t s);
@@ -267,8 +268,8 @@ static int ensure_buffers(gllm_hip_model* m, int p) {
     if (m->scores) (void)hipFree(m->scores);
     // every attention path of a chunk, the long-span one included, works in
     // this buffer (none grows the thread's scratch)
-    GLLM_HIP(hipMalloc(&m->scores, ((size_t)p * c.n_heads * (c.max_len + 1) +
-                                    (size_t)c.n_heads * ((c.max_len + 31) / 32) + 64) * 4));
+    GLLM_HIP(hipMalloc(&m->scores,
+                       attend_exact_floats(m->kv, p, c.n_heads, c.n_kv_heads, c.head_dim, c.max_len) * 4));
     m->max_p = p;
     drop_decode_graph(m);  // it captured the old buffers
     return GLLM_OK;
