@@ -363,8 +363,8 @@ __device__ __forceinline__ void sb_scale_min(const u4v h, int j, uint32_t& sc, u
 // for the kernel before it, which staged the dequantised f16 weights in LDS
 // and ran all eight lanes of a 16 x 32 tile in a wave (two waves per SIMD,
 // LDS traffic 370 KB per block), 195 us with eight waves of 32 rows x 64
-// tokens (two per SIMD), 202 us with eight waves of 16 rows x 128 tokens, 183
-// us like this.  What is left is issue: per wave and block 64 chain steps, 37
+// tokens (two per SIMD), 202 us with eight waves of 16 rows x 128 tokens, 180
+// us like this.  What is left is issue: per wave and block 64 chain steps, 40
 // VALU operations of dequantisation and 11 matrix instructions, which hardly
 // overlap the VALU on this part (a 16x16x32 f16 MFMA and four fmas take 30
 // cycles at four waves per SIMD, the MFMA alone 20).
@@ -444,6 +444,20 @@ __device__ __forceinline__ h8v dequant_nib(uint32_t w, h2v s, h2v n, const NibMa
 // A chain step ends here: the compiler may not sink it past this point.
 __device__ __forceinline__ void pin4(float (&v)[4]) {
     asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+}
+
+// (s0 + s1) + (s2 + s3) of the four waves of row group rq, from the exchange
+// ex[rq][kp][token tile][i][lane]: wave (rq, kp) stores token tile kp.
+__device__ __forceinline__ void lanes_store(const PfArgs& a, const float* ex, int row0, int tok0, int rq, int kp,
+                                            int lane) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        float v[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) v[q] = ex[(((rq * 4 + q) * 4 + kp) * 4 + i) * 64 + lane];
+        const int t = tok0 + 16 * kp + 4 * (lane >> 4) + i, rr = row0 + 16 * rq + (lane & 15);
+        if (t < a.p && rr < a.rows) a.out[(size_t)t * a.out_stride + rr] = (v[0] + v[1]) + (v[2] + v[3]);
+    }
 }
 
 __global__ __launch_bounds__(1024) void prefill_q4k_lanes_kernel(PfArgs a, TlMap mp) {
@@ -544,6 +558,11 @@ __global__ __launch_bounds__(1024) void prefill_q4k_lanes_kernel(PfArgs a, TlMap
     auto block = [&](int b, LnStage& S, LnStage& N) __attribute__((always_inline)) {
         copy_tokens(b + 1, N);
         copy_raw(b + 2, S);  // row b is in registers
+        // LDS addresses are rebuilt from the lane each block: kept across
+        // blocks they would spill
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        const int g = ln >> 4, c = ln & 15;
         const f16v z16 = {0.0f};
 #pragma unroll
         for (int kk = 0; kk < 2; kk++) {
@@ -556,7 +575,7 @@ __global__ __launch_bounds__(1024) void prefill_q4k_lanes_kernel(PfArgs a, TlMap
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        const f16v dxs = __builtin_amdgcn_mfma_f32_16x16x1f32(S.xs[lane], row.d, z16, 0, 0, 0);
+        const f16v dxs = __builtin_amdgcn_mfma_f32_16x16x1f32(S.xs[ln], row.d, z16, 0, 0, 0);
         // step u = (kk, tt): reads step u + 2's activations, issues its own
         // product and runs the chains of step u - 1
         const f4v z = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -610,31 +629,31 @@ __global__ __launch_bounds__(1024) void prefill_q4k_lanes_kernel(PfArgs a, TlMap
         }
     wait_lgkm0();
     lds_barrier();
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        float v[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) v[q] = ex[(((rq * 4 + q) * 4 + kp) * 4 + i) * 64 + lane];
-        const int t = tok0 + 16 * kp + 4 * g + i, rr = row0 + 16 * rq + c;
-        if (t < a.p && rr < a.rows) a.out[(size_t)t * a.out_stride + rr] = (v[0] + v[1]) + (v[2] + v[3]);
-    }
+    lanes_store(a, ex, row0, tok0, rq, kp, lane);
+}
+
+// One workgroup of 1024 threads per 64 x 64 tile.
+template <size_t LDS>
+static int launch_lanes(void (*kern)(PfArgs, TlMap), bool lds_ok, const PfArgs& a, hipStream_t s) {
+    static_assert(LDS >= 65536 && LDS <= 160 * 1024, "the stages, and the exchange over them");
+    if (!lds_ok) return fail(GLLM_EDEVICE, "prefill: %zu bytes of LDS were refused", LDS);
+    const TlMap mp = tl_map(a.rows, a.p);
+    hipLaunchKernelGGL(kern, dim3(8 * mp.tg_size * mp.rg_size), dim3(1024), LDS, s, a, mp);
+    return GLLM_OK;
+}
+static bool lanes_lds(const void* kern, size_t lds) {
+    if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
 }
 
 static int launch_q4k_lanes(const PfArgs& a, hipStream_t s) {
     constexpr size_t lds = 2 * sizeof(LnStage);
-    static_assert(lds >= 65536 && lds <= 160 * 1024, "the stages, and the exchange over them");
-    static const bool ok = hipFuncSetAttribute((const void*)prefill_q4k_lanes_kernel,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
-    if (!ok) {
-        (void)hipGetLastError();
-        return fail(GLLM_EDEVICE, "prefill: %zu bytes of LDS were refused", lds);
-    }
-    const TlMap mp = tl_map(a.rows, a.p);
-    hipLaunchKernelGGL(prefill_q4k_lanes_kernel, dim3(8 * mp.tg_size * mp.rg_size), dim3(1024), lds, s, a, mp);
-    return GLLM_OK;
+    static const bool ok = lanes_lds((const void*)prefill_q4k_lanes_kernel, lds);
+    return launch_lanes<lds>(prefill_q4k_lanes_kernel, ok, a, s);
 }
 
-// --- Q6_K, more than 16 activation rows: 64 x 64 staged tiles --------------
+// --- Q6_K, more than 16 activation rows: one pair of AVX2 lanes per wave ---
 // q6kDotQ8KRow (kernels_amd64.s Q6KQ8QUAD, the batch-1 row kernel
 // gemv_q6k_kernel) per AVX2 lane k of a 256-element block b:
 //   I       = sum over the lane's 32 elements of sc(e) * code(e) * q8(e)
@@ -647,238 +666,204 @@ static int launch_q4k_lanes(const PfArgs& a, hipStream_t s) {
 // with |sc * (code >> 4)| <= 384 and |sc * (code & 15)| <= 1920 exact in f16
 // and every partial sum of 32 products an integer below 2^24, so each of
 // the two v_mfma_f32_16x16x32_f16 results is its exact integer sum and
-// fma(hi, 16, lo) rounds 16 hi + lo once: float(I).  The chains then run in
-// VALU registers in the reference's order.
-// Workgroup: 64 rows x 64 tokens, eight waves; wave w owns rows 16 (w & 3)
-// .. + 15 and the token tiles 2 (w >> 2), 2 (w >> 2) + 1.  Per block,
-// double-buffered in LDS and copied global -> LDS one block ahead: the 64
-// rows' block bytes as stored (ql, qh, scales; the A operands are built
-// from them by the wave that uses them, lane (g, c) the 8 codes of row c,
-// lane k, kappa 8 g .. + 7), the four 16-token B tiles (the quantiser's f16
-// layout) and the tokens' xs16 and xscale; the rows' scales and d as floats
-// are prepared once per block.  Weights need rows * rb < 4 GiB and
-// 16-byte aligned blocks (blocks % 8 == 0).
-constexpr int kQ6Rows = 64, kQ6Tok = 64;
-constexpr int kQ6RawPieces = 64 * 13;  // 64 rows x 13 pieces of 16 bytes (208-byte blocks)
+// fma(hi, 16, lo) rounds 16 hi + lo once: float(I).
+// The split of the work is prefill_q4k_lanes_kernel's: wave (rq, kp) owns 16
+// rows, 64 tokens and the lanes kp and kp + 4; o2 is a product and an fma of
+// outer products, two v_mfma_f32_16x16x1, and d * xscale a third.  Three VALU
+// steps per product are left (fma(hi, 16, lo) and the two chains).  Weights
+// need rows * rb < 4 GiB and 16-byte aligned blocks (blocks % 8 == 0).
+// With the quantiser launch, 4096 x 14336 x 333 (1.5 rounds of workgroups) and
+// 14336 x 4096 x 512: 473 and 490 us for 64 x 64 tiles that ran all eight
+// lanes in a wave and built the A operands twice, 259 and 273 us like this.
+// Bound by issue: per wave and block 96 chain steps, about 70 operations of
+// dequantisation and 21 matrix instructions.
+struct Q6Raw {
+    uint8_t q[64][16];   // [16 part + row c]: lane kp's ql, lane kp + 4's ql, the 16 bytes with their qh
+    uint8_t sc[16][16];  // [row c]
+    uint32_t dw[16];     // [row c]: the dword holding d of blocks b & ~1, b | 1
+};
 struct Q6Stage {
-    uint8_t q[kQ6RawPieces * 16];  // [row][208]: ql 128, qh 64, scales 16
-    uint32_t dw[64];               // [row]: the dword holding d of blocks b & ~1, b | 1
     uint8_t b16[4 * 8 * 4 * 256];  // [token tile][lane k][group g][token c][8 halves]
-    float x16[kQ6Tok][16];         // [token][16-group] xs16
-    float xs[kQ6Tok];
-    float sc[16][kQ6Rows];         // [scale index][row] int8 scale
-    float d[kQ6Rows];
+    float x16[4][kTlTok][4];       // [16-group / 4][token][16-group % 4] xs16
+    float xs[kTlTok];
+    Q6Raw raw[16];                 // [wave]
 };
 
-// Block b's operands into S: the 832 raw pieces (two 1 KB copies on waves
-// 0-5, one on wave 6), the rows' d dwords (wave 7), four 1 KB pieces of B
-// per wave, the tokens' xs16 (waves 0-3) and xscales (wave 4).
-__device__ __forceinline__ void q6_copy(const PfArgs& a, int w, int lane, int row0, int tile0, int tok0,
-                                        int b, Q6Stage& S) {
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        // pieces 128 w + 64 i + lane of 832: waves 0-5 two each, wave 6 one
-        const int pc = 128 * w + 64 * i + lane;
-        if (pc < kQ6RawPieces) {  // wave-uniform: 832 = 6.5 x 128
-            const int r = pc / 13, off = (pc % 13) * 16;
-            const size_t row = (size_t)min(row0 + r, a.rows - 1);
-            lds_copy16_s(a.w, (uint32_t)(row * a.rb + (size_t)b * 208 + off), lds_addr(S.q + 16 * (pc - lane)));
-        }
-    }
-    if (w == 7) {
-        const size_t row = (size_t)min(row0 + lane, a.rows - 1);
-        lds_copy4_s(a.w, (uint32_t)(row * a.rb + (size_t)a.blocks * 208 + (size_t)(b & ~1) * 2),
-                    lds_addr(&S.dw[0]));
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int ch = 4 * w + i, tt = ch >> 3, piece = ch & 7;
-        const int gt = min(tile0 + tt, a.act.tiles - 1);
-        const uint8_t* base = (const uint8_t*)a.act.b16t + ((size_t)b * a.act.tiles + gt) * 8192 + piece * 1024;
-        lds_copy16_s(base, 16 * lane, lds_addr(S.b16 + tt * 8192 + piece * 1024));
-    }
-    if (w < 4) {
-        const int t = min(tok0 + 16 * w + (lane >> 2), a.p - 1);
-        lds_copy16_s(a.act.xs16, (uint32_t)(((size_t)t * (a.blocks * 16) + (size_t)b * 16) * 4 + 16 * (lane & 3)),
-                     lds_addr(&S.x16[16 * w][0]));
-    } else if (w == 4) {
-        lds_copy4_s(a.act.xscale + b, (uint32_t)min(tok0 + lane, a.p - 1) * a.blocks * 4, lds_addr(&S.xs[0]));
-    }
-}
-
-// The rows' scales and d of block b as floats: thread t scale index t >> 5
-// of rows t & 31 and 32 + (t & 31); threads 0-63 d of row t.
-__device__ __forceinline__ void q6_prep(int tid, int b, Q6Stage& S) {
-    const int idx = tid >> 5, r = tid & 31;
-    S.sc[idx][r] = (float)(int8_t)S.q[r * 208 + 192 + idx];
-    S.sc[idx][32 + r] = (float)(int8_t)S.q[(32 + r) * 208 + 192 + idx];
-    if (tid < 64) S.d[tid] = f16_bits_to_f32((S.dw[tid] >> (16 * (b & 1))) & 0xffffu);
-}
-
-// four bytes (values 0..255, exact) -> two half2 words
-__device__ __forceinline__ void u8x4_to_h(uint32_t v, uint32_t& lo, uint32_t& hi) {
-    typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-    const h2v bias = {(_Float16)-1024.0f, (_Float16)-1024.0f};
-    const h2v a = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x64646464u, v, 0x05020400u)) + bias;
-    const h2v c = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x64646464u, v, 0x05030401u)) + bias;
-    lo = __builtin_bit_cast(uint32_t, a);
-    hi = __builtin_bit_cast(uint32_t, c);
-}
-
-// A operands (low and high code fields) of lane (g, c) for lane k from its
-// row's raw bytes: quads m = 2g, 2g + 1 of lane k (ql dwords 2h, 2h + 1 and
-// qh dword h of the lane, h = g >> 1, nibble / bit-pair shift 4 (g & 1))
-// with scales 8h + 4 (g & 1) + (k >> 2) and + 2.
-struct Q6Raw8 {
-    uint2 ql;
-    uint32_t qh, sc;
+// Field of four code bytes as two half2 words of B16's byte pairs (0, 2) and
+// (1, 3): y0 / y1 hold the field at bits 4 .. of the pairs' low bytes, and
+// under f16 exponent bits of 64 they read 64 + field.
+struct Q6Masks {
+    uint32_t nib, lo2, hi2, exp;
 };
-__device__ __forceinline__ void q6_raw(const uint8_t* row, int k, int g, Q6Raw8& o) {
-    const int h = g >> 1;
-    o.ql = *(const uint2*)(row + 16 * k + 8 * h);
-    o.qh = *(const uint32_t*)(row + 128 + 8 * k + 4 * h);
-    o.sc = *(const uint32_t*)(row + 192 + 8 * h + 4 * (g & 1));
-}
-__device__ __forceinline__ void q6_operands(const Q6Raw8& o, int k, int g, h8v& lo, h8v& hi) {
-    typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-    const int sh = 4 * (g & 1), hk = k >> 2;
-    // scale bytes hk and hk + 2 of o.sc, as exact f16 (byte ^ 0x80 = s + 128)
-    const uint32_t sv = o.sc ^ 0x80808080u;
-    const h2v m1152 = {(_Float16)-1152.0f, (_Float16)-1152.0f};
-    const h2v f0 = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x64646464u, sv, hk ? 0x04010401u : 0x04000400u)) + m1152;
-    const h2v f1 = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x64646464u, sv, hk ? 0x04030403u : 0x04020402u)) + m1152;
-    uint32_t l0, l1, l2, l3, h0, h1, h2, h3;
-    u8x4_to_h((o.ql.x >> sh) & 0x0f0f0f0fu, l0, l1);
-    u8x4_to_h((o.ql.y >> sh) & 0x0f0f0f0fu, l2, l3);
-    u8x4_to_h((o.qh >> sh) & 0x03030303u, h0, h1);
-    u8x4_to_h((o.qh >> (sh + 2)) & 0x03030303u, h2, h3);
-    // exact: products of small integers below 2048
-    const h2v a0 = __builtin_bit_cast(h2v, l0) * f0, a1 = __builtin_bit_cast(h2v, l1) * f0;
-    const h2v a2 = __builtin_bit_cast(h2v, l2) * f1, a3 = __builtin_bit_cast(h2v, l3) * f1;
-    const h2v b0 = __builtin_bit_cast(h2v, h0) * f0, b1 = __builtin_bit_cast(h2v, h1) * f0;
-    const h2v b2 = __builtin_bit_cast(h2v, h2) * f1, b3 = __builtin_bit_cast(h2v, h3) * f1;
-    lo[0] = a0[0]; lo[1] = a0[1]; lo[2] = a1[0]; lo[3] = a1[1];
-    lo[4] = a2[0]; lo[5] = a2[1]; lo[6] = a3[0]; lo[7] = a3[1];
-    hi[0] = b0[0]; hi[1] = b0[1]; hi[2] = b1[0]; hi[3] = b1[1];
-    hi[4] = b2[0]; hi[5] = b2[1]; hi[6] = b3[0]; hi[7] = b3[1];
-}
 
-__global__ __launch_bounds__(512) void prefill_q6k_tiled_kernel(PfArgs a, TlMap mp) {
-    __shared__ __align__(16) Q6Stage st[2];
+__global__ __launch_bounds__(1024) void prefill_q6k_lanes_kernel(PfArgs a, TlMap mp) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t dyn[];
+    Q6Stage* const st = (Q6Stage*)dyn;
     const int id = blockIdx.x, xcd = id & 7, local = id >> 3;
     const int lt = local % mp.tg_size, lrow = local / mp.tg_size;
     const int ttile = (xcd % mp.h) * mp.tg_size + lt, rtile = (xcd / mp.h) * mp.rg_size + lrow;
     if (lrow >= mp.rg_size || ttile >= mp.tok_tiles || rtile >= mp.row_tiles) return;  // whole workgroup
-    const int row0 = rtile * kQ6Rows, tok0 = ttile * kQ6Tok, tile0 = tok0 / 16;
-    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int row0 = rtile * kTlRows, tok0 = ttile * kTlTok, tile0 = tok0 / 16;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 4, c = lane & 15;
-    const int rg = w & 3, tg = w >> 2;
+    const int kp = w & 3, rq = w >> 2;
     const int nb = a.blocks;
 
-    float accF[2][8][4], accM[2][8][4];
-#pragma unroll
-    for (int n = 0; n < 2; n++)
-#pragma unroll
-        for (int k = 0; k < 8; k++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) accF[n][k][i] = accM[n][k][i] = 0.0f;
-
-    q6_copy(a, w, lane, row0, tile0, tok0, 0, st[0]);
-    wait_vmem_le<0>();
-    lds_barrier();
-    q6_prep(tid, 0, st[0]);
-    wait_lgkm0();
-    lds_barrier();
-#pragma unroll 1
-    for (int b = 0; b < nb; b++) {
-        // unconditional copies of block b + 1 (clamped to the last block)
-        // into the stage not read this iteration
-        q6_copy(a, w, lane, row0, tile0, tok0, min(b + 1, nb - 1), st[(b + 1) & 1]);
-        const Q6Stage& S = st[b & 1];
-        // per-lane LDS offsets, rebuilt every block behind an empty asm so
-        // the compiler keeps one register per operand stream instead of
-        // hoisting an address per (lane k, tile) out of the loop
-        const int h = g >> 1;
-        uint32_t o_ql = (16 * rg + c) * 208 + 8 * h, o_qh = (16 * rg + c) * 208 + 128 + 4 * h;
-        uint32_t o_sc = (16 * rg + c) * 208 + 192 + 8 * h + 4 * (g & 1);
-        uint32_t o_b = (2 * tg * 8 * 4 + g) * 256 + c * 16, o_x = (32 * tg + c) * 64;
-        uint32_t o_k = (16 * rg + 4 * g) * 4;
-        asm volatile("" : "+v"(o_ql), "+v"(o_qh), "+v"(o_sc), "+v"(o_b), "+v"(o_x), "+v"(o_k));
-        const uint8_t* q = S.q;
-        const uint8_t* bt = S.b16;
-        const uint8_t* xt = (const uint8_t*)&S.x16[0][0];
-        const uint8_t* sct = (const uint8_t*)&S.sc[0][0];
-        float dv[4], dxs[2][4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) dv[i] = S.d[16 * rg + 4 * g + i];
-#pragma unroll
-        for (int n = 0; n < 2; n++) {
-            const float xv = S.xs[32 * tg + 16 * n + c];
-#pragma unroll
-            for (int i = 0; i < 4; i++) dxs[n][i] = dv[i] * xv;  // VMULSS d * xscale
+    // Copies of one block's tokens: two 1 KB pieces of B16 (as in the Q4_K
+    // kernel), the tokens' xs16 (waves 0-3, four 16-groups each) and xscales
+    // (wave 4)
+    const int last = a.act.tiles - 1, tok = min(tok0 + lane, a.p - 1);
+    const size_t bstep = (size_t)a.act.tiles * 8192;
+    const uint8_t* bsrc = (const uint8_t*)a.act.b16t + (size_t)min(tile0 + rq, last) * 8192 + 2048 * kp;
+    const uint32_t xoff = w < 4 ? (uint32_t)tok * nb * 64 + 16 * w : (uint32_t)tok * nb * 4;
+    auto copy_tokens = [&](int b, Q6Stage& S) __attribute__((always_inline)) {
+        b = min(b, nb - 1);
+        const uint8_t* src = bsrc + b * bstep;
+        const uint32_t dst = lds_addr(S.b16 + rq * 8192 + 2048 * kp);
+        lds_copy16_s(src, 16 * lane, dst);
+        lds_copy16_s(src + 1024, 16 * lane, dst + 1024);
+        if (w < 4) lds_copy16_s(a.act.xs16 + (size_t)b * 16, xoff, lds_addr(&S.x16[w][0][0]));
+        else if (w == 4) lds_copy4_s(a.act.xscale + b, xoff, lds_addr(&S.xs[0]));
+    };
+    // The wave's rows: three copies
+    const uint32_t rbase = (uint32_t)min(row0 + 16 * rq + c, a.rows - 1) * (uint32_t)a.rb;
+    const uint32_t qoff = rbase + (g < 2 ? 16 * (kp + 4 * g) : 128 + 16 * ((kp >> 1) + 2 * (g - 2)));
+    auto copy_raw = [&](int b, Q6Stage& S) __attribute__((always_inline)) {
+        b = min(b, nb - 1);
+        const uint8_t* src = a.w + (size_t)b * 208;
+        lds_copy16_s(src, qoff, lds_addr(&S.raw[w].q[0][0]));
+        if (lane < 16) {
+            lds_copy16_s(src + 192, rbase, lds_addr(&S.raw[w].sc[0][0]));
+            lds_copy4_s(a.w, rbase + (uint32_t)(nb * 208 + (b & ~1) * 2), lds_addr(&S.raw[w].dw[0]));
         }
-        const f4v z = {0.0f, 0.0f, 0.0f, 0.0f};
+    };
+
+    // [lane k = kp + 4 kk][token tile tt][i]
+    float accF[2][4][4], accM[2][4][4];
 #pragma unroll
-        for (int k = 0; k < 8; k++) {
-            Q6Raw8 raw;
-            raw.ql = *(const uint2*)(q + o_ql + 16 * k);
-            raw.qh = *(const uint32_t*)(q + o_qh + 8 * k);
-            raw.sc = *(const uint32_t*)(q + o_sc);
-            h8v bv[2];
-            float x0[2], x8[2];
+    for (int kk = 0; kk < 2; kk++)
 #pragma unroll
-            for (int n = 0; n < 2; n++) {
-                bv[n] = *(const h8v*)(bt + o_b + n * 8192 + k * 1024);
-                x0[n] = *(const float*)(xt + o_x + n * 1024 + 4 * k) * 32.0f;  // ScaleF32(xs, 32)
-                x8[n] = *(const float*)(xt + o_x + n * 1024 + 4 * (8 + k)) * 32.0f;
+        for (int tt = 0; tt < 4; tt++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) accF[kk][tt][i] = accM[kk][tt][i] = 0.0f;
+
+    Q6Masks m{0x00f000f0u, 0x00300030u, 0x00c000c0u, 0x54005400u};
+    asm("" : "+s"(m.nib), "+s"(m.lo2), "+s"(m.hi2), "+v"(m.exp));
+    const h2v quarter = {(_Float16)1.0f, (_Float16)0.25f}, m64 = {(_Float16)-64.0f, (_Float16)-64.0f};
+    const h2v m1152 = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+    // f16 operands of the 8 codes of a dword pair (quads 2g, 2g + 1), scales S
+    auto lows = [&](uint2 ql, h2v S, uint32_t s0, uint32_t s1) __attribute__((always_inline)) {
+        const h2v N = S * m64;  // (64 + q) S + N, exact: below 2^11 after 9 + 8 bits
+        const h2v sl = {S[0], S[0]}, nl = {N[0], N[0]}, sh = {S[1], S[1]}, nh = {N[1], N[1]};
+        const h2v p0 = __builtin_bit_cast(h2v, ((ql.x << s0) & m.nib) | m.exp), p1 = __builtin_bit_cast(h2v, ((ql.x >> s1) & m.nib) | m.exp);
+        const h2v p2 = __builtin_bit_cast(h2v, ((ql.y << s0) & m.nib) | m.exp), p3 = __builtin_bit_cast(h2v, ((ql.y >> s1) & m.nib) | m.exp);
+        const h2v a0 = __builtin_elementwise_fma(p0, sl, nl), a1 = __builtin_elementwise_fma(p1, sl, nl);
+        const h2v a2 = __builtin_elementwise_fma(p2, sh, nh), a3 = __builtin_elementwise_fma(p3, sh, nh);
+        return h8v{a0[0], a0[1], a1[0], a1[1], a2[0], a2[1], a3[0], a3[1]};
+    };
+    auto highs = [&](uint32_t qh, h2v S, uint32_t s0, uint32_t s1) __attribute__((always_inline)) {
+        const h2v T = S * quarter, N = T * m64;  // quad 2g + 1's field sits two bits higher: 64 + 4 q
+        const h2v sl = {T[0], T[0]}, nl = {N[0], N[0]}, sh = {T[1], T[1]}, nh = {N[1], N[1]};
+        const uint32_t y0 = qh << s0, y1 = qh >> s1;
+        const h2v p0 = __builtin_bit_cast(h2v, (y0 & m.lo2) | m.exp), p1 = __builtin_bit_cast(h2v, (y1 & m.lo2) | m.exp);
+        const h2v p2 = __builtin_bit_cast(h2v, (y0 & m.hi2) | m.exp), p3 = __builtin_bit_cast(h2v, (y1 & m.hi2) | m.exp);
+        const h2v a0 = __builtin_elementwise_fma(p0, sl, nl), a1 = __builtin_elementwise_fma(p1, sl, nl);
+        const h2v a2 = __builtin_elementwise_fma(p2, sh, nh), a3 = __builtin_elementwise_fma(p3, sh, nh);
+        return h8v{a0[0], a0[1], a1[0], a1[1], a2[0], a2[1], a3[0], a3[1]};
+    };
+
+    copy_raw(0, st[0]);
+    copy_tokens(0, st[0]);
+    copy_raw(1, st[1]);
+    wait_vmem_le<3>();
+    lds_barrier();
+    // Block b from stage S, N the other one; register 4 tt + i of an outer
+    // product is token 16 tt + 4g + i
+    auto block = [&](int b, Q6Stage& S, Q6Stage& N) __attribute__((always_inline)) {
+        copy_tokens(b + 1, N);
+        const Q6Raw& R = S.raw[w];
+        // LDS addresses are rebuilt from the lane each block: kept across
+        // blocks they would spill
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        const int g = ln >> 4, c = ln & 15, lane = ln;
+        const uint32_t s0 = 4 - 4 * (g & 1), s1 = 4 + 4 * (g & 1);  // the lane's nibble to bits 4-7
+        const int8_t* rsc = (const int8_t*)R.sc[c];
+        const uint32_t sv = *(const uint32_t*)&R.sc[c][4 * g] ^ 0x80808080u;  // s + 128
+        const float d = f16_bits_to_f32((R.dw[c] >> (16 * (b & 1))) & 0xffffu);
+        const f16v z16 = {0.0f};
+#pragma unroll
+        for (int kk = 0; kk < 2; kk++) {
+            const float x0 = S.x16[kk][lane][kp] * 32.0f;      // ScaleF32(xs, 32)
+            const float x8 = S.x16[2 + kk][lane][kp] * 32.0f;
+            const float sk = (float)rsc[kp + 4 * kk], sk8 = (float)rsc[8 + kp + 4 * kk];
+            f16v P = __builtin_amdgcn_mfma_f32_16x16x1f32(x0, sk, z16, 0, 0, 0);  // VMULPS
+            P = __builtin_amdgcn_mfma_f32_16x16x1f32(x8, sk8, P, 0, 0, 0);        // VFMADD231PS
+#pragma unroll
+            for (int tt = 0; tt < 4; tt++) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) accM[kk][tt][i] = fmaf(d, P[4 * tt + i], accM[kk][tt][i]);
+                pin4(accM[kk][tt]);
             }
-            const f4v sk = *(const f4v*)(sct + o_k + k * 256);
-            const f4v sk8 = *(const f4v*)(sct + o_k + (8 + k) * 256);
-            h8v alo, ahi;
-            q6_operands(raw, k, g, alo, ahi);
-#pragma unroll
-            for (int n = 0; n < 2; n++) {
-                const f4v plo = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bv[n], z, 0, 0, 0);
-                const f4v phi = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bv[n], z, 0, 0, 0);
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const float iv = fmaf(phi[i], 16.0f, plo[i]);  // float(I)
-                    float o2 = sk[i] * x0[n];                      // VMULPS
-                    o2 = fmaf(sk8[i], x8[n], o2);                  // VFMADD231PS
-                    accM[n][k][i] = fmaf(dv[i], o2, accM[n][k][i]);
-                    accF[n][k][i] = fmaf(iv, dxs[n][i], accF[n][k][i]);
-                }
-            }
-            // lane k's accumulators final here: without the pin the compiler
-            // interleaves the eight lanes' chains past the register file
-#pragma unroll
-            for (int n = 0; n < 2; n++)
-                asm volatile("" : "+v"(accF[n][k][0]), "+v"(accF[n][k][1]), "+v"(accF[n][k][2]),
-                             "+v"(accF[n][k][3]), "+v"(accM[n][k][0]), "+v"(accM[n][k][1]),
-                             "+v"(accM[n][k][2]), "+v"(accM[n][k][3]));
             __builtin_amdgcn_sched_barrier(0);
         }
-        wait_vmem_le<0>();  // block b + 1's copies, issued before this block's products
-        lds_barrier();
-        q6_prep(tid, min(b + 1, nb - 1), st[(b + 1) & 1]);
+        const f16v dxs = __builtin_amdgcn_mfma_f32_16x16x1f32(S.xs[lane], d, z16, 0, 0, 0);
+        // step u = (kk, tt); the next step's activations are read ahead
+        const f4v z = {0.0f, 0.0f, 0.0f, 0.0f};
+        auto acts = [&](int u) __attribute__((always_inline)) {
+            return *(const h8v*)(S.b16 + (((u & 3) * 8 + kp + 4 * (u >> 2)) * 4 + g) * 256 + c * 16);
+        };
+        h8v bv[2], wl, wh;
+        bv[0] = acts(0);
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const int kk = u >> 2, tt = u & 3;
+            if (u < 7) bv[(u + 1) & 1] = acts(u + 1);
+            if (tt == 0) {
+                const uint2 ql = *(const uint2*)&R.q[16 * kk + c][8 * (g >> 1)];
+                const uint32_t qh = *(const uint32_t*)&R.q[32 + 16 * kk + c][8 * (kp & 1) + 4 * (g >> 1)];
+                const h2v sc = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x64646464u, sv, kk ? 0x04030401u : 0x04020400u)) + m1152;
+                wl = lows(ql, sc, s0, s1);
+                wh = highs(qh, sc, s0, s1);
+            }
+            const f4v lo = __builtin_amdgcn_mfma_f32_16x16x32_f16(bv[u & 1], wl, z, 0, 0, 0);
+            const f4v hi = __builtin_amdgcn_mfma_f32_16x16x32_f16(bv[u & 1], wh, z, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float iv = fmaf(hi[i], 16.0f, lo[i]);  // float(I)
+                accF[kk][tt][i] = fmaf(iv, dxs[4 * tt + i], accF[kk][tt][i]);
+            }
+            pin4(accF[kk][tt]);
+            __builtin_amdgcn_sched_barrier(0);
+            // the wave's last read of its raw rows has returned: refill their
+            // slot two blocks ahead
+            if (u == 4) copy_raw(b + 2, S);
+        }
+        wait_vmem_le<3>();  // block b + 1 has landed (all but the raw copies of b + 2)
         wait_lgkm0();
         lds_barrier();
+    };
+#pragma unroll 1
+    for (int b = 0;;) {
+        block(b, st[0], st[1]);
+        if (++b == nb) break;
+        block(b, st[1], st[0]);
+        if (++b == nb) break;
     }
+    wait_vmem_le<0>();  // the last copies, never read
+    lds_barrier();
+    // the tree, as in the Q4_K kernel
+    float* ex = (float*)dyn;  // [rq][kp][tt][i][lane]
 #pragma unroll
-    for (int n = 0; n < 2; n++) {
-        const int t = tok0 + 32 * tg + 16 * n + c;
-        if (t >= a.p) continue;
+    for (int tt = 0; tt < 4; tt++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const int rr = row0 + 16 * rg + 4 * g + i;
-            if (rr >= a.rows) continue;
-            float v[8];
-#pragma unroll
-            for (int k = 0; k < 8; k++) v[k] = accF[n][k][i] - accM[n][k][i];
-            const float s0 = v[0] + v[4], s1 = v[1] + v[5], s2 = v[2] + v[6], s3 = v[3] + v[7];
-            a.out[(size_t)t * a.out_stride + rr] = (s0 + s1) + (s2 + s3);
+            const float v0 = accF[0][tt][i] - accM[0][tt][i], v1 = accF[1][tt][i] - accM[1][tt][i];
+            ex[((w * 4 + tt) * 4 + i) * 64 + lane] = v0 + v1;
         }
-    }
+    wait_lgkm0();
+    lds_barrier();
+    lanes_store(a, ex, row0, tok0, rq, kp, lane);
 }
 
 int launch_q6k_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,
@@ -888,9 +873,9 @@ int launch_q6k_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const 
         return fail(GLLM_EINVAL, "prefill: Q6_K tiles need > %d tokens, blocks %% 8 == 0, < 4 GiB",
                     kTiledMinP);
     PfArgs a{d_w, rb, rows, blocks, act, p, out, out_stride};
-    const TlMap mp = tl_map(rows, p);
-    hipLaunchKernelGGL(prefill_q6k_tiled_kernel, dim3(8 * mp.tg_size * mp.rg_size), dim3(512), 0, s, a,
-                       mp);
+    constexpr size_t lds = 2 * sizeof(Q6Stage);
+    static const bool ok = lanes_lds((const void*)prefill_q6k_lanes_kernel, lds);
+    GLLM_TRY((launch_lanes<lds>(prefill_q6k_lanes_kernel, ok, a, s)));
     GLLM_HIP(hipGetLastError());
     return GLLM_OK;
 }

@@ -56,6 +56,14 @@ def test_prefill_tile_edges(hip, rows, cols, p):
     assert_bits(w.matvec_batch(xs), amd64(data, xs, rows, cols), f"{rows}x{cols} p={p}")
 
 
+@pytest.mark.parametrize("rows,cols,p", [(1, 2048, 17), (65, 2048, 65), (64, 4096, 128), (130, 2048, 129)])
+def test_prefill_q6k_tile_edges(hip, rows, cols, p):
+    data, _ = quant_matrix(ref.Q6_K, rows, cols, 910 + rows)
+    w = hip.Weight.from_host(data, ref.Q6_K, rows, cols)
+    xs = normal(911 + p, (p, cols))
+    assert_bits(w.matvec_batch(xs), amd64(data, xs, rows, cols, ref.Q6_K), f"{rows}x{cols} p={p}")
+
+
 def test_prefill_degenerate_blocks(hip):
     """All-zero tokens, zero 256-blocks inside a token, a lone large value and
     NaN-free extremes (q8kQuantize's scale-0 blocks, quant_q8k_portable.go:36-62)."""
