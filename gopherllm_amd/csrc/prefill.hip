@@ -363,7 +363,7 @@ __device__ __forceinline__ void sb_scale_min(const u4v h, int j, uint32_t& sc, u
 // for the kernel before it, which staged the dequantised f16 weights in LDS
 // and ran all eight lanes of a 16 x 32 tile in a wave (two waves per SIMD,
 // LDS traffic 370 KB per block), 195 us with eight waves of 32 rows x 64
-// tokens (two per SIMD), 202 us with eight waves of 16 rows x 128 tokens, 180
+// tokens (two per SIMD), 202 us with eight waves of 16 rows x 128 tokens, 175
 // us like this.  What is left is issue: per wave and block 64 chain steps, 40
 // VALU operations of dequantisation and 11 matrix instructions, which hardly
 // overlap the VALU on this part (a 16x16x32 f16 MFMA and four fmas take 30
@@ -439,6 +439,16 @@ __device__ __forceinline__ h8v dequant_nib(uint32_t w, h2v s, h2v n, const NibMa
     const h2v a0 = __builtin_elementwise_fma(p0, sl, nl), a1 = __builtin_elementwise_fma(p1, sl, nl);
     const h2v a2 = __builtin_elementwise_fma(p2, sh, nh), a3 = __builtin_elementwise_fma(p3, sh, nh);
     return h8v{a0[0], a0[1], a1[0], a1[1], a2[0], a2[1], a3[0], a3[1]};
+}
+
+// An f16 factor of many chain steps, converted once.  Left alone the compiler
+// folds the conversion into each fma as v_fma_mix_f32, which issues more
+// slowly (14336 x 4096 x 512 with / without: Q8_0 348 / 305 us, Q4_K 180 /
+// 175 us; Q6_K 4096 x 14336 x 333 259 / 245 us).
+__device__ __forceinline__ float factor_f16(uint32_t h) {
+    float v = f16_bits_to_f32(h & 0xffffu);
+    asm("" : "+v"(v));
+    return v;
 }
 
 // A chain step ends here: the compiler may not sink it past this point.
@@ -523,7 +533,7 @@ __global__ __launch_bounds__(1024) void prefill_q4k_lanes_kernel(PfArgs a, TlMap
         r.nd[0] = *(const uint32_t*)&S.raw[w][c][4 * g];
         r.nd[1] = *(const uint32_t*)&S.raw[w][16 + c][4 * g];
         r.d = f16_bits_to_f32(h.x & 0xffffu);
-        r.dm = f16_bits_to_f32(h.x >> 16);
+        r.dm = factor_f16(h.x >> 16);
         r.mn[0] = (float)__builtin_amdgcn_ubfe(h.z, 8 * kp, 6);
         r.mn[1] = (float)((__builtin_amdgcn_ubfe(h.z, 8 * kp + 6, 2) << 4) | __builtin_amdgcn_ubfe(h.w, 8 * kp + 4, 4));
         const uint32_t sb = (((hs >> sh0) & low) | ((h.y >> (sh0 + 2)) & ~low)) & 0x3f3fu;
@@ -674,7 +684,7 @@ static int launch_q4k_lanes(const PfArgs& a, hipStream_t s) {
 // need rows * rb < 4 GiB and 16-byte aligned blocks (blocks % 8 == 0).
 // With the quantiser launch, 4096 x 14336 x 333 (1.5 rounds of workgroups) and
 // 14336 x 4096 x 512: 473 and 490 us for 64 x 64 tiles that ran all eight
-// lanes in a wave and built the A operands twice, 259 and 273 us like this.
+// lanes in a wave and built the A operands twice, 245 and 260 us like this.
 // Bound by issue: per wave and block 96 chain steps, about 70 operations of
 // dequantisation and 21 matrix instructions.
 struct Q6Raw {
@@ -790,7 +800,7 @@ __global__ __launch_bounds__(1024) void prefill_q6k_lanes_kernel(PfArgs a, TlMap
         const uint32_t s0 = 4 - 4 * (g & 1), s1 = 4 + 4 * (g & 1);  // the lane's nibble to bits 4-7
         const int8_t* rsc = (const int8_t*)R.sc[c];
         const uint32_t sv = *(const uint32_t*)&R.sc[c][4 * g] ^ 0x80808080u;  // s + 128
-        const float d = f16_bits_to_f32((R.dw[c] >> (16 * (b & 1))) & 0xffffu);
+        const float d = factor_f16(R.dw[c] >> (16 * (b & 1)));
         const f16v z16 = {0.0f};
 #pragma unroll
         for (int kk = 0; kk < 2; kk++) {
@@ -880,135 +890,161 @@ int launch_q6k_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const 
     return GLLM_OK;
 }
 
-// --- Q8_0, more than 16 activation rows: 64 x 64 staged tiles ---------------
+// --- Q8_0, more than 16 activation rows: one pair of AVX2 lanes per wave ----
 // q8_0DotQ8KRow (kernels_amd64.s Q80CHUNK) per AVX2 lane k of a 256-element
 // group: for its eight 32-value blocks q in order
 //   acc12 = fma(d_q, float(I_qk), acc12)   I_qk: the exact dot of the lane's
 //                                           4 weight and 4 activation bytes
 // then acc11[k] = fma(xscale, acc12, acc11[k]) and tree8(acc11).  The
-// per-block float chain sets the cost (25 VALU operations per row, token,
-// group and lane with v_dot4_i32_i8 for I), so this kernel stays on the
-// vector units and reads every weight byte once per 64 tokens.
-// Workgroup: 64 rows x 64 tokens, 512 threads; thread (rp, tq) = (t >> 4,
-// t & 15) owns rows 2 rp, 2 rp + 1 and tokens tq + 16 j (j < 4).  Per group,
-// double-buffered in LDS: the 64 rows' 272-byte groups as stored (8 f16 d,
-// then lane k's 8 dwords at 16 + 32 k) and the 64 tokens' q8perm bytes
-// (lane k's 32 at 32 k) in 272-byte rows, both copied global -> LDS one
-// group ahead, and the tokens' xscales.
-constexpr int kQ80Pieces = 64 * 17;  // 16-byte pieces of 64 rows (or tokens) x 272 bytes
-struct Q80Stage {
-    uint8_t w[kQ80Pieces * 16];  // [row][272]
-    uint8_t q[kQ80Pieces * 16];  // [token][272]: 256 q8perm bytes, 16 unused
-    float xs[64];
+// float chain over q is nine VALU steps per product and lane; the dots in
+// front of it are matrix products with K = 4, so v_mfma_f32_16x16x4 (f16,
+// four blocks) delivers float(I) for four q of a 16 x 16 tile at once, exact
+// (integers below 2^17) where the VALU takes a v_dot4_i32_i8 and a
+// conversion each.
+// The split of the work is prefill_q4k_lanes_kernel's: wave (rq, kp) owns 16
+// rows, 64 tokens and the lanes kp and kp + 4.  A lane's 16 bytes of B16 hold
+// blocks 2g (first four halves) and 2g + 1, so the even and the odd q are one
+// instruction each.
+// With the quantiser launch, 14336 x 4096 x 512: 718 us for 64 x 64 tiles on
+// the vector units (25 VALU operations per lane product), 305 us like this.
+struct Q80Raw {
+    uint8_t q[64][16];  // [32 (k / 4) + 16 half + row c]
+    uint8_t d[16][16];  // [row c]: eight f16 scales
 };
+struct Q80Stage {
+    uint8_t b16[4 * 8 * 4 * 256];  // [token tile][lane k][group g][token c][8 halves]
+    float xs[kTlTok];
+    Q80Raw raw[16];                // [wave]
+};
+typedef _Float16 h4v __attribute__((ext_vector_type(4)));
 
-// Group b's operands into S: two 1 KB pieces of the rows and two of the
-// tokens per wave, the remaining 64 row pieces on wave 0, 64 token pieces on
-// wave 1, the xscales on wave 2: five copies on waves 0-2, four on 3-7.
-__device__ __forceinline__ void q80_copy(const PfArgs& a, int w, int lane, int row0, int tok0, int b,
-                                         Q80Stage& S) {
-    const int cols = a.blocks * 256;
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-        if (i == 2 && w != 0) break;  // wave-uniform
-        const int pc = (i < 2 ? 128 * w + 64 * i : 1024) + lane, r = pc / 17, off = (pc % 17) * 16;
-        const size_t row = (size_t)min(row0 + r, a.rows - 1);
-        lds_copy16_s(a.w, (uint32_t)(row * a.rb + (size_t)b * 272 + off), lds_addr(S.w + 16 * (pc - lane)));
-    }
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-        if (i == 2 && w != 1) break;  // wave-uniform
-        const int pc = (i < 2 ? 128 * w + 64 * i : 1024) + lane, t = pc / 17, off = min((pc % 17) * 16, 240);
-        const size_t tok = (size_t)min(tok0 + t, a.p - 1);
-        lds_copy16_s(a.act.q8perm, (uint32_t)(tok * cols + (size_t)b * 256 + off), lds_addr(S.q + 16 * (pc - lane)));
-    }
-    if (w == 2)
-        lds_copy4_s(a.act.xscale + b, (uint32_t)min(tok0 + lane, a.p - 1) * a.blocks * 4, lds_addr(&S.xs[0]));
-}
-
-__global__ __launch_bounds__(512) void prefill_q8_0_tiled_kernel(PfArgs a, TlMap mp) {
-    __shared__ __align__(16) Q80Stage st[2];
+__global__ __launch_bounds__(1024) void prefill_q8_0_lanes_kernel(PfArgs a, TlMap mp) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t dyn[];
+    Q80Stage* const st = (Q80Stage*)dyn;
     const int id = blockIdx.x, xcd = id & 7, local = id >> 3;
     const int lt = local % mp.tg_size, lrow = local / mp.tg_size;
     const int ttile = (xcd % mp.h) * mp.tg_size + lt, rtile = (xcd / mp.h) * mp.rg_size + lrow;
     if (lrow >= mp.rg_size || ttile >= mp.tok_tiles || rtile >= mp.row_tiles) return;  // whole workgroup
-    const int row0 = rtile * kTlRows, tok0 = ttile * kTlTok;
-    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int rp = tid >> 4, tq = tid & 15;
+    const int row0 = rtile * kTlRows, tok0 = ttile * kTlTok, tile0 = tok0 / 16;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kp = w & 3, rq = w >> 2;
     const int nb = a.blocks;
 
-    float acc11[2][4][8];
-#pragma unroll
-    for (int r = 0; r < 2; r++)
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-#pragma unroll
-            for (int k = 0; k < 8; k++) acc11[r][j][k] = 0.0f;
+    // Copies of one group's tokens: two 1 KB pieces of B16 (as in the Q4_K
+    // kernel) and the xscales (wave 0)
+    const int last = a.act.tiles - 1;
+    const size_t bstep = (size_t)a.act.tiles * 8192;
+    const uint8_t* bsrc = (const uint8_t*)a.act.b16t + (size_t)min(tile0 + rq, last) * 8192 + 2048 * kp;
+    const uint32_t xoff = (uint32_t)min(tok0 + lane, a.p - 1) * nb * 4;
+    auto copy_tokens = [&](int b, Q80Stage& S) __attribute__((always_inline)) {
+        b = min(b, nb - 1);
+        const uint8_t* src = bsrc + b * bstep;
+        const uint32_t dst = lds_addr(S.b16 + rq * 8192 + 2048 * kp);
+        lds_copy16_s(src, 16 * lane, dst);
+        lds_copy16_s(src + 1024, 16 * lane, dst + 1024);
+        if (w == 0) lds_copy4_s(a.act.xscale + b, xoff, lds_addr(&S.xs[0]));
+    };
+    // The wave's rows: two copies
+    const uint32_t rbase = (uint32_t)min(row0 + 16 * rq + (lane & 15), a.rows - 1) * (uint32_t)a.rb;
+    const uint32_t qoff = rbase + 16 + 32 * (kp + 4 * (lane >> 5)) + 16 * ((lane >> 4) & 1);
+    auto copy_raw = [&](int b, Q80Stage& S) __attribute__((always_inline)) {
+        const uint8_t* src = a.w + (size_t)min(b, nb - 1) * 272;
+        lds_copy16_s(src, qoff, lds_addr(&S.raw[w].q[0][0]));
+        if (lane < 16) lds_copy16_s(src, rbase, lds_addr(&S.raw[w].d[0][0]));
+    };
 
-    q80_copy(a, w, lane, row0, tok0, 0, st[0]);
-    wait_vmem_le<0>();
+    float acc[2][4][4];  // acc11 of [lane k = kp + 4 kk][token tile tt][i]
+#pragma unroll
+    for (int kk = 0; kk < 2; kk++)
+#pragma unroll
+        for (int tt = 0; tt < 4; tt++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[kk][tt][i] = 0.0f;
+
+    uint32_t bytes = 0x00ff00ffu, exp = 0x64006400u;
+    asm("" : "+s"(bytes), "+v"(exp));
+    const h2v m1152 = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+    // a dword of int8 as f16, bytes 0, 2, 1, 3: 1024 + (v + 128) - 1152
+    auto halves = [&](uint32_t v) __attribute__((always_inline)) {
+        v ^= 0x80808080u;
+        const h2v p0 = __builtin_bit_cast(h2v, (v & bytes) | exp) + m1152;
+        const h2v p1 = __builtin_bit_cast(h2v, ((v >> 8) & bytes) | exp) + m1152;
+        return h4v{p0[0], p0[1], p1[0], p1[1]};
+    };
+
+    copy_raw(0, st[0]);
+    copy_tokens(0, st[0]);
+    copy_raw(1, st[1]);
+    wait_vmem_le<2>();
     lds_barrier();
-#pragma unroll 1
-    for (int b = 0; b < nb; b++) {
-        // unconditional copies (clamped to the last group, into the stage
-        // not read this iteration): five on waves 0-2, four on 3-7
-        q80_copy(a, w, lane, row0, tok0, min(b + 1, nb - 1), st[(b + 1) & 1]);
-        const Q80Stage& S = st[b & 1];
-        float d[2][8], xs[4];
+    auto block = [&](int b, Q80Stage& S, Q80Stage& N) __attribute__((always_inline)) {
+        copy_tokens(b + 1, N);
+        int ln = lane;  // LDS addresses are rebuilt each block: kept across blocks they would spill
+        asm volatile("" : "+v"(ln));
+        const int g = ln >> 4, c = ln & 15;
+        const Q80Raw& R = S.raw[w];
+        const u4v dh = *(const u4v*)&R.d[c][0];
+        float d[8];
 #pragma unroll
-        for (int r = 0; r < 2; r++) {
-            const uint4 dh = *(const uint4*)(S.w + (2 * rp + r) * 272);
-            const uint32_t dw[4] = {dh.x, dh.y, dh.z, dh.w};
+        for (int q = 0; q < 8; q++) d[q] = factor_f16(dh[q >> 1] >> (16 * (q & 1)));
+        // step u = (kk, tt): token 16 tt + 4g + i, weight row 16 rq + c
+        auto acts = [&](int u) __attribute__((always_inline)) {
+            return *(const h8v*)(S.b16 + (((u & 3) * 8 + kp + 4 * (u >> 2)) * 4 + g) * 256 + c * 16);
+        };
+        h8v bv[2];
+        h4v we, wo;
+        bv[0] = acts(0);
 #pragma unroll
-            for (int q = 0; q < 8; q++) d[r][q] = f16_bits_to_f32((dw[q >> 1] >> (16 * (q & 1))) & 0xffffu);
-        }
+        for (int u = 0; u < 8; u++) {
+            const int kk = u >> 2, tt = u & 3;
+            if (u < 7) bv[(u + 1) & 1] = acts(u + 1);
+            if (tt == 0) {
+                const uint2 v = *(const uint2*)&R.q[32 * kk + 16 * (g >> 1) + c][8 * (g & 1)];
+                we = halves(v.x);
+                wo = halves(v.y);
+            }
+            const f4v xs = *(const f4v*)&S.xs[16 * tt + 4 * g];
+            const h8v x = bv[u & 1];
+            const f16v z16 = {0.0f};
+            const f16v E = __builtin_amdgcn_mfma_f32_16x16x4f16(h4v{x[0], x[1], x[2], x[3]}, we, z16, 0, 0, 0);
+            const f16v O = __builtin_amdgcn_mfma_f32_16x16x4f16(h4v{x[4], x[5], x[6], x[7]}, wo, z16, 0, 0, 0);
+            float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int j = 0; j < 4; j++) xs[j] = S.xs[tq + 16 * j];
+            for (int q = 0; q < 4; q++) {
 #pragma unroll
-        for (int k = 0; k < 8; k++) {
-            int wv[2][8], qv[4][8];
+                for (int i = 0; i < 4; i++) y[i] = fmaf(E[4 * q + i], d[2 * q], y[i]);  // VFMADD231PS
 #pragma unroll
-            for (int r = 0; r < 2; r++) {
-                const int4 lo = *(const int4*)(S.w + (2 * rp + r) * 272 + 16 + 32 * k);
-                const int4 hi = *(const int4*)(S.w + (2 * rp + r) * 272 + 32 + 32 * k);
-                wv[r][0] = lo.x; wv[r][1] = lo.y; wv[r][2] = lo.z; wv[r][3] = lo.w;
-                wv[r][4] = hi.x; wv[r][5] = hi.y; wv[r][6] = hi.z; wv[r][7] = hi.w;
+                for (int i = 0; i < 4; i++) y[i] = fmaf(O[4 * q + i], d[2 * q + 1], y[i]);
             }
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int4 lo = *(const int4*)(S.q + (tq + 16 * j) * 272 + 32 * k);
-                const int4 hi = *(const int4*)(S.q + (tq + 16 * j) * 272 + 32 * k + 16);
-                qv[j][0] = lo.x; qv[j][1] = lo.y; qv[j][2] = lo.z; qv[j][3] = lo.w;
-                qv[j][4] = hi.x; qv[j][5] = hi.y; qv[j][6] = hi.z; qv[j][7] = hi.w;
-            }
-#pragma unroll
-            for (int r = 0; r < 2; r++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    float acc12 = 0.0f;
-#pragma unroll
-                    for (int q = 0; q < 8; q++)
-                        acc12 = fmaf((float)sdot4(wv[r][q], qv[j][q], 0), d[r][q], acc12);  // VFMADD231PS
-                    acc11[r][j][k] = fmaf(acc12, xs[j], acc11[r][j][k]);
-                }
+            for (int i = 0; i < 4; i++) acc[kk][tt][i] = fmaf(y[i], xs[i], acc[kk][tt][i]);
+            pin4(acc[kk][tt]);
             __builtin_amdgcn_sched_barrier(0);
+            // the wave's last read of its raw rows has returned: refill their
+            // slot two groups ahead
+            if (u == 4) copy_raw(b + 2, S);
         }
-        wait_vmem_le<0>();  // group b + 1's copies, issued before this group's products
+        wait_vmem_le<2>();  // group b + 1 has landed (all but the raw copies of b + 2)
+        wait_lgkm0();
         lds_barrier();
+    };
+#pragma unroll 1
+    for (int b = 0;;) {
+        block(b, st[0], st[1]);
+        if (++b == nb) break;
+        block(b, st[1], st[0]);
+        if (++b == nb) break;
     }
+    wait_vmem_le<0>();  // the last copies, never read
+    lds_barrier();
+    float* ex = (float*)dyn;  // [rq][kp][tt][i][lane]
 #pragma unroll
-    for (int r = 0; r < 2; r++) {
-        const int rr = row0 + 2 * rp + r;
-        if (rr >= a.rows) continue;
+    for (int tt = 0; tt < 4; tt++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int t = tok0 + tq + 16 * j;
-            if (t >= a.p) continue;
-            const float* v = acc11[r][j];
-            const float s0 = v[0] + v[4], s1 = v[1] + v[5], s2 = v[2] + v[6], s3 = v[3] + v[7];
-            a.out[(size_t)t * a.out_stride + rr] = (s0 + s1) + (s2 + s3);
-        }
-    }
+        for (int i = 0; i < 4; i++) ex[((w * 4 + tt) * 4 + i) * 64 + lane] = acc[0][tt][i] + acc[1][tt][i];
+    wait_lgkm0();
+    lds_barrier();
+    lanes_store(a, ex, row0, tok0, rq, kp, lane);
 }
 
 int launch_q8_0_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,
@@ -1017,9 +1053,9 @@ int launch_q8_0_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const
     if (p <= kTiledMinP || (size_t)rows * rb >= ((size_t)1 << 32) || (size_t)p * blocks * 256 >= ((size_t)1 << 32))
         return fail(GLLM_EINVAL, "prefill: Q8_0 tiles need > %d tokens and < 4 GiB operands", kTiledMinP);
     PfArgs a{d_w, rb, rows, blocks, act, p, out, out_stride};
-    const TlMap mp = tl_map(rows, p);
-    hipLaunchKernelGGL(prefill_q8_0_tiled_kernel, dim3(8 * mp.tg_size * mp.rg_size), dim3(512), 0, s,
-                       a, mp);
+    constexpr size_t lds = 2 * sizeof(Q80Stage);
+    static const bool ok = lanes_lds((const void*)prefill_q8_0_lanes_kernel, lds);
+    GLLM_TRY((launch_lanes<lds>(prefill_q8_0_lanes_kernel, ok, a, s)));
     GLLM_HIP(hipGetLastError());
     return GLLM_OK;
 }

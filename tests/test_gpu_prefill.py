@@ -1,5 +1,5 @@
-"""Batched prefill products: Q4_K and Q6_K on the matrix cores,
-Q8_0 on 64 x 64 tiles of the vector units.
+"""Batched prefill products: Q4_K, Q6_K and Q8_0 on the matrix
+cores.
 
 matvecBatchQ8 (kernels_amd64.go:470-581) evaluates q4kDotQ8KRow once per
 (row, token), so the batched result must equal the per-token row kernel bit
@@ -62,6 +62,14 @@ def test_prefill_q6k_tile_edges(hip, rows, cols, p):
     w = hip.Weight.from_host(data, ref.Q6_K, rows, cols)
     xs = normal(911 + p, (p, cols))
     assert_bits(w.matvec_batch(xs), amd64(data, xs, rows, cols, ref.Q6_K), f"{rows}x{cols} p={p}")
+
+
+@pytest.mark.parametrize("rows,cols,p", [(1, 256, 17), (65, 768, 65), (64, 512, 128), (130, 1280, 129)])
+def test_prefill_q8_0_tile_edges(hip, rows, cols, p):
+    data, _ = quant_matrix(ref.Q8_0, rows, cols, 920 + rows)
+    w = hip.Weight.from_host(data, ref.Q8_0, rows, cols)
+    xs = normal(921 + p, (p, cols))
+    assert_bits(w.matvec_batch(xs), amd64(data, xs, rows, cols, ref.Q8_0), f"{rows}x{cols} p={p}")
 
 
 def test_prefill_degenerate_blocks(hip):
