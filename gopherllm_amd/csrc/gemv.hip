@@ -2185,6 +2185,18 @@ static bool q6k_tiled_fits(const ActQ8& act, int p, const gllm_hip_weight* w) {
            (size_t)w->rows * w->row_bytes < ((size_t)1 << 32);
 }
 
+// The small-batch matrix-core kernel applies (launch_small_lanes).  Its cost
+// hardly depends on the tokens, the row kernels' does: at 14336 x 4096 Q4_K
+// takes 13.2 / 16.2 us at 2 / 4 tokens on the row kernels and 15.8 / 16.3 here
+// (at 4096 columns they walk a row in few steps; 4096 x 14336 at 2 tokens
+// takes 25.1 there and 18.3 here); Q6_K 4096 x 14336 takes 24.5 / 29.4 / 33.1
+// at 2 / 3 / 4 and 14336 x 4096 18.2 / 21.2 / 24.1, here 26.5 and 23.8.
+static bool small_batch_fits(const ActQ8& act, int p, const gllm_hip_weight* w) {
+    if (!act.rec || p < 2 || (size_t)w->rows * w->row_bytes >= ((size_t)1 << 32)) return false;
+    if (w->type == GLLM_TYPE_Q4_K) return p > 4 || w->cols > 4096;
+    return w->type == GLLM_TYPE_Q6_K && w->blocks % 8 == 0 && p >= 4;
+}
+
 int run_gemv(int n, gllm_hip_weight* const* ws, const ActQ8& act, int p, float* const* outs,
              const int* strides, hipStream_t s, const float* xf, const NormIn* ni = nullptr,
              const ArgmaxOut* am = nullptr) {
@@ -2226,6 +2238,12 @@ int run_gemv(int n, gllm_hip_weight* const* ws, const ActQ8& act, int p, float* 
     }
     j.wg_begin[n] = wg;
     if (wg == 0) return GLLM_OK;
+    if (small_batch_fits(act, p, w0)) {
+        for (int i = 0; i < n; i++)
+            GLLM_TRY(launch_small_lanes(w0->type == GLLM_TYPE_Q6_K, ws[i]->d_data, ws[i]->row_bytes, ws[i]->rows,
+                                        ws[i]->blocks, act, p, outs[i], j.out_stride[i], s));
+        return GLLM_OK;
+    }
     if (w0->type == GLLM_TYPE_Q4_K && p >= kMfmaMinTok) {
         // batched prefill: matrix-core products, same bits as the row kernel
         for (int i = 0; i < n; i++)
@@ -2295,6 +2313,8 @@ int gemv_f32(int n, gllm_hip_weight* const* ws, const float* d_xs, int p, float*
         } else {
             if (!quantised) {
                 act_carve(act_buf, cols, p, &act);
+                // records only for a weight that reads them
+                if (std::none_of(ws + i, ws + n, [&](auto* w) { return small_batch_fits(act, p, w); })) act.rec = nullptr;
                 GLLM_TRY(launch_q8k_prep(d_xs, cols, p, act, s));
                 quantised = true;
             }
@@ -2412,6 +2432,7 @@ int gemv_silu_f32(gllm_hip_weight* w, const float* gate, const float* up, int p,
     }
     ActQ8 act;
     act_carve(act_buf, w->cols, p, &act);
+    if (!small_batch_fits(act, p, w)) act.rec = nullptr;
     GLLM_TRY(launch_q8k_prep_silu(gate, up, w->cols, p, act, s));
     return run_gemv(1, ws, act, p, outs, nullptr, s, nullptr);
 }

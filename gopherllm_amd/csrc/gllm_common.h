@@ -63,9 +63,19 @@ struct ActQ8 {
     uint16_t* b16t;
     float* xs32t;    // xs32 of the same batches as [block][tile][lane k][token c]
     int tiles;       // ceil(p / 16) when b16t is set
+    // Batches of 2 .. kTiledMinP rows of up to kSmallCols columns carry what
+    // one wave of the small-batch kernels reads of a block as one record of
+    // small_rec(p) bytes instead, [block][lane pair k, k + 4]; see SmallRec.
+    uint8_t* rec;
     int cols, p;
 };
 constexpr int kTiledMinP = 16;
+constexpr int kSmallCols = 65536;  // keeps act_bytes of the small batches under 4 MiB
+__host__ __device__ __forceinline__ int small_pt(int p) { return p <= 8 ? 8 : 16; }
+// A record for pt (8 or 16) tokens, zero past p, q8 as f16 in b16t's order:
+//   f16 b16[2 lanes][4 groups g][pt][8]; f32 xs32[2 lanes][pt]; f32 xscale[pt];
+//   f32 xs16[4: k, k + 4, k + 8, k + 12][pt]
+__host__ __device__ __forceinline__ int small_rec(int pt) { return pt * 128 + pt * 28; }
 // Place, among the eight halves, of byte kappa % 8: bytes 0, 2, 1, 3 of each
 // weight dword, the order in which two masks of the dword give the pairs.
 __host__ __device__ __forceinline__ int b16_slot(int kappa) {
@@ -82,6 +92,10 @@ int launch_q4k_mfma(const uint8_t* d_w, size_t rb, int rows, int blocks, const A
 // tiles (p > kTiledMinP), blocks % 8 == 0 and rows * rb < 4 GiB.
 int launch_q6k_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,
                      float* out, int out_stride, hipStream_t s);
+// 2 to kTiledMinP rows of Q4_K (q6: Q6_K, blocks % 8 == 0) x Q8_K, same
+// contract; needs act.rec and rows * rb < 4 GiB.
+int launch_small_lanes(bool q6, const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,
+                       float* out, int out_stride, hipStream_t s);
 // Batched Q8_0 x Q8_K on the matrix cores, same contract; needs the f16 tiles
 // (p > kTiledMinP) and operands under 4 GiB.
 int launch_q8_0_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,

@@ -316,26 +316,6 @@ static void launch_pf(const PfArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((prefill_q4k_mfma_kernel<RW, TW>), grid, dim3(64 * RW * TW), 0, s, a);
 }
 
-// One block's per-row and per-token factors of a 16 x 16 tile (rows 0..15,
-// tokens 0..15), shared by the waves of the 16-row kernels below.
-struct SbParams {  // one block's factors: rows 0..15 and tokens 0..15 of the tile
-    float d[16], dmin[16], m[8][16];
-    float xs[16], xsum[8][16];
-};
-// getScaleMinK4 (simd.go:1672-1677): 6-bit scale and min of sub-block j
-__device__ __forceinline__ void sb_scale_min(const u4v h, int j, uint32_t& sc, uint32_t& mn) {
-    const uint32_t s03 = h.y, s47 = h.z, s811 = h.w;
-    if (j < 4) {
-        sc = (s03 >> (8 * j)) & 63u;
-        mn = (s47 >> (8 * j)) & 63u;
-    } else {
-        const int jj = j - 4;
-        const uint32_t b8 = (s811 >> (8 * jj)) & 0xffu;
-        sc = (b8 & 15u) | (((s03 >> (8 * jj + 6)) & 3u) << 4);
-        mn = (b8 >> 4) | (((s47 >> (8 * jj + 6)) & 3u) << 4);
-    }
-}
-
 // --- more than 16 activation rows: one pair of AVX2 lanes per wave ---------
 // A workgroup of sixteen waves covers 64 weight rows x 64 tokens.  The eight
 // AVX2 lanes k of a row never meet before the final tree, so the waves split
@@ -699,12 +679,38 @@ struct Q6Stage {
     Q6Raw raw[16];                 // [wave]
 };
 
-// Field of four code bytes as two half2 words of B16's byte pairs (0, 2) and
-// (1, 3): y0 / y1 hold the field at bits 4 .. of the pairs' low bytes, and
-// under f16 exponent bits of 64 they read 64 + field.
-struct Q6Masks {
+// A code field of two bytes (0 and 2, or 1 and 3) at bits 4 .. under f16
+// exponent bits of 64 reads 64 + field.
+struct Q6Masks {  // held in registers, as NibMasks
     uint32_t nib, lo2, hi2, exp;
 };
+
+// f16 operands of a lane (g, c)'s 8 codes of one AVX2 lane: quads 2g (scale
+// S[0]) and 2g + 1 (S[1]) from ql dwords 2 (g / 2), 2 (g / 2) + 1 and qh dword
+// g / 2, the nibble (bit pairs) 4 (g % 2) up.
+__device__ __forceinline__ h8v q6_lows(uint2 ql, h2v S, int g, const Q6Masks& m) {
+    const uint32_t s0 = 4 - 4 * (g & 1), s1 = 4 + 4 * (g & 1);  // the nibble to bits 4-7
+    const h2v m64 = {(_Float16)-64.0f, (_Float16)-64.0f};
+    const h2v N = S * m64;  // (64 + q) S + N is exact
+    const h2v sl = {S[0], S[0]}, nl = {N[0], N[0]}, sh = {S[1], S[1]}, nh = {N[1], N[1]};
+    const h2v p0 = __builtin_bit_cast(h2v, ((ql.x << s0) & m.nib) | m.exp), p1 = __builtin_bit_cast(h2v, ((ql.x >> s1) & m.nib) | m.exp);
+    const h2v p2 = __builtin_bit_cast(h2v, ((ql.y << s0) & m.nib) | m.exp), p3 = __builtin_bit_cast(h2v, ((ql.y >> s1) & m.nib) | m.exp);
+    const h2v a0 = __builtin_elementwise_fma(p0, sl, nl), a1 = __builtin_elementwise_fma(p1, sl, nl);
+    const h2v a2 = __builtin_elementwise_fma(p2, sh, nh), a3 = __builtin_elementwise_fma(p3, sh, nh);
+    return h8v{a0[0], a0[1], a1[0], a1[1], a2[0], a2[1], a3[0], a3[1]};
+}
+__device__ __forceinline__ h8v q6_highs(uint32_t qh, h2v S, int g, const Q6Masks& m) {
+    const uint32_t s0 = 4 - 4 * (g & 1), s1 = 4 + 4 * (g & 1);
+    const h2v quarter = {(_Float16)1.0f, (_Float16)0.25f}, m64 = {(_Float16)-64.0f, (_Float16)-64.0f};
+    const h2v T = S * quarter, N = T * m64;  // quad 2g + 1's field sits two bits higher: 64 + 4 q
+    const h2v sl = {T[0], T[0]}, nl = {N[0], N[0]}, sh = {T[1], T[1]}, nh = {N[1], N[1]};
+    const uint32_t y0 = qh << s0, y1 = qh >> s1;
+    const h2v p0 = __builtin_bit_cast(h2v, (y0 & m.lo2) | m.exp), p1 = __builtin_bit_cast(h2v, (y1 & m.lo2) | m.exp);
+    const h2v p2 = __builtin_bit_cast(h2v, (y0 & m.hi2) | m.exp), p3 = __builtin_bit_cast(h2v, (y1 & m.hi2) | m.exp);
+    const h2v a0 = __builtin_elementwise_fma(p0, sl, nl), a1 = __builtin_elementwise_fma(p1, sl, nl);
+    const h2v a2 = __builtin_elementwise_fma(p2, sh, nh), a3 = __builtin_elementwise_fma(p3, sh, nh);
+    return h8v{a0[0], a0[1], a1[0], a1[1], a2[0], a2[1], a3[0], a3[1]};
+}
 
 __global__ __launch_bounds__(1024) void prefill_q6k_lanes_kernel(PfArgs a, TlMap mp) {
     extern __shared__ __attribute__((aligned(16))) uint8_t dyn[];
@@ -759,29 +765,7 @@ __global__ __launch_bounds__(1024) void prefill_q6k_lanes_kernel(PfArgs a, TlMap
 
     Q6Masks m{0x00f000f0u, 0x00300030u, 0x00c000c0u, 0x54005400u};
     asm("" : "+s"(m.nib), "+s"(m.lo2), "+s"(m.hi2), "+v"(m.exp));
-    const h2v quarter = {(_Float16)1.0f, (_Float16)0.25f}, m64 = {(_Float16)-64.0f, (_Float16)-64.0f};
     const h2v m1152 = {(_Float16)-1152.0f, (_Float16)-1152.0f};
-    // f16 operands of the 8 codes of a dword pair (quads 2g, 2g + 1), scales S
-    auto lows = [&](uint2 ql, h2v S, uint32_t s0, uint32_t s1) __attribute__((always_inline)) {
-        const h2v N = S * m64;  // (64 + q) S + N, exact: below 2^11 after 9 + 8 bits
-        const h2v sl = {S[0], S[0]}, nl = {N[0], N[0]}, sh = {S[1], S[1]}, nh = {N[1], N[1]};
-        const h2v p0 = __builtin_bit_cast(h2v, ((ql.x << s0) & m.nib) | m.exp), p1 = __builtin_bit_cast(h2v, ((ql.x >> s1) & m.nib) | m.exp);
-        const h2v p2 = __builtin_bit_cast(h2v, ((ql.y << s0) & m.nib) | m.exp), p3 = __builtin_bit_cast(h2v, ((ql.y >> s1) & m.nib) | m.exp);
-        const h2v a0 = __builtin_elementwise_fma(p0, sl, nl), a1 = __builtin_elementwise_fma(p1, sl, nl);
-        const h2v a2 = __builtin_elementwise_fma(p2, sh, nh), a3 = __builtin_elementwise_fma(p3, sh, nh);
-        return h8v{a0[0], a0[1], a1[0], a1[1], a2[0], a2[1], a3[0], a3[1]};
-    };
-    auto highs = [&](uint32_t qh, h2v S, uint32_t s0, uint32_t s1) __attribute__((always_inline)) {
-        const h2v T = S * quarter, N = T * m64;  // quad 2g + 1's field sits two bits higher: 64 + 4 q
-        const h2v sl = {T[0], T[0]}, nl = {N[0], N[0]}, sh = {T[1], T[1]}, nh = {N[1], N[1]};
-        const uint32_t y0 = qh << s0, y1 = qh >> s1;
-        const h2v p0 = __builtin_bit_cast(h2v, (y0 & m.lo2) | m.exp), p1 = __builtin_bit_cast(h2v, (y1 & m.lo2) | m.exp);
-        const h2v p2 = __builtin_bit_cast(h2v, (y0 & m.hi2) | m.exp), p3 = __builtin_bit_cast(h2v, (y1 & m.hi2) | m.exp);
-        const h2v a0 = __builtin_elementwise_fma(p0, sl, nl), a1 = __builtin_elementwise_fma(p1, sl, nl);
-        const h2v a2 = __builtin_elementwise_fma(p2, sh, nh), a3 = __builtin_elementwise_fma(p3, sh, nh);
-        return h8v{a0[0], a0[1], a1[0], a1[1], a2[0], a2[1], a3[0], a3[1]};
-    };
-
     copy_raw(0, st[0]);
     copy_tokens(0, st[0]);
     copy_raw(1, st[1]);
@@ -797,7 +781,6 @@ __global__ __launch_bounds__(1024) void prefill_q6k_lanes_kernel(PfArgs a, TlMap
         int ln = lane;
         asm volatile("" : "+v"(ln));
         const int g = ln >> 4, c = ln & 15, lane = ln;
-        const uint32_t s0 = 4 - 4 * (g & 1), s1 = 4 + 4 * (g & 1);  // the lane's nibble to bits 4-7
         const int8_t* rsc = (const int8_t*)R.sc[c];
         const uint32_t sv = *(const uint32_t*)&R.sc[c][4 * g] ^ 0x80808080u;  // s + 128
         const float d = factor_f16(R.dw[c] >> (16 * (b & 1)));
@@ -833,8 +816,8 @@ __global__ __launch_bounds__(1024) void prefill_q6k_lanes_kernel(PfArgs a, TlMap
                 const uint2 ql = *(const uint2*)&R.q[16 * kk + c][8 * (g >> 1)];
                 const uint32_t qh = *(const uint32_t*)&R.q[32 + 16 * kk + c][8 * (kp & 1) + 4 * (g >> 1)];
                 const h2v sc = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x64646464u, sv, kk ? 0x04030401u : 0x04020400u)) + m1152;
-                wl = lows(ql, sc, s0, s1);
-                wh = highs(qh, sc, s0, s1);
+                wl = q6_lows(ql, sc, g, m);
+                wh = q6_highs(qh, sc, g, m);
             }
             const f4v lo = __builtin_amdgcn_mfma_f32_16x16x32_f16(bv[u & 1], wl, z, 0, 0, 0);
             const f4v hi = __builtin_amdgcn_mfma_f32_16x16x32_f16(bv[u & 1], wh, z, 0, 0, 0);
@@ -1060,368 +1043,266 @@ int launch_q8_0_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const
     return GLLM_OK;
 }
 
-// --- at most 16 activation rows, operands through a per-wave LDS ring -----
-// One workgroup per 16 weight rows; wave w computes the MFMA products of
-// blocks b = w, w + NW, ... (16-row x 16-token tiles, one per AVX2 lane k),
-// the waves exchange the exact products through LDS per group of blocks and
-// run the float chains in block order (only the integer products are
-// block-parallel, so the bits are the row kernel's).  Each wave copies its
-// own operands global -> LDS, DEPTH blocks ahead, in layouts that make every
-// MFMA operand read of a wave conflict-free:
-//   nib [lane k][row c][16 bytes]   (lane (g, c) reads dword g: consecutive)
-//   q8  [lane k][token t][32 bytes] (lane (g, c) reads 8 bytes at 8 g)
-// The copies are inline-asm global_load_lds, so their vmcnt waits are
-// explicit counts: NC copies per block, DEPTH blocks in flight.
-template <int PT>  // tokens staged per block (8 or 16)
-struct SsSlot {
-    uint8_t nib[8][16][16];
-    uint8_t hdr[16][16];
-    uint8_t q8[8][PT][32];
-    float xs32[PT][8];
-    float xs[64];  // [token]; copy lanes past the tokens land in the tail
+// --- 2 to 16 activation rows: one pair of AVX2 lanes per wave ---------------
+// A decode batch reads the weights once for few tokens, so a workgroup is 16
+// rows, split over 4 / KP waves of KP lane pairs (kp, kp + 4), and every wave
+// streams what it needs of a block by itself, kSmRing blocks ahead in LDS: 16
+// rows' nibbles of its lanes, their headers, and its records of the
+// activations (small_rec: f16 operands and sums).  No wave waits for another
+// before the final tree, so there is no barrier in the loop.
+// KP: four waves take 16-byte pieces of each 128-byte weight line at
+// different times; with many rows that is what bounds the launch (the L1 does
+// not hold the lines between them), so two pairs per wave are faster there,
+// and one pair per wave where rows are few and waves scarce.
+// Up to 8 tokens (PT = 8) both lanes share one MFMA tile: D rows 0-7 hold lane
+// kp's eight tokens and rows 8-15 lane kp + 4's, two MFMAs accumulating into
+// it with the other lane's A rows zero (read from a zeroed LDS row; every sum
+// is an exact integer below 2^24), so the chains run on full registers.
+// Q6_K has the code's two fields and xs16, as in prefill_q6k_lanes_kernel.
+// With the quantiser launch (3-4 us of it): Q4_K 14336 x 4096 at 8 tokens 21.0
+// us for 64-row tiles staged per block, 16.5 like this; 4096 x 14336 at 3 / 8 /
+// 16 tokens 31.8 / 23.4 / 37.8 -> 17.5 / 18.0 / 21.2 us; Q6_K 4096 x 14336 at 5
+// / 16 tokens 40.4 / 107 -> 26.3 / 30.9 us for the row kernels.
+constexpr int kSmRing = 4;
+
+template <int PT, bool Q6, int KP>
+struct SmSlot {
+    // Q6Raw, or nibbles [32 j + 16 (k / 4) + row c of pair j] and headers [row c]
+    static constexpr int kRaw = Q6 ? 64 * 16 + 16 * 16 + 16 * 4 : (32 * KP + 16) * 16;
+    uint8_t raw[kRaw];
+    uint8_t rec[KP][PT * 128 + PT * 28];
 };
-template <int PT>
-constexpr int ss_copies() { return 2 + 1 + PT / 4 + PT / 8 + 1; }
+template <int PT, bool Q6, int KP>
+struct SmLds {
+    SmSlot<PT, Q6, KP> ring[4 / KP][kSmRing];  // [wave]
+    uint8_t zero[16];
+    float ex[4][64][4];
+};
 
-template <int PT>
-__device__ __forceinline__ void ss_copy(const PfArgs& a, int b, uint32_t slot, int lane) {
-    typedef SsSlot<PT> S;
-    b = min(b, a.blocks - 1);  // past the end: the last block again (never read)
-    const int cols = a.blocks * 256;
-    const int row0 = blockIdx.x * 16;
-#pragma unroll
-    for (int i = 0; i < 2; i++) {  // piece 64 i + lane = (k, c)
-        const int idx = 64 * i + lane, k = idx >> 4, c = idx & 15;
-        const size_t r = (size_t)min(row0 + c, a.rows - 1);
-        lds_copy16_s(a.w, (uint32_t)(r * a.rb + q4k_nib_off(a.blocks, b) + 16 * k),
-                     slot + offsetof(S, nib) + 1024 * i);
-    }
-    {
-        const size_t r = (size_t)min(row0 + (lane >> 2), a.rows - 1);
-        lds_copy4_s(a.w, (uint32_t)(r * a.rb + q4k_hdr_off(b) + 4 * (lane & 3)), slot + offsetof(S, hdr));
-    }
-#pragma unroll
-    for (int i = 0; i < PT / 4; i++) {  // piece 64 i + lane = ((k, t), half)
-        const int idx = 64 * i + lane, h = idx & 1, t = (idx >> 1) % PT, k = (idx >> 1) / PT;
-        const size_t tok = (size_t)min(t, a.p - 1);
-        lds_copy16_s(a.act.q8perm, (uint32_t)(tok * cols + (size_t)b * 256 + 32 * k + 16 * h),
-                     slot + offsetof(S, q8) + 1024 * i);
-    }
-#pragma unroll
-    for (int i = 0; i < PT / 8; i++) {  // dword 64 i + lane = (t, k)
-        const int idx = 64 * i + lane;
-        const size_t t = (size_t)min(idx >> 3, a.p - 1);
-        lds_copy4_s(a.act.xs32, (uint32_t)((t * (cols / 32) + (size_t)b * 8 + (idx & 7)) * 4),
-                    slot + offsetof(S, xs32) + 256 * i);
-    }
-    {
-        const size_t t = (size_t)min(lane, a.p - 1);
-        lds_copy4_s(a.act.xscale, (uint32_t)((t * a.blocks + b) * 4), slot + offsetof(S, xs));
-    }
-}
-
-template <int NW, int DEPTH, int PT>
-constexpr size_t ss_lds_bytes() {
-    return sizeof(f4v) * NW * 8 * 64 + sizeof(SbParams) * NW + sizeof(SsSlot<PT>) * NW * DEPTH;
-}
-
-template <int NW, int DEPTH, int PT>
-__global__ __launch_bounds__(64 * NW) void prefill_q4k_b16s_kernel(PfArgs a) {
-    constexpr int KK = 8 / NW;
-    constexpr int NC = ss_copies<PT>();
-    typedef SsSlot<PT> S;
-    extern __shared__ __attribute__((aligned(16))) uint8_t dyn[];
-    f4v (*sdI)[8][64] = (f4v (*)[8][64])dyn;                         // [wave][lane k][MFMA lane]
-    SbParams* sp = (SbParams*)(dyn + sizeof(f4v) * NW * 8 * 64);      // [wave]
-    uint8_t* ring = dyn + sizeof(f4v) * NW * 8 * 64 + sizeof(SbParams) * NW;
-    const int lane = threadIdx.x & 63;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+template <int PT, bool Q6, int KP>
+__global__ __launch_bounds__(256 / KP) void small_lanes_kernel(PfArgs a) {
+    static_assert(KP == 1 || !Q6, "two pairs per wave: Q4_K");
+    constexpr int KK = PT == 8 ? 1 : 2;  // MFMA tiles of a pair: both lanes in one, or one each
+    __shared__ __attribute__((aligned(16))) SmLds<PT, Q6, KP> L;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kp = KP * wave;  // the wave's first pair
     const int g = lane >> 4, c = lane & 15;
-    const int row0 = blockIdx.x * 16;
-    const int tc = min(c, a.p - 1);  // B token of this lane
-    const int nb = a.blocks;
-    const uint32_t ring_w = lds_addr(ring + sizeof(S) * DEPTH * w);
-    float accF[KK][4], accM[KK][4];
-#pragma unroll
-    for (int kk = 0; kk < KK; kk++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) accF[kk][i] = accM[kk][i] = 0.0f;
-#pragma unroll
-    for (int d = 0; d < DEPTH; d++) ss_copy<PT>(a, w + NW * d, ring_w + sizeof(S) * d, lane);
-    int slot = 0;
-#pragma unroll 1
-    for (int q0 = 0; q0 < nb; q0 += NW) {
-        // this wave's block q0 + w is in `slot` once the later copies alone
-        // are outstanding
-        wait_vmem_le<(DEPTH - 1) * NC>();
-        const S& sl = *(const S*)(ring + sizeof(S) * (DEPTH * w + slot));
-        {
-            const u4v hdr = *(const u4v*)&sl.hdr[c][0];
-            uint32_t sc_lo, sc_hi, mn;
-            sb_scale_min(hdr, 2 * g, sc_lo, mn);
-            sb_scale_min(hdr, 2 * g + 1, sc_hi, mn);
-            const _Float16 hl = (_Float16)(float)sc_lo, nl = (_Float16)(-1024.0f * (float)sc_lo);
-            const _Float16 hh = (_Float16)(float)sc_hi, nh = (_Float16)(-1024.0f * (float)sc_hi);
-            const uint32_t bl = __builtin_bit_cast(uint16_t, hl), bnl = __builtin_bit_cast(uint16_t, nl);
-            const uint32_t bh = __builtin_bit_cast(uint16_t, hh), bnh = __builtin_bit_cast(uint16_t, nh);
-            const uint32_t sh_lo = bl | (bl << 16), sn_lo = bnl | (bnl << 16);
-            const uint32_t sh_hi = bh | (bh << 16), sn_hi = bnh | (bnh << 16);
-#pragma unroll
-            for (int k = 0; k < 8; k++) {
-                const uint32_t wd = *(const uint32_t*)&sl.nib[k][c][4 * g];
-                const uint2 q8 = *(const uint2*)&sl.q8[k][tc][8 * g];
-                const h8v av = dequant_a(wd, sh_lo, sn_lo, sh_hi, sn_hi);
-                uint32_t v[4];
-                i8x4_to_h(q8.x, v[0], v[1]);
-                i8x4_to_h(q8.y, v[2], v[3]);
-                const h8v bv = __builtin_bit_cast(h8v, u4v{v[0], v[1], v[2], v[3]});
-                const f4v z = {0.0f, 0.0f, 0.0f, 0.0f};
-                sdI[w][k][lane] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bv, z, 0, 0, 0);
+    const int row0 = blockIdx.x * 16, nb = a.blocks;
+    if (threadIdx.x < 4) ((uint32_t*)L.zero)[threadIdx.x] = 0;
+    const uint32_t rbase = (uint32_t)min(row0 + c, a.rows - 1) * (uint32_t)a.rb;
+    uint32_t roff;  // the lane's source in the first raw copy
+    if constexpr (Q6) roff = rbase + (g < 2 ? 16 * (kp + 4 * g) : 128 + 16 * ((kp >> 1) + 2 * (g - 2)));
+    else if constexpr (KP == 1) roff = rbase + (g < 2 ? 16 * nb + 16 * (kp + 4 * g) : 0);
+    else roff = rbase + 16 * nb + 16 * (kp + (g >> 1) + 4 * (g & 1));
+    constexpr int REC = PT * 128 + PT * 28, RECS = KP * REC;
+    constexpr int kCopies = (Q6 ? 3 : KP) + RECS / 1024 + 1;  // per block
+    const uint8_t* rec = a.act.rec + (size_t)kp * REC;
+    auto copy = [&](int b, SmSlot<PT, Q6, KP>& S) __attribute__((always_inline)) {
+        b = min(b, nb - 1);
+        const uint32_t raw = lds_addr(S.raw), dst = lds_addr(S.rec[0]);
+        if constexpr (Q6) {
+            const uint8_t* src = a.w + (size_t)b * 208;
+            lds_copy16_s(src, roff, raw);
+            if (lane < 16) {
+                lds_copy16_s(src + 192, rbase, raw + 1024);
+                lds_copy4_s(a.w, rbase + (uint32_t)(nb * 208 + (b & ~1) * 2), raw + 1280);
             }
-            if (g == 0) {
-                sp[w].d[c] = f16_bits_to_f32(hdr.x & 0xffffu);
-                sp[w].dmin[c] = f16_bits_to_f32(hdr.x >> 16);
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    uint32_t scj, mnj;
-                    sb_scale_min(hdr, j, scj, mnj);
-                    sp[w].m[j][c] = (float)mnj;
-                }
-            } else if (g == 1) {
-                sp[w].xs[c] = sl.xs[tc];
-#pragma unroll
-                for (int k = 0; k < 8; k++) sp[w].xsum[k][c] = sl.xs32[tc][k];
+        } else {
+            if constexpr (KP == 1) {
+                if (lane < 48) lds_copy16_s(a.w, roff + (uint32_t)b * (g < 2 ? 128 : 16), raw);
+            } else {
+                lds_copy16_s(a.w + (size_t)b * 128, roff, raw);
+                if (lane < 16) lds_copy16_s(a.w + (size_t)b * 16, rbase, raw + 1024);
             }
         }
-        // the slot's reads are done: refill it DEPTH groups ahead
-        wait_lgkm0();
-        ss_copy<PT>(a, q0 + w + NW * DEPTH, ring_w + sizeof(S) * slot, lane);
-        slot = slot + 1 == DEPTH ? 0 : slot + 1;
-        lds_barrier();
-        // the group's blocks in order: chains of lanes k = KK w .. for rows
-        // 4g + i and token c (the MFMA D layout of this lane)
+        const uint8_t* src = rec + (size_t)b * 4 * REC;
 #pragma unroll
-        for (int u = 0; u < NW; u++) {
-            if (q0 + u >= nb) break;  // uniform
-            const SbParams& P = sp[u];
-            const f4v d4 = *(const f4v*)&P.d[4 * g];
-            const f4v dm4 = *(const f4v*)&P.dmin[4 * g];
-            const float xs = P.xs[c];
-            float dxs[4];
+        for (int i = 0; i < RECS / 1024; i++) lds_copy16_s(src + 1024 * i, 16 * lane, dst + 1024 * i);
+        if (lane < RECS % 1024 / 16) lds_copy16_s(src + RECS / 1024 * 1024, 16 * lane, dst + RECS / 1024 * 1024);
+    };
+    static_assert(RECS % 1024 != 0, "copies per block");
+
+    float accF[KP][KK][4], accM[KP][KK][4];
 #pragma unroll
-            for (int i = 0; i < 4; i++) dxs[i] = d4[i] * xs;
+    for (int j = 0; j < KP; j++)
+#pragma unroll
+        for (int kk = 0; kk < KK; kk++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) accF[j][kk][i] = accM[j][kk][i] = 0.0f;
+    const NibMasks nm = nib_masks();
+    Q6Masks m6{0x00f000f0u, 0x00300030u, 0x00c000c0u, 0x54005400u};
+    asm("" : "+s"(m6.nib), "+s"(m6.lo2), "+s"(m6.hi2), "+v"(m6.exp));
+    const h2v m1024 = {(_Float16)-1024.0f, (_Float16)-1024.0f}, m1152 = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+    __syncthreads();  // the zero row
+#pragma unroll
+    for (int d = 0; d < kSmRing; d++) copy(d, L.ring[wave][d]);
+    const f4v z = {0.0f, 0.0f, 0.0f, 0.0f};
+
+    // one block; the lane's D registers are tokens t4 .. t4 + 3 of lane k
+    auto block = [&](int b, SmSlot<PT, Q6, KP>& S) __attribute__((always_inline)) {
+        wait_vmem_le<(kSmRing - 1) * kCopies>();
+        asm volatile("" ::: "memory");
+        const int odd = PT == 8 ? g >> 1 : 0, t4 = PT == 8 ? 4 * (g & 1) : 4 * g;
+        // the records: A operands, lane (g, r) token r % PT of lane k, and
+        // rows of PT floats: xs32 k, k + 4, xscale, xs16 x 4
+        h8v av[KP][2];
+        f4v xc[KP], xs[KP][KK], x0[KK], x8[KK];
+#pragma unroll
+        for (int j = 0; j < KP; j++) {
+            const float* rf = (const float*)(S.rec[j] + PT * 128);
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const uint8_t* src = S.rec[j] + ((k * 4 + g) * PT + (c & (PT - 1))) * 16;
+                if (PT == 8 && (c >> 3) != k) src = L.zero;
+                av[j][k] = *(const h8v*)src;
+            }
+            xc[j] = *(const f4v*)&rf[2 * PT + t4];
 #pragma unroll
             for (int kk = 0; kk < KK; kk++) {
-                const int k = KK * w + kk;
-                const f4v dI = sdI[u][k][lane];
-                const f4v m4 = *(const f4v*)&P.m[k][4 * g];
-                const float xk = P.xsum[k][c];
+                const int k = PT == 8 ? odd : kk;
+                if constexpr (Q6) {
+                    x0[kk] = *(const f4v*)&rf[(3 + k) * PT + t4];
+                    x8[kk] = *(const f4v*)&rf[(5 + k) * PT + t4];
+                } else {
+                    xs[j][kk] = *(const f4v*)&rf[k * PT + t4];
+                }
+            }
+        }
+        if constexpr (Q6) {
+            const Q6Raw& R = *(const Q6Raw*)S.raw;
+            const int8_t* rsc = (const int8_t*)R.sc[c];
+            float s0[KK], s8[KK];
+#pragma unroll
+            for (int kk = 0; kk < KK; kk++) {
+                const int k = kp + 4 * (PT == 8 ? odd : kk);
+                s0[kk] = (float)rsc[k];
+                s8[kk] = (float)rsc[8 + k];
+            }
+            const uint32_t sv = *(const uint32_t*)&R.sc[c][4 * g] ^ 0x80808080u;
+            const float d = factor_f16(R.dw[c] >> (16 * (b & 1)));
+            uint2 ql[2];
+            uint32_t qh[2];
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                ql[k] = *(const uint2*)&R.q[16 * k + c][8 * (g >> 1)];
+                qh[k] = *(const uint32_t*)&R.q[32 + 16 * k + c][8 * (kp & 1) + 4 * (g >> 1)];
+            }
+            f4v lo[KK], hi[KK];
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const h2v sc = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x64646464u, sv, k ? 0x04030401u : 0x04020400u)) + m1152;
+                const h8v wl = q6_lows(ql[k], sc, g, m6), wh = q6_highs(qh[k], sc, g, m6);
+                const int kk = KK == 1 ? 0 : k;
+                lo[kk] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[0][k], wl, KK == 1 && k ? lo[kk] : z, 0, 0, 0);
+                hi[kk] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[0][k], wh, KK == 1 && k ? hi[kk] : z, 0, 0, 0);
+            }
+            wait_lgkm0();
+            copy(b + kSmRing, S);
+#pragma unroll
+            for (int kk = 0; kk < KK; kk++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    accF[kk][i] = fmaf(dI[i], dxs[i], accF[kk][i]);
-                    const float mx = m4[i] * xk;
-                    accM[kk][i] = fmaf(dm4[i], mx, accM[kk][i]);
+                    float o2 = s0[kk] * (x0[kk][i] * 32.0f);             // VMULPS, ScaleF32(xs, 32)
+                    o2 = fmaf(s8[kk], x8[kk][i] * 32.0f, o2);            // VFMADD231PS
+                    accM[0][kk][i] = fmaf(d, o2, accM[0][kk][i]);
+                    accF[0][kk][i] = fmaf(fmaf(hi[kk][i], 16.0f, lo[kk][i]), d * xc[0][i], accF[0][kk][i]);
+                }
+        } else {
+            const uint8_t (*raw)[16] = (const uint8_t (*)[16])S.raw;
+            const u4v h = *(const u4v*)raw[32 * KP + c];
+            uint32_t nd[KP][2];
+#pragma unroll
+            for (int j = 0; j < KP; j++)
+#pragma unroll
+                for (int k = 0; k < 2; k++) nd[j][k] = *(const uint32_t*)&raw[32 * j + 16 * k + c][4 * g];
+            const float d = f16_bits_to_f32(h.x & 0xffffu), dm = factor_f16(h.x >> 16);
+            const uint32_t top = (h.w & 0x0f0f0f0fu) | ((h.y >> 2) & 0x30303030u);
+            const uint32_t sb = ((g & 2) ? top : h.y & 0x3f3f3f3fu) >> (16 * (g & 1));
+            const h2v one16 = {(_Float16)1.0f, (_Float16)0.0625f}, off16 = {(_Float16)-1024.0f, (_Float16)-64.0f};
+            const h2v s = __builtin_elementwise_fma(
+                __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x64646464u, sb, 0x04010400u)), one16, off16);
+            const h2v n = s * m1024;
+            f4v D[KP][KK];
+#pragma unroll
+            for (int j = 0; j < KP; j++) {
+                D[j][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[j][0], dequant_nib(nd[j][0], s, n, nm), z, 0, 0, 0);
+                D[j][KK - 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[j][1], dequant_nib(nd[j][1], s, n, nm),
+                                                                      KK == 1 ? D[j][0] : z, 0, 0, 0);
+            }
+            wait_lgkm0();
+            copy(b + kSmRing, S);
+#pragma unroll
+            for (int j = 0; j < KP; j++) {
+                const int k8 = 8 * (kp + j);
+                const float mlo = (float)__builtin_amdgcn_ubfe(h.z, k8, 6);
+                const float mhi = (float)((__builtin_amdgcn_ubfe(h.z, k8 + 6, 2) << 4) | __builtin_amdgcn_ubfe(h.w, k8 + 4, 4));
+#pragma unroll
+                for (int kk = 0; kk < KK; kk++) {
+                    const float mn = (PT == 8 ? odd : kk) ? mhi : mlo;
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        accM[j][kk][i] = fmaf(dm, mn * xs[j][kk][i], accM[j][kk][i]);
+                        accF[j][kk][i] = fmaf(D[j][kk][i], d * xc[j][i], accF[j][kk][i]);
+                    }
                 }
             }
         }
-        wait_lgkm0();
-        lds_barrier();
+    };
+#pragma unroll 1
+    for (int b = 0; b < nb; b += kSmRing) {
+#pragma unroll
+        for (int d = 0; d < kSmRing; d++) {
+            if (b + d >= nb) break;  // uniform
+            block(b + d, L.ring[wave][d]);
+        }
     }
-    wait_vmem_le<0>();  // the last refills (never read) have landed
-    // tree8 over the lanes k (held by the waves) through LDS
-    float* vb = (float*)dyn;  // [k][MFMA lane][row i]
+    wait_vmem_le<0>();  // the last copies, never read
+    // the reference's tree: s_kp = v_kp + v_(kp + 4), then (s0 + s1) + (s2 + s3)
 #pragma unroll
-    for (int kk = 0; kk < KK; kk++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) vb[((KK * w + kk) * 64 + lane) * 4 + i] = accF[kk][i] - accM[kk][i];
-    __syncthreads();
-    if (w == 0 && c < a.p) {
+    for (int j = 0; j < KP; j++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const int r = row0 + 4 * g + i;
-            if (r >= a.rows) continue;
-            float v[8];
-#pragma unroll
-            for (int k = 0; k < 8; k++) v[k] = vb[(k * 64 + lane) * 4 + i];
-            const float s0 = v[0] + v[4], s1 = v[1] + v[5], s2 = v[2] + v[6], s3 = v[3] + v[7];
-            a.out[(size_t)c * a.out_stride + r] = (s0 + s1) + (s2 + s3);
+            float v = accF[j][0][i] - accM[j][0][i];
+            if constexpr (KK == 2) v = v + (accF[j][KK - 1][i] - accM[j][KK - 1][i]);
+            L.ex[kp + j][lane][i] = v;
         }
-    }
-}
-
-// At most 8 tokens: lane pairs.  Tile m of a block holds AVX2 lanes 2m
-// (MFMA columns 0-7, tokens 0-7) and 2m + 1 (columns 8-15): two MFMAs
-// accumulate into it, each with the other lane's B columns zero, so every
-// column is a real (lane, token) product (the exact integer I, below 2^24,
-// whatever the accumulation order).  Eight waves, wave w: the block w of each
-// group for the MFMA phase, then the chains of pair w / 2 for rows
-// 4g + 2 (w % 2) .. + 1 of each D lane.  Half the products in LDS, half the
-// chain steps and B conversions of prefill_q4k_b16s_kernel, and room for a
-// ring three blocks deep.
-template <int DEPTH>
-constexpr size_t sp_lds_bytes() {
-    return sizeof(f4v) * 8 * 4 * 64 + sizeof(SbParams) * 8 + sizeof(SsSlot<8>) * 8 * DEPTH;
-}
-template <int DEPTH>
-__global__ __launch_bounds__(512) void prefill_q4k_b16p_kernel(PfArgs a) {
-    constexpr int NW = 8;
-    constexpr int NC = ss_copies<8>();
-    typedef SsSlot<8> S;
-    extern __shared__ __attribute__((aligned(16))) uint8_t dyn[];
-    f4v (*sdI)[4][64] = (f4v (*)[4][64])dyn;                          // [block][pair][MFMA lane]
-    SbParams* sp = (SbParams*)(dyn + sizeof(f4v) * NW * 4 * 64);       // [block]
-    uint8_t* ring = dyn + sizeof(f4v) * NW * 4 * 64 + sizeof(SbParams) * NW;
-    const int lane = threadIdx.x & 63;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int g = lane >> 4, c = lane & 15;
-    const int row0 = blockIdx.x * 16;
-    const int odd = c >> 3, t = c & 7;    // this lane's B column: lane parity, token
-    const int tb = min(t, a.p - 1);      // token whose q8 this lane supplies
-    const int tc = min(c, a.p - 1);      // token of the per-token factors (columns < 8 used)
-    const int nb = a.blocks;
-    const int pm = w >> 1, ih = w & 1;   // chain phase: pair, row half
-    const uint32_t ring_w = lds_addr(ring + sizeof(S) * DEPTH * w);
-    float accF[2], accM[2];
-    accF[0] = accF[1] = accM[0] = accM[1] = 0.0f;
-#pragma unroll
-    for (int d = 0; d < DEPTH; d++) ss_copy<8>(a, w + NW * d, ring_w + sizeof(S) * d, lane);
-    int slot = 0;
-#pragma unroll 1
-    for (int q0 = 0; q0 < nb; q0 += NW) {
-        wait_vmem_le<(DEPTH - 1) * NC>();
-        const S& sl = *(const S*)(ring + sizeof(S) * (DEPTH * w + slot));
-        {
-            const u4v hdr = *(const u4v*)&sl.hdr[c][0];
-            uint32_t sc_lo, sc_hi, mn;
-            sb_scale_min(hdr, 2 * g, sc_lo, mn);
-            sb_scale_min(hdr, 2 * g + 1, sc_hi, mn);
-            const _Float16 hl = (_Float16)(float)sc_lo, nl = (_Float16)(-1024.0f * (float)sc_lo);
-            const _Float16 hh = (_Float16)(float)sc_hi, nh = (_Float16)(-1024.0f * (float)sc_hi);
-            const uint32_t bl = __builtin_bit_cast(uint16_t, hl), bnl = __builtin_bit_cast(uint16_t, nl);
-            const uint32_t bh = __builtin_bit_cast(uint16_t, hh), bnh = __builtin_bit_cast(uint16_t, nh);
-            const uint32_t sh_lo = bl | (bl << 16), sn_lo = bnl | (bnl << 16);
-            const uint32_t sh_hi = bh | (bh << 16), sn_hi = bnh | (bnh << 16);
-#pragma unroll
-            for (int m = 0; m < 4; m++) {
-                const uint32_t w0 = *(const uint32_t*)&sl.nib[2 * m][c][4 * g];
-                const uint32_t w1 = *(const uint32_t*)&sl.nib[2 * m + 1][c][4 * g];
-                const uint2 q8 = *(const uint2*)&sl.q8[2 * m + odd][tb][8 * g];
-                const h8v a0 = dequant_a(w0, sh_lo, sn_lo, sh_hi, sn_hi);
-                const h8v a1 = dequant_a(w1, sh_lo, sn_lo, sh_hi, sn_hi);
-                uint32_t v[4];
-                i8x4_to_h(q8.x, v[0], v[1]);
-                i8x4_to_h(q8.y, v[2], v[3]);
-                const u4v zero = {0u, 0u, 0u, 0u};
-                const u4v bu = {v[0], v[1], v[2], v[3]};
-                const h8v b0 = __builtin_bit_cast(h8v, odd ? zero : bu);
-                const h8v b1 = __builtin_bit_cast(h8v, odd ? bu : zero);
-                const f4v z = {0.0f, 0.0f, 0.0f, 0.0f};
-                f4v dd = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, b0, z, 0, 0, 0);
-                dd = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, b1, dd, 0, 0, 0);
-                sdI[w][m][lane] = dd;
-            }
-            if (g == 0) {
-                sp[w].d[c] = f16_bits_to_f32(hdr.x & 0xffffu);
-                sp[w].dmin[c] = f16_bits_to_f32(hdr.x >> 16);
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    uint32_t scj, mnj;
-                    sb_scale_min(hdr, j, scj, mnj);
-                    sp[w].m[j][c] = (float)mnj;
-                }
-            } else if (g == 1) {
-                sp[w].xs[c] = sl.xs[tc];
-#pragma unroll
-                for (int k = 0; k < 8; k++) sp[w].xsum[k][c] = sl.xs32[tc][k];
-            }
-        }
-        wait_lgkm0();
-        ss_copy<8>(a, q0 + w + NW * DEPTH, ring_w + sizeof(S) * slot, lane);
-        slot = slot + 1 == DEPTH ? 0 : slot + 1;
-        lds_barrier();
-        // chains of pair pm, rows 4g + 2 ih + ii, lane k = 2 pm + odd, token t
-        const int k = 2 * pm + odd;
-#pragma unroll
-        for (int u = 0; u < NW; u++) {
-            if (q0 + u >= nb) break;  // uniform
-            const SbParams& P = sp[u];
-            const f4v dI = sdI[u][pm][lane];
-            const float xs = P.xs[t];
-            const float xk = P.xsum[k][t];
-#pragma unroll
-            for (int ii = 0; ii < 2; ii++) {
-                const int i = 2 * ih + ii;
-                const float dxs = P.d[4 * g + i] * xs;
-                accF[ii] = fmaf(dI[i], dxs, accF[ii]);
-                const float mx = P.m[k][4 * g + i] * xk;
-                accM[ii] = fmaf(P.dmin[4 * g + i], mx, accM[ii]);
-            }
-        }
-        wait_lgkm0();
-        lds_barrier();
-    }
-    wait_vmem_le<0>();
-    // tree8 over the lanes k through LDS: vb[k][row][token]
-    float* vb = (float*)dyn;
-#pragma unroll
-    for (int ii = 0; ii < 2; ii++)
-        vb[((2 * pm + odd) * 16 + 4 * g + 2 * ih + ii) * 8 + t] = accF[ii] - accM[ii];
     __syncthreads();
-    const int tid = threadIdx.x;
-    if (tid < 128) {
-        const int r = tid >> 3, tt = tid & 7;
-        if (tt < a.p && row0 + r < a.rows) {
-            float v[8];
+    for (int o = threadIdx.x; o < 16 * PT; o += 256 / KP) {
+        const int t = o >> 4, r = o & 15;
+        if (t >= a.p || row0 + r >= a.rows) continue;
+        float s[4];
 #pragma unroll
-            for (int kk = 0; kk < 8; kk++) v[kk] = vb[(kk * 16 + r) * 8 + tt];
-            const float s0 = v[0] + v[4], s1 = v[1] + v[5], s2 = v[2] + v[6], s3 = v[3] + v[7];
-            a.out[(size_t)tt * a.out_stride + row0 + r] = (s0 + s1) + (s2 + s3);
+        for (int q = 0; q < 4; q++) {
+            s[q] = L.ex[q][16 * (t >> 2) + r][t & 3];
+            if constexpr (KK == 1) s[q] = s[q] + L.ex[q][16 * (2 + (t >> 2)) + r][t & 3];
         }
+        a.out[(size_t)t * a.out_stride + row0 + r] = (s[0] + s[1]) + (s[2] + s[3]);
     }
 }
 
-template <int DEPTH>
-static bool launch_b16p(const PfArgs& a, hipStream_t s) {
-    constexpr size_t lds = sp_lds_bytes<DEPTH>();
-    static_assert(lds <= 160 * 1024, "LDS");
-    static const bool ok = hipFuncSetAttribute((const void*)prefill_q4k_b16p_kernel<DEPTH>,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               (int)lds) == hipSuccess;
-    if (!ok) {
-        (void)hipGetLastError();
-        return false;
-    }
-    hipLaunchKernelGGL((prefill_q4k_b16p_kernel<DEPTH>), dim3((a.rows + 15) / 16), dim3(512), lds,
-                       s, a);
-    return true;
+// Batched Q4_K or Q6_K products of 2 to kTiledMinP rows (act.rec set); Q6_K
+// blocks % 8 == 0; rows * rb < 4 GiB.
+int launch_small_lanes(bool q6, const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,
+                       float* out, int out_stride, hipStream_t s) {
+    if (rows <= 0 || blocks <= 0 || p <= 0) return GLLM_OK;
+    if (!act.rec || p > kTiledMinP || (size_t)rows * rb >= ((size_t)1 << 32) || (q6 && blocks % 8))
+        return fail(GLLM_EINVAL, "small batch: %d tokens, %d blocks, %d rows of %zu B", p, blocks, rows, rb);
+    PfArgs a{d_w, rb, rows, blocks, act, p, out, out_stride};
+    const dim3 grid((rows + 15) / 16);
+    const bool many = (int)grid.x >= 2 * device_cus();
+    if (q6 && p <= 8) hipLaunchKernelGGL((small_lanes_kernel<8, true, 1>), grid, dim3(256), 0, s, a);
+    else if (q6) hipLaunchKernelGGL((small_lanes_kernel<16, true, 1>), grid, dim3(256), 0, s, a);
+    else if (p <= 8 && many) hipLaunchKernelGGL((small_lanes_kernel<8, false, 2>), grid, dim3(128), 0, s, a);
+    else if (p <= 8) hipLaunchKernelGGL((small_lanes_kernel<8, false, 1>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((small_lanes_kernel<16, false, 1>), grid, dim3(256), 0, s, a);
+    GLLM_HIP(hipGetLastError());
+    return GLLM_OK;
 }
 
-template <int NW, int DEPTH, int PT>
-static bool launch_b16s(const PfArgs& a, hipStream_t s) {
-    constexpr size_t lds = ss_lds_bytes<NW, DEPTH, PT>();
-    static_assert(lds <= 160 * 1024, "LDS");
-    static const bool ok = hipFuncSetAttribute((const void*)prefill_q4k_b16s_kernel<NW, DEPTH, PT>,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               (int)lds) == hipSuccess;
-    if (!ok) {
-        (void)hipGetLastError();
-        return false;
-    }
-    hipLaunchKernelGGL((prefill_q4k_b16s_kernel<NW, DEPTH, PT>), dim3((a.rows + 15) / 16),
-                       dim3(64 * NW), lds, s, a);
-    return true;
-}
-
-
-// Kernel choice.  More than 16 activation rows: 64 x 64 tiles split by AVX2
-// lane (prefill_q4k_lanes_kernel).  At most 16 rows (a decode batch): 64 rows x
-// 16 tokens (prefill_q4k_mfma_kernel); the per-block staging (q8 to f16,
-// scale decoding) is a fixed cost per workgroup, so 64 rows per workgroup
-// beat smaller tiles that would fill more CUs (measured at batch 8: 22.8 vs
-// 28.4 us for 14336 x 4096), except where 64-row tiles leave a third of the
-// CUs idle: there 16-row tiles with block-parallel waves and operands in
-// per-wave LDS rings (prefill_q4k_b16p_kernel up to 8 tokens, four-wave
-// prefill_q4k_b16s_kernel at 9-16).  The tiled and ring kernels address a
+// Kernel choice for Q4_K from 8 rows on, after run_gemv's small batches
+// (launch_small_lanes): 64 x 64 tiles split by AVX2 lane above 16 rows, and 64
+// rows x 16 tokens (prefill_q4k_mfma_kernel) for batches without records, that
+// is past kSmallCols columns or 4 GiB of weight.  The other kernels address a
 // weight with 32-bit offsets.
 int launch_q4k_mfma(const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,
                     float* out, int out_stride, hipStream_t s) {
@@ -1432,11 +1313,9 @@ int launch_q4k_mfma(const uint8_t* d_w, size_t rb, int rows, int blocks, const A
         if (!act.b16t || !fits)
             return fail(GLLM_EINVAL, "prefill: %d rows of %zu B need f16 tiles and < 4 GiB", rows, rb);
         GLLM_TRY(launch_q4k_lanes(a, s));
-    } else if ((rows + 63) / 64 < 2 * device_cus() / 3) {
-        if (!fits) return fail(GLLM_EINVAL, "prefill: weights of %zu B past 4 GiB", (size_t)rows * rb);
-        const bool done = p > 8 ? launch_b16s<4, 3, 16>(a, s) : launch_b16p<2>(a, s);
-        if (!done) return fail(GLLM_EDEVICE, "prefill: the LDS of the 16-row kernel was refused");
     } else {
+        if ((rows + 63) / 64 < 2 * device_cus() / 3 && !fits)
+            return fail(GLLM_EINVAL, "prefill: weights of %zu B past 4 GiB", (size_t)rows * rb);
         launch_pf<4, 1>(a, s);
     }
     GLLM_HIP(hipGetLastError());

@@ -21,6 +21,9 @@ size_t act_bytes(int cols, int p) {
         n = (n + 255) & ~(size_t)255;
         n += (size_t)(p + 15) / 16 * 16 * cols * 2;  // b16t
         n += (size_t)(p + 15) / 16 * 16 * (cols / 32) * 4;  // xs32t
+    } else if (p > 1 && cols <= kSmallCols) {
+        n = (n + 255) & ~(size_t)255;
+        n += (size_t)(cols / 256) * 4 * small_rec(small_pt(p));  // rec
     }
     return n + 256;
 }
@@ -39,6 +42,9 @@ void act_carve(void* base, int cols, int p, ActQ8* a) {
     a->b16t = nullptr;
     a->xs32t = nullptr;
     a->tiles = 0;
+    a->rec = nullptr;
+    if (p > 1 && p <= kTiledMinP && cols <= kSmallCols)
+        a->rec = (uint8_t*)(((uintptr_t)c + 255) & ~(uintptr_t)255);
     if (p > kTiledMinP) {
         c = (uint8_t*)(((uintptr_t)c + 255) & ~(uintptr_t)255);
         a->tiles = (p + 15) / 16;
@@ -65,6 +71,14 @@ __global__ __launch_bounds__(256) void q8k_prep_kernel(const float* __restrict__
         a.b16t[((size_t)b * a.tiles + (t >> 4)) * 4096 + ((kappa >> 3) * 16 + (t & 15)) * 8 +
                b16_slot(kappa)] = 0;
         if (e < 8) a.xs32t[(((size_t)b * a.tiles + (t >> 4)) * 8 + e) * 16 + (t & 15)] = 0.0f;
+        return;
+    }
+    const int pt = small_pt(a.p);
+    if (a.rec && t >= a.p) {  // padding tokens of the records (uniform per workgroup)
+        const int kappa = q8perm_offset(e), k = kappa >> 5;
+        uint8_t* r = a.rec + ((size_t)b * 4 + (k & 3)) * small_rec(pt);
+        ((uint16_t*)r)[(((k >> 2) * 4 + ((kappa >> 3) & 3)) * pt + t) * 8 + b16_slot(kappa)] = 0;
+        if (e < 28) ((float*)(a.rec + ((size_t)b * 4 + (e & 3)) * small_rec(pt) + pt * 128))[(e >> 2) * pt + t] = 0.0f;
         return;
     }
     __shared__ float sx[256];
@@ -97,6 +111,17 @@ __global__ __launch_bounds__(256) void q8k_prep_kernel(const float* __restrict__
         a.b16t[((size_t)b * a.tiles + (t >> 4)) * 4096 + ((kappa >> 3) * 16 + (t & 15)) * 8 +
                b16_slot(kappa)] = __builtin_bit_cast(uint16_t, (_Float16)(float)q);
     }
+    // the records' floats of lane pair k: rows 0, 1 xs32, 2 xscale, 3 .. 6 xs16
+    auto rec_f = [&](int k, int row) -> float& {
+        return ((float*)(a.rec + ((size_t)b * 4 + k) * small_rec(pt) + pt * 128))[row * pt + t];
+    };
+    if (a.rec) {
+        const int k = kappa >> 5;
+        uint8_t* r = a.rec + ((size_t)b * 4 + (k & 3)) * small_rec(pt);
+        ((uint16_t*)r)[(((k >> 2) * 4 + ((kappa >> 3) & 3)) * pt + t) * 8 + b16_slot(kappa)] =
+            __builtin_bit_cast(uint16_t, (_Float16)(float)q);
+        if (e < 4) rec_f(e, 2) = scale;
+    }
     if (e == 0) a.xscale[(size_t)t * nb + b] = scale;
     if (e < 8) {
         // sumF32Groups32: v_k = ((x[k] + x[8+k]) + x[16+k]) + x[24+k]
@@ -108,6 +133,7 @@ __global__ __launch_bounds__(256) void q8k_prep_kernel(const float* __restrict__
         const float xs = (a0 + a1) + (a2 + a3);
         a.xs32[(size_t)t * (cols / 32) + b * 8 + e] = xs;
         if (a.xs32t) a.xs32t[(((size_t)b * a.tiles + (t >> 4)) * 8 + e) * 16 + (t & 15)] = xs;
+        if (a.rec) rec_f(e & 3, e >> 2) = xs;
     } else if (e >= 64 && e < 80) {
         // sumF32Groups16: v_k = x[k] + x[8+k], then the same tree, then x32
         const int gi = e - 64;
@@ -116,13 +142,15 @@ __global__ __launch_bounds__(256) void q8k_prep_kernel(const float* __restrict__
 #pragma unroll
         for (int k = 0; k < 8; k++) s[k] = g[k] + g[8 + k];
         const float a0 = s[0] + s[4], a1 = s[1] + s[5], a2 = s[2] + s[6], a3 = s[3] + s[7];
-        a.xs16[(size_t)t * (cols / 16) + b * 16 + gi] = (a0 + a1) + (a2 + a3);
+        const float xs = (a0 + a1) + (a2 + a3);
+        a.xs16[(size_t)t * (cols / 16) + b * 16 + gi] = xs;
+        if (a.rec) rec_f(gi & 3, 3 + (gi >> 2)) = xs;
     }
 }
 
 int launch_q8k_prep(const float* d_x, int cols, int p, const ActQ8& a, hipStream_t s) {
     if (cols <= 0 || cols % 256 || p <= 0) return fail(GLLM_EINVAL, "q8k: cols %d p %d", cols, p);
-    dim3 grid(cols / 256, a.b16t ? 16 * a.tiles : p);
+    dim3 grid(cols / 256, a.b16t ? 16 * a.tiles : a.rec ? small_pt(p) : p);
     hipLaunchKernelGGL(q8k_prep_kernel, grid, dim3(256), 0, s, d_x, cols, a, (int8_t*)nullptr,
                        (float*)nullptr, (const float*)nullptr);
     GLLM_HIP(hipGetLastError());
@@ -132,7 +160,7 @@ int launch_q8k_prep(const float* d_x, int cols, int p, const ActQ8& a, hipStream
 int launch_q8k_prep_silu(const float* d_gate, const float* d_up, int cols, int p, const ActQ8& a,
                          hipStream_t s) {
     if (cols <= 0 || cols % 256 || p <= 0) return fail(GLLM_EINVAL, "q8k: cols %d p %d", cols, p);
-    dim3 grid(cols / 256, a.b16t ? 16 * a.tiles : p);
+    dim3 grid(cols / 256, a.b16t ? 16 * a.tiles : a.rec ? small_pt(p) : p);
     hipLaunchKernelGGL(q8k_prep_kernel, grid, dim3(256), 0, s, d_gate, cols, a, (int8_t*)nullptr,
                        (float*)nullptr, d_up);
     GLLM_HIP(hipGetLastError());

@@ -72,6 +72,22 @@ def test_prefill_q8_0_tile_edges(hip, rows, cols, p):
     assert_bits(w.matvec_batch(xs), amd64(data, xs, rows, cols, ref.Q8_0), f"{rows}x{cols} p={p}")
 
 
+@pytest.mark.parametrize("qtype", [ref.Q4_K, ref.Q6_K])
+@pytest.mark.parametrize("rows,cols,p", [(1, 6144, 2), (17, 2048, 5), (40, 6144, 8), (33, 4096, 9), (16, 2048, 16),
+                                         (8200, 2048, 7), (8200, 2048, 13), (20, 8192, 4)])
+def test_small_batch_edges(hip, qtype, rows, cols, p):
+    """One to three row tiles with a short last one, both token widths with and
+    without padding, both splits of the lane pairs, block counts that end a
+    turn of the ring and, for Q4_K, ones that do not."""
+    if qtype == ref.Q4_K:
+        cols += 256
+    data, _ = quant_matrix(qtype, rows, cols, 930 + rows)
+    w = hip.Weight.from_host(data, qtype, rows, cols)
+    xs = normal(931 + p, (p, cols))
+    xs[p // 2, :256] = 0.0
+    assert_bits(w.matvec_batch(xs), amd64(data, xs, rows, cols, qtype), f"{rows}x{cols} p={p}")
+
+
 def test_prefill_degenerate_blocks(hip):
     """All-zero tokens, zero 256-blocks inside a token, a lone large value and
     NaN-free extremes (q8kQuantize's scale-0 blocks, quant_q8k_portable.go:36-62)."""
