@@ -350,11 +350,18 @@ static void launch_pf(const PfArgs& a, hipStream_t s) {
 // cycles at four waves per SIMD, the MFMA alone 20).
 constexpr int kTlRows = 64, kTlTok = 64;
 
+// Q5_K (q5kDotQ8KRow, kernels_amd64.s:578-663) has the same chains; its codes
+// take a fifth bit from the qh plane (sc * code <= 63 * 31, exact in f16), so
+// a nibble dword's pairs get one more masked term each: 206 us at 14336 x 4096 x
+// 512, where the row kernels, eight tokens at a time, took 2889 us.
+template <bool Q5>
 struct LnStage {
     uint8_t b16[4 * 8 * 4 * 256];  // [token tile][lane k][group g][token c][8 halves]
     float xsum[4][8][16];          // [token tile][lane k][token c]
     float xs[kTlTok];
-    uint8_t raw[16][48][16];       // [wave]: nibbles [lane kp, kp + 4][row c], headers [row c]
+    // [wave]: nibbles [lane kp, kp + 4][row c], headers [row c], and for Q5_K
+    // the 16 bytes with the two lanes' qh dwords [lane kp, kp + 4][row c]
+    uint8_t raw[16][Q5 ? 80 : 48][16];
 };
 
 // Direct global -> LDS copies addressed by a wave-uniform base and a 32-bit
@@ -421,6 +428,20 @@ __device__ __forceinline__ h8v dequant_nib(uint32_t w, h2v s, h2v n, const NibMa
     return h8v{a0[0], a0[1], a1[0], a1[1], a2[0], a2[1], a3[0], a3[1]};
 }
 
+// The same for Q5_K: bits 0 and 1 of every byte of qh are the fifth bits of
+// the low and the high nibbles, at mantissa bits 4 and 8 of their pairs.
+__device__ __forceinline__ h8v dequant_q5(uint32_t w, uint32_t qh, h2v s, h2v n, const NibMasks& m) {
+    const uint32_t v = w >> 8;
+    const uint32_t b0 = m.exp | ((qh << 4) & 0x00100010u), b1 = m.exp | ((qh >> 4) & 0x00100010u);
+    const uint32_t b2 = m.exp | ((qh << 7) & 0x01000100u), b3 = m.exp | ((qh >> 1) & 0x01000100u);
+    const h2v p0 = __builtin_bit_cast(h2v, (w & m.lo) | b0), p1 = __builtin_bit_cast(h2v, (v & m.lo) | b1);
+    const h2v p2 = __builtin_bit_cast(h2v, (w & m.hi) | b2), p3 = __builtin_bit_cast(h2v, (v & m.hi) | b3);
+    const h2v sl = {s[0], s[0]}, nl = {n[0], n[0]}, sh = {s[1], s[1]}, nh = {n[1], n[1]};
+    const h2v a0 = __builtin_elementwise_fma(p0, sl, nl), a1 = __builtin_elementwise_fma(p1, sl, nl);
+    const h2v a2 = __builtin_elementwise_fma(p2, sh, nh), a3 = __builtin_elementwise_fma(p3, sh, nh);
+    return h8v{a0[0], a0[1], a1[0], a1[1], a2[0], a2[1], a3[0], a3[1]};
+}
+
 // An f16 factor of many chain steps, converted once.  Left alone the compiler
 // folds the conversion into each fma as v_fma_mix_f32, which issues more
 // slowly (14336 x 4096 x 512 with / without: Q8_0 348 / 305 us, Q4_K 180 /
@@ -450,9 +471,10 @@ __device__ __forceinline__ void lanes_store(const PfArgs& a, const float* ex, in
     }
 }
 
+template <bool Q5>
 __global__ __launch_bounds__(1024) void prefill_q4k_lanes_kernel(PfArgs a, TlMap mp) {
     extern __shared__ __attribute__((aligned(16))) uint8_t dyn[];
-    LnStage* const st = (LnStage*)dyn;
+    LnStage<Q5>* const st = (LnStage<Q5>*)dyn;
     const int id = blockIdx.x, xcd = id & 7, local = id >> 3;
     const int lt = local % mp.tg_size, lrow = local / mp.tg_size;
     const int ttile = (xcd % mp.h) * mp.tg_size + lt, rtile = (xcd / mp.h) * mp.rg_size + lrow;
@@ -472,7 +494,7 @@ __global__ __launch_bounds__(1024) void prefill_q4k_lanes_kernel(PfArgs a, TlMap
     const uint8_t* bsrc = (const uint8_t*)a.act.b16t + (size_t)min(tile0 + rq, last) * 8192 + 2048 * kp;
     const uint32_t xoff = w < 2 ? (uint32_t)(min(tile0 + 2 * w + (lane >> 5), last) * 512 + 16 * (lane & 31))
                                 : (uint32_t)min(tok0 + lane, a.p - 1) * nb * 4;
-    auto copy_tokens = [&](int b, LnStage& S) __attribute__((always_inline)) {
+    auto copy_tokens = [&](int b, LnStage<Q5>& S) __attribute__((always_inline)) {
         b = min(b, nb - 1);
         const uint8_t* src = bsrc + b * bstep;
         const uint32_t dst = lds_addr(S.b16 + rq * 8192 + 2048 * kp);
@@ -486,10 +508,15 @@ __global__ __launch_bounds__(1024) void prefill_q4k_lanes_kernel(PfArgs a, TlMap
     // other (roff: this lane's source offset of the next one)
     const int kc = min(lane >> 4, 2);
     uint32_t roff = (uint32_t)min(row0 + 16 * rq + c, a.rows - 1) * (uint32_t)a.rb +
-                    (kc < 2 ? 16 * nb + 16 * (kp + 4 * kc) : 0);
-    const uint32_t rstep = kc < 2 ? 128 : 16;
-    auto copy_raw = [&](int b, LnStage& S) __attribute__((always_inline)) {
+                    (kc < 2 ? (Q5 ? 16 : 16 * nb) + 16 * (kp + 4 * kc) : 0);
+    const uint32_t rstep = Q5 ? 176 : kc < 2 ? 128 : 16;
+    constexpr int kRawCopies = Q5 ? 2 : 1;
+    auto copy_raw = [&](int b, LnStage<Q5>& S) __attribute__((always_inline)) {
         if (lane < 48) lds_copy16_s(a.w, roff, lds_addr(&S.raw[w][0][0]));
+        if constexpr (Q5) {  // the same lanes 0-31: row and lane k, less the lane's nibble offset
+            if (lane < 32)
+                lds_copy16_s(a.w, roff - (16 + 16 * (kp + 4 * kc)) + 144 + 16 * kc, lds_addr(&S.raw[w][48][0]));
+        }
         if (b < nb - 1) roff += rstep;
     };
     // This lane's weight row 16 rq + c in one block: factors, mins of the two
@@ -501,17 +528,21 @@ __global__ __launch_bounds__(1024) void prefill_q4k_lanes_kernel(PfArgs a, TlMap
     struct Row {
         float d, dm, mn[2];
         h2v s, n;  // {sc_2g, sc_(2g + 1) / 16} and -1024 times them
-        uint32_t nd[2];
+        uint32_t nd[2], qh[2];
     };
     const uint32_t sel = g < 2 ? 4 : 12, sh0 = 16 * (g & 1), low = g < 2 ? 0x3f3fu : 0x0f0fu;
     const h2v one16 = {(_Float16)1.0f, (_Float16)0.0625f}, off16 = {(_Float16)-1024.0f, (_Float16)-64.0f};
     const h2v m1024 = {(_Float16)-1024.0f, (_Float16)-1024.0f};
-    auto row_of = [&](const LnStage& S) __attribute__((always_inline)) {
+    auto row_of = [&](const LnStage<Q5>& S) __attribute__((always_inline)) {
         Row r;
         const u4v h = *(const u4v*)&S.raw[w][32 + c][0];
         const uint32_t hs = *(const uint32_t*)&S.raw[w][32 + c][sel];
         r.nd[0] = *(const uint32_t*)&S.raw[w][c][4 * g];
         r.nd[1] = *(const uint32_t*)&S.raw[w][16 + c][4 * g];
+        if constexpr (Q5) {
+            r.qh[0] = *(const uint32_t*)&S.raw[w][48 + c][4 * kp];
+            r.qh[1] = *(const uint32_t*)&S.raw[w][64 + c][4 * kp];
+        }
         r.d = f16_bits_to_f32(h.x & 0xffffu);
         r.dm = factor_f16(h.x >> 16);
         r.mn[0] = (float)__builtin_amdgcn_ubfe(h.z, 8 * kp, 6);
@@ -535,7 +566,7 @@ __global__ __launch_bounds__(1024) void prefill_q4k_lanes_kernel(PfArgs a, TlMap
     copy_raw(0, st[0]);
     copy_tokens(0, st[0]);
     copy_raw(1, st[1]);
-    wait_vmem_le<1>();
+    wait_vmem_le<kRawCopies>();
     asm volatile("" ::: "memory");
     Row row = row_of(st[0]);
     wait_lgkm0();
@@ -545,7 +576,7 @@ __global__ __launch_bounds__(1024) void prefill_q4k_lanes_kernel(PfArgs a, TlMap
     // hold the order (the compiler would keep more operands at once than four
     // waves per SIMD have registers for).  Register 4 tt + i of an outer
     // product is token 16 tt + 4g + i.
-    auto block = [&](int b, LnStage& S, LnStage& N) __attribute__((always_inline)) {
+    auto block = [&](int b, LnStage<Q5>& S, LnStage<Q5>& N) __attribute__((always_inline)) {
         copy_tokens(b + 1, N);
         copy_raw(b + 2, S);  // row b is in registers
         // LDS addresses are rebuilt from the lane each block: kept across
@@ -579,7 +610,9 @@ __global__ __launch_bounds__(1024) void prefill_q4k_lanes_kernel(PfArgs a, TlMap
 #pragma unroll
         for (int u = 0; u <= 8; u++) {
             if (u < 6) bv[(u + 2) % 3] = acts(u + 2);
-            if (u == 0 || u == 4) wv = dequant_nib(row.nd[u >> 2], row.s, row.n, nm);
+            if (u == 0 || u == 4)
+                wv = Q5 ? dequant_q5(row.nd[u >> 2], row.qh[u >> 2] >> (2 * g), row.s, row.n, nm)
+                        : dequant_nib(row.nd[u >> 2], row.s, row.n, nm);
             if (u < 8) D[u & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bv[u % 3], wv, z, 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
             if (u > 0) {
@@ -592,7 +625,7 @@ __global__ __launch_bounds__(1024) void prefill_q4k_lanes_kernel(PfArgs a, TlMap
             __builtin_amdgcn_sched_barrier(0);
         }
         // block b + 1 has landed (all but the raw copy of b + 2)
-        wait_vmem_le<1>();
+        wait_vmem_le<kRawCopies>();
         asm volatile("" ::: "memory");
         row = row_of(N);
         wait_lgkm0();
@@ -637,10 +670,21 @@ static bool lanes_lds(const void* kern, size_t lds) {
     return false;
 }
 
+template <bool Q5>
 static int launch_q4k_lanes(const PfArgs& a, hipStream_t s) {
-    constexpr size_t lds = 2 * sizeof(LnStage);
-    static const bool ok = lanes_lds((const void*)prefill_q4k_lanes_kernel, lds);
-    return launch_lanes<lds>(prefill_q4k_lanes_kernel, ok, a, s);
+    constexpr size_t lds = 2 * sizeof(LnStage<Q5>);
+    static const bool ok = lanes_lds((const void*)prefill_q4k_lanes_kernel<Q5>, lds);
+    return launch_lanes<lds>(prefill_q4k_lanes_kernel<Q5>, ok, a, s);
+}
+
+int launch_q5k_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,
+                     float* out, int out_stride, hipStream_t s) {
+    if (rows <= 0 || blocks <= 0 || p <= 0) return GLLM_OK;
+    if (!act.b16t || p <= kTiledMinP || (size_t)rows * rb >= ((size_t)1 << 32))
+        return fail(GLLM_EINVAL, "prefill: Q5_K tiles need > %d tokens and < 4 GiB", kTiledMinP);
+    GLLM_TRY(launch_q4k_lanes<true>(PfArgs{d_w, rb, rows, blocks, act, p, out, out_stride}, s));
+    GLLM_HIP(hipGetLastError());
+    return GLLM_OK;
 }
 
 // --- Q6_K, more than 16 activation rows: one pair of AVX2 lanes per wave ---
@@ -1312,7 +1356,7 @@ int launch_q4k_mfma(const uint8_t* d_w, size_t rb, int rows, int blocks, const A
     if (p > kTiledMinP) {
         if (!act.b16t || !fits)
             return fail(GLLM_EINVAL, "prefill: %d rows of %zu B need f16 tiles and < 4 GiB", rows, rb);
-        GLLM_TRY(launch_q4k_lanes(a, s));
+        GLLM_TRY(launch_q4k_lanes<false>(a, s));
     } else {
         if ((rows + 63) / 64 < 2 * device_cus() / 3 && !fits)
             return fail(GLLM_EINVAL, "prefill: weights of %zu B past 4 GiB", (size_t)rows * rb);

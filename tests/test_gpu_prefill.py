@@ -11,7 +11,7 @@ token (the reference's batched == per-token invariant, forward_batch_test.go).
 import numpy as np
 import pytest
 
-from conftest import normal, quant_matrix
+from conftest import extreme_row, normal, quant_matrix, random_rows
 from oracle import oracle as ref
 
 pytestmark = pytest.mark.gpu
@@ -70,6 +70,18 @@ def test_prefill_q8_0_tile_edges(hip, rows, cols, p):
     w = hip.Weight.from_host(data, ref.Q8_0, rows, cols)
     xs = normal(921 + p, (p, cols))
     assert_bits(w.matvec_batch(xs), amd64(data, xs, rows, cols, ref.Q8_0), f"{rows}x{cols} p={p}")
+
+
+@pytest.mark.parametrize("rows,cols,p", [(1, 256, 17), (65, 768, 65), (64, 512, 128), (130, 4096, 129)])
+def test_prefill_q5k_tile_edges(hip, rows, cols, p):
+    """Q5_K on the Q4_K kernel's tiles; the last row has every code, scale and
+    min at its maximum (sc * code = 63 * 31, the largest f16 operand)."""
+    data = random_rows(ref.Q5_K, rows, cols, 940 + rows)
+    data[-(cols // 256) * 176:] = extreme_row(ref.Q5_K, cols)
+    w = hip.Weight.from_host(data, ref.Q5_K, rows, cols)
+    xs = normal(941 + p, (p, cols))
+    xs[p - 1] = 127.0
+    assert_bits(w.matvec_batch(xs), amd64(data, xs, rows, cols, ref.Q5_K), f"{rows}x{cols} p={p}")
 
 
 @pytest.mark.parametrize("qtype", [ref.Q4_K, ref.Q6_K])
