@@ -2238,7 +2238,8 @@ int run_gemv(int n, gllm_hip_weight* const* ws, const ActQ8& act, int p, float* 
     }
     j.wg_begin[n] = wg;
     if (wg == 0) return GLLM_OK;
-    if (small_batch_fits(act, p, w0)) {
+    auto all = [&](auto fits) { return std::all_of(ws, ws + n, fits); };
+    if (all([&](auto* w) { return small_batch_fits(act, p, w); })) {
         for (int i = 0; i < n; i++)
             GLLM_TRY(launch_small_lanes(w0->type == GLLM_TYPE_Q6_K, ws[i]->d_data, ws[i]->row_bytes, ws[i]->rows,
                                         ws[i]->blocks, act, p, outs[i], j.out_stride[i], s));
@@ -2258,7 +2259,8 @@ int run_gemv(int n, gllm_hip_weight* const* ws, const ActQ8& act, int p, float* 
                                        act, p, outs[i], j.out_stride[i], s));
         return GLLM_OK;
     }
-    if (w0->type == GLLM_TYPE_Q5_K && p > kTiledMinP && (size_t)w0->rows * w0->row_bytes < ((size_t)1 << 32)) {
+    if (w0->type == GLLM_TYPE_Q5_K && p > kTiledMinP &&
+        all([](auto* w) { return (size_t)w->rows * w->row_bytes < ((size_t)1 << 32); })) {
         for (int i = 0; i < n; i++)
             GLLM_TRY(launch_q5k_tiled(ws[i]->d_data, ws[i]->row_bytes, ws[i]->rows, ws[i]->blocks,
                                       act, p, outs[i], j.out_stride[i], s));
