@@ -2259,11 +2259,12 @@ int run_gemv(int n, gllm_hip_weight* const* ws, const ActQ8& act, int p, float* 
                                        act, p, outs[i], j.out_stride[i], s));
         return GLLM_OK;
     }
-    if (w0->type == GLLM_TYPE_Q5_K && p > kTiledMinP &&
+    if ((w0->type == GLLM_TYPE_Q5_K || w0->type == GLLM_TYPE_Q4_0) && p > kTiledMinP &&
         all([](auto* w) { return (size_t)w->rows * w->row_bytes < ((size_t)1 << 32); })) {
+        const auto launch = w0->type == GLLM_TYPE_Q5_K ? launch_q5k_tiled : launch_q4_0_tiled;
         for (int i = 0; i < n; i++)
-            GLLM_TRY(launch_q5k_tiled(ws[i]->d_data, ws[i]->row_bytes, ws[i]->rows, ws[i]->blocks,
-                                      act, p, outs[i], j.out_stride[i], s));
+            GLLM_TRY(launch(ws[i]->d_data, ws[i]->row_bytes, ws[i]->rows, ws[i]->blocks, act, p, outs[i],
+                            j.out_stride[i], s));
         return GLLM_OK;
     }
     if (w0->type == GLLM_TYPE_Q6_K && q6k_tiled_fits(act, p, w0)) {

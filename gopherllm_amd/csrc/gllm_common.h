@@ -96,6 +96,9 @@ int launch_q6k_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const 
 // (p > kTiledMinP) and rows * rb < 4 GiB.
 int launch_q5k_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,
                      float* out, int out_stride, hipStream_t s);
+// Batched Q4_0 x Q8_K on the matrix cores, same contract and needs.
+int launch_q4_0_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,
+                      float* out, int out_stride, hipStream_t s);
 // 2 to kTiledMinP rows of Q4_K (q6: Q6_K, blocks % 8 == 0) x Q8_K, same
 // contract; needs act.rec and rows * rb < 4 GiB.
 int launch_small_lanes(bool q6, const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,

@@ -1,4 +1,5 @@
-// prefill.hip -- batched Q4_K x Q8_K products on the matrix cores.
+// prefill.hip -- batched products on the matrix cores: Q4_K, Q5_K, Q6_K, Q8_0
+// and Q4_0 x Q8_K.  Q4_K's arithmetic first; the others' stands at their kernels.
 //
 // matvecBatchQ8 (kernels_amd64.go:470-581) runs the batch-1 row kernel
 // q4kDotQ8KRow (kernels_amd64.s:437-543) once per (row, token), so a batched
@@ -24,12 +25,16 @@
 // 8s + 4 + i (high nibble, sub-block 2s + 1).  MFMA lane L supplies
 // kappa = 8(L/16) .. 8(L/16) + 7 of both operands, i.e. one weight dword.
 //
-// Workgroup: RW x TW waves over 16 RW weight rows x 16 TW tokens; wave w
-// owns the 16x16 tile of rows 16 (w % RW) .. + 15 and tokens
-// 16 (w / RW) .. + 15.  Per block the workgroup
-// stages the 32 tokens' q8 (as f16), xsums and xscales and the 64 rows'
-// decoded scales/mins and nibble bytes in LDS (double-buffered, loaded one
-// block ahead).
+// Three kinds of kernel follow: prefill_q4k_mfma_kernel (8 to 16 tokens of
+// weights or columns past what the others address), the *_lanes_kernels (more
+// than 16 tokens, every format below on its own chains) and
+// small_lanes_kernel (2 to 16 tokens).
+//
+// prefill_q4k_mfma_kernel: a workgroup is RW x TW waves over 16 RW weight
+// rows x 16 TW tokens; wave w owns the 16x16 tile of rows 16 (w % RW) .. + 15
+// and tokens 16 (w / RW) .. + 15.  Per block the workgroup stages the tokens'
+// q8 (as f16), xsums and xscales and the rows' decoded scales/mins and nibble
+// bytes in LDS (double-buffered, loaded one block ahead).
 #include <cstdlib>
 
 #include "gllm_common.h"
@@ -458,16 +463,20 @@ __device__ __forceinline__ void pin4(float (&v)[4]) {
 }
 
 // (s0 + s1) + (s2 + s3) of the four waves of row group rq, from the exchange
-// ex[rq][kp][token tile][i][lane]: wave (rq, kp) stores token tile kp.
+// ex[rq][kp][token tile][i][lane]: wave (rq, kp) stores token tile kp, with
+// its offset chains added where a format has them.
+template <bool OFF = false>
 __device__ __forceinline__ void lanes_store(const PfArgs& a, const float* ex, int row0, int tok0, int rq, int kp,
-                                            int lane) {
+                                            int lane, f4v off = {}) {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         float v[4];
 #pragma unroll
         for (int q = 0; q < 4; q++) v[q] = ex[(((rq * 4 + q) * 4 + kp) * 4 + i) * 64 + lane];
         const int t = tok0 + 16 * kp + 4 * (lane >> 4) + i, rr = row0 + 16 * rq + (lane & 15);
-        if (t < a.p && rr < a.rows) a.out[(size_t)t * a.out_stride + rr] = (v[0] + v[1]) + (v[2] + v[3]);
+        float r = (v[0] + v[1]) + (v[2] + v[3]);
+        if constexpr (OFF) r = r + off[i];
+        if (t < a.p && rr < a.rows) a.out[(size_t)t * a.out_stride + rr] = r;
     }
 }
 
@@ -1083,6 +1092,172 @@ int launch_q8_0_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const
     constexpr size_t lds = 2 * sizeof(Q80Stage);
     static const bool ok = lanes_lds((const void*)prefill_q8_0_lanes_kernel, lds);
     GLLM_TRY((launch_lanes<lds>(prefill_q8_0_lanes_kernel, ok, a, s)));
+    GLLM_HIP(hipGetLastError());
+    return GLLM_OK;
+}
+
+// --- Q4_0, more than 16 activation rows: one pair of AVX2 lanes per wave ----
+// q4_0DotQ8KRow (kernels_amd64.s:679-732) per 32-value block q:
+//   accF[k] = fma(d_q * xscale, float(I_qk), accF[k])   I_qk: the exact dot of the lane's
+//                                                       4 codes and 4 activation bytes
+//   accS    = fma(-8, d_q * xsum_q, accS)               one chain per row
+// and tree8(accF) + accS.  The split of the work and the dots are
+// prefill_q8_0_lanes_kernel's; a wave's lanes kp and kp + 4 are the low and
+// the high nibbles of the same 32 bytes.  d_q * xscale of four q is one
+// v_mfma_f32_16x16x1 (block j of the four: q = 2j, or 2j + 1) per token tile,
+// for both lanes, and the offset chains of token tile kp go with wave
+// (rq, kp), which stores that tile.
+// With the quantiser launch, the row kernels eight tokens at a time / this:
+// 14336 x 4096 x 512 3304 / 441 us, 4096 x 14336 x 333 3914 / 388, 4096 x 4096
+// x 64 243 / 56, 14336 x 4096 x 24 154 / 41; where 16 workgroups are all there
+// is, 1000 x 14336 x 17 133 / 115 and 1000 x 4096 x 17 49 / 38 us (179 and 56
+// with the token tiles past p computed too).  Bound by issue: per wave and
+// block 288 chain steps and 26 matrix instructions.
+struct Q40Stage {
+    uint8_t b16[4 * 8 * 4 * 256];  // [token tile][lane k][group g][token c][8 halves]
+    float xsum[4][8][16];          // [token tile][32-block q][token c]
+    float xs[kTlTok];
+    uint8_t raw[16][48][16];       // [wave]: nibbles [16 half + row c], eight f16 scales [32 + row c]
+};
+
+__global__ __launch_bounds__(1024) void prefill_q4_0_lanes_kernel(PfArgs a, TlMap mp) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t dyn[];
+    Q40Stage* const st = (Q40Stage*)dyn;
+    const int id = blockIdx.x, xcd = id & 7, local = id >> 3;
+    const int lt = local % mp.tg_size, lrow = local / mp.tg_size;
+    const int ttile = (xcd % mp.h) * mp.tg_size + lt, rtile = (xcd / mp.h) * mp.rg_size + lrow;
+    if (lrow >= mp.rg_size || ttile >= mp.tok_tiles || rtile >= mp.row_tiles) return;  // whole workgroup
+    const int row0 = rtile * kTlRows, tok0 = ttile * kTlTok, tile0 = tok0 / 16;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kp = w & 3, rq = w >> 2;
+    const int nb = a.blocks, left = a.p - tok0;  // token tiles past p are left out
+
+    // Copies of one block's tokens, as in the Q4_K kernel
+    const int last = a.act.tiles - 1;
+    const size_t bstep = (size_t)a.act.tiles * 8192;
+    const uint8_t* bsrc = (const uint8_t*)a.act.b16t + (size_t)min(tile0 + rq, last) * 8192 + 2048 * kp;
+    const uint32_t xoff = w < 2 ? (uint32_t)(min(tile0 + 2 * w + (lane >> 5), last) * 512 + 16 * (lane & 31))
+                                : (uint32_t)min(tok0 + lane, a.p - 1) * nb * 4;
+    auto copy_tokens = [&](int b, Q40Stage& S) __attribute__((always_inline)) {
+        b = min(b, nb - 1);
+        const uint8_t* src = bsrc + b * bstep;
+        const uint32_t dst = lds_addr(S.b16 + rq * 8192 + 2048 * kp);
+        lds_copy16_s(src, 16 * lane, dst);
+        lds_copy16_s(src + 1024, 16 * lane, dst + 1024);
+        if (w < 2) lds_copy16_s(a.act.xs32t + (size_t)b * a.act.tiles * 128, xoff, lds_addr(&S.xsum[2 * w][0][0]));
+        else if (w == 2) lds_copy4_s(a.act.xscale + b, xoff, lds_addr(&S.xs[0]));
+    };
+    // The wave's rows: one copy
+    const uint32_t roff = (uint32_t)min(row0 + 16 * rq + (lane & 15), a.rows - 1) * (uint32_t)a.rb +
+                          (lane < 32 ? 16 + 32 * kp + 16 * (lane >> 4) : 0);
+    auto copy_raw = [&](int b, Q40Stage& S) __attribute__((always_inline)) {
+        if (lane < 48) lds_copy16_s(a.w + (size_t)min(b, nb - 1) * 144, roff, lds_addr(&S.raw[w][0][0]));
+    };
+
+    float acc[2][4][4];  // accF of [lane k = kp + 4 kk][token tile tt][i]
+    f4v off = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int kk = 0; kk < 2; kk++)
+#pragma unroll
+        for (int tt = 0; tt < 4; tt++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[kk][tt][i] = 0.0f;
+
+    uint32_t nib = 0x000f000fu, exp = 0x64006400u;
+    asm("" : "+s"(nib), "+v"(exp));
+    const h2v m1024 = {(_Float16)-1024.0f, (_Float16)-1024.0f};
+    // the low nibbles of a dword as f16, bytes 0, 2, 1, 3: 1024 + code - 1024
+    auto halves = [&](uint32_t v) __attribute__((always_inline)) {
+        const h2v p0 = __builtin_bit_cast(h2v, (v & nib) | exp) + m1024;
+        const h2v p1 = __builtin_bit_cast(h2v, ((v >> 8) & nib) | exp) + m1024;
+        return h4v{p0[0], p0[1], p1[0], p1[1]};
+    };
+
+    copy_raw(0, st[0]);
+    copy_tokens(0, st[0]);
+    copy_raw(1, st[1]);
+    wait_vmem_le<1>();
+    lds_barrier();
+    auto block = [&](int b, Q40Stage& S, Q40Stage& N) __attribute__((always_inline)) {
+        copy_tokens(b + 1, N);
+        int ln = lane;  // LDS addresses are rebuilt each block: kept across blocks they would spill
+        asm volatile("" : "+v"(ln));
+        const int g = ln >> 4, c = ln & 15;
+        // this lane's codes and scales: 32-blocks 2g, 2g + 1 of row c
+        const uint2 v = *(const uint2*)&S.raw[w][16 * (g >> 1) + c][8 * (g & 1)];
+        const uint32_t dd = *(const uint32_t*)&S.raw[w][32 + c][4 * g];
+        wait_lgkm0();
+        copy_raw(b + 2, S);  // the wave's rows are in registers
+        const float de = f16_bits_to_f32(dd & 0xffffu), dn = f16_bits_to_f32(dd >> 16);
+        const f16v z16 = {0.0f};
+        {
+            const f16v E = __builtin_amdgcn_mfma_f32_16x16x1f32(S.xsum[kp][2 * g][c], de, z16, 0, 0, 0);
+            const f16v O = __builtin_amdgcn_mfma_f32_16x16x1f32(S.xsum[kp][2 * g + 1][c], dn, z16, 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) off[i] = fmaf(-8.0f, E[4 * q + i], off[i]);  // VFMADD231SS
+#pragma unroll
+                for (int i = 0; i < 4; i++) off[i] = fmaf(-8.0f, O[4 * q + i], off[i]);
+            }
+            asm volatile("" : "+v"(off));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // token 16 tt + 4g + i, weight row 16 rq + c
+#pragma unroll
+        for (int tt = 0; tt < 4; tt++) {
+            if (16 * tt >= left) break;
+            const float xs = S.xs[16 * tt + c];
+            const f16v dE = __builtin_amdgcn_mfma_f32_16x16x1f32(xs, de, z16, 0, 0, 0);  // VMULSS
+            const f16v dO = __builtin_amdgcn_mfma_f32_16x16x1f32(xs, dn, z16, 0, 0, 0);
+#pragma unroll
+            for (int kk = 0; kk < 2; kk++) {
+                const h8v x = *(const h8v*)(S.b16 + ((tt * 8 + kp + 4 * kk) * 4 + g) * 256 + c * 16);
+                const f16v E = __builtin_amdgcn_mfma_f32_16x16x4f16(h4v{x[0], x[1], x[2], x[3]}, halves(v.x >> (4 * kk)), z16, 0, 0, 0);
+                const f16v O = __builtin_amdgcn_mfma_f32_16x16x4f16(h4v{x[4], x[5], x[6], x[7]}, halves(v.y >> (4 * kk)), z16, 0, 0, 0);
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) acc[kk][tt][i] = fmaf(E[4 * q + i], dE[4 * q + i], acc[kk][tt][i]);  // VFMADD231PS
+#pragma unroll
+                    for (int i = 0; i < 4; i++) acc[kk][tt][i] = fmaf(O[4 * q + i], dO[4 * q + i], acc[kk][tt][i]);
+                }
+                pin4(acc[kk][tt]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        wait_vmem_le<1>();  // block b + 1 has landed (all but the raw copy of b + 2)
+        wait_lgkm0();
+        lds_barrier();
+    };
+#pragma unroll 1
+    for (int b = 0;;) {
+        block(b, st[0], st[1]);
+        if (++b == nb) break;
+        block(b, st[1], st[0]);
+        if (++b == nb) break;
+    }
+    wait_vmem_le<0>();  // the last copies, never read
+    lds_barrier();
+    float* ex = (float*)dyn;  // [rq][kp][tt][i][lane]
+#pragma unroll
+    for (int tt = 0; tt < 4; tt++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) ex[((w * 4 + tt) * 4 + i) * 64 + lane] = acc[0][tt][i] + acc[1][tt][i];
+    wait_lgkm0();
+    lds_barrier();
+    lanes_store<true>(a, ex, row0, tok0, rq, kp, lane, off);
+}
+
+int launch_q4_0_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,
+                      float* out, int out_stride, hipStream_t s) {
+    if (rows <= 0 || blocks <= 0 || p <= 0) return GLLM_OK;
+    if (!act.b16t || p <= kTiledMinP || (size_t)rows * rb >= ((size_t)1 << 32))
+        return fail(GLLM_EINVAL, "prefill: Q4_0 tiles need > %d tokens and < 4 GiB", kTiledMinP);
+    PfArgs a{d_w, rb, rows, blocks, act, p, out, out_stride};
+    constexpr size_t lds = 2 * sizeof(Q40Stage);
+    static const bool ok = lanes_lds((const void*)prefill_q4_0_lanes_kernel, lds);
+    GLLM_TRY((launch_lanes<lds>(prefill_q4_0_lanes_kernel, ok, a, s)));
     GLLM_HIP(hipGetLastError());
     return GLLM_OK;
 }

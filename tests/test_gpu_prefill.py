@@ -84,6 +84,18 @@ def test_prefill_q5k_tile_edges(hip, rows, cols, p):
     assert_bits(w.matvec_batch(xs), amd64(data, xs, rows, cols, ref.Q5_K), f"{rows}x{cols} p={p}")
 
 
+@pytest.mark.parametrize("rows,cols,p", [(1, 256, 17), (65, 768, 65), (64, 512, 128), (130, 4096, 129)])
+def test_prefill_q4_0_tile_edges(hip, rows, cols, p):
+    """Every code at its maximum in the last row, and a token of zeros."""
+    data = random_rows(ref.Q4_0, rows, cols, 950 + rows)
+    data[-(cols // 32) * 18:] = extreme_row(ref.Q4_0, cols)
+    w = hip.Weight.from_host(data, ref.Q4_0, rows, cols)
+    xs = normal(951 + p, (p, cols))
+    xs[p // 2] = 0.0
+    xs[p - 1] = 127.0
+    assert_bits(w.matvec_batch(xs), amd64(data, xs, rows, cols, ref.Q4_0), f"{rows}x{cols} p={p}")
+
+
 @pytest.mark.parametrize("qtype", [ref.Q4_K, ref.Q6_K])
 @pytest.mark.parametrize("rows,cols,p", [(1, 6144, 2), (17, 2048, 5), (40, 6144, 8), (33, 4096, 9), (16, 2048, 16),
                                          (8200, 2048, 7), (8200, 2048, 13), (20, 8192, 4)])
