@@ -353,7 +353,12 @@ static void launch_pf(const PfArgs& a, hipStream_t s) {
 // VALU operations of dequantisation and 11 matrix instructions, which hardly
 // overlap the VALU on this part (a 16x16x32 f16 MFMA and four fmas take 30
 // cycles at four waves per SIMD, the MFMA alone 20).
-constexpr int kTlRows = 64, kTlTok = 64;
+// Up to kHalfTok tokens the products and chains run on two of the four token
+// tiles only (NT = 2).  17 tokens, four / two tiles: 4096 x 14336 Q4_K 78 / 64 us,
+// Q5_K 91 / 77, Q6_K 120 / 96, Q8_0 138 / 86.  As a branch inside one kernel it
+// also served the last tile of a longer prompt, which gained nothing there
+// and cost Q8_0 and Q4_K up to 2 percent at full tiles.
+constexpr int kTlRows = 64, kTlTok = 64, kHalfTok = 32;
 
 // Q5_K (q5kDotQ8KRow, kernels_amd64.s:578-663) has the same chains; its codes
 // take a fifth bit from the qh plane (sc * code <= 63 * 31, exact in f16), so
@@ -480,7 +485,7 @@ __device__ __forceinline__ void lanes_store(const PfArgs& a, const float* ex, in
     }
 }
 
-template <bool Q5>
+template <bool Q5, int NT>
 __global__ __launch_bounds__(1024) void prefill_q4k_lanes_kernel(PfArgs a, TlMap mp) {
     extern __shared__ __attribute__((aligned(16))) uint8_t dyn[];
     LnStage<Q5>* const st = (LnStage<Q5>*)dyn;
@@ -598,7 +603,7 @@ __global__ __launch_bounds__(1024) void prefill_q4k_lanes_kernel(PfArgs a, TlMap
         for (int kk = 0; kk < 2; kk++) {
             const f16v P = __builtin_amdgcn_mfma_f32_16x16x1f32(S.xsum[g][kp + 4 * kk][c], row.mn[kk], z16, 0, 0, 0);
 #pragma unroll
-            for (int tt = 0; tt < 4; tt++) {
+            for (int tt = 0; tt < NT; tt++) {
 #pragma unroll
                 for (int i = 0; i < 4; i++) accM[kk][tt][i] = fmaf(row.dm, P[4 * tt + i], accM[kk][tt][i]);
                 pin4(accM[kk][tt]);
@@ -610,22 +615,22 @@ __global__ __launch_bounds__(1024) void prefill_q4k_lanes_kernel(PfArgs a, TlMap
         // product and runs the chains of step u - 1
         const f4v z = {0.0f, 0.0f, 0.0f, 0.0f};
         auto acts = [&](int u) __attribute__((always_inline)) {
-            return *(const h8v*)(S.b16 + (((u & 3) * 8 + kp + 4 * (u >> 2)) * 4 + g) * 256 + c * 16);
+            return *(const h8v*)(S.b16 + ((u % NT * 8 + kp + 4 * (u / NT)) * 4 + g) * 256 + c * 16);
         };
         h8v bv[3], wv;
         f4v D[2];
         bv[0] = acts(0);
         bv[1] = acts(1);
 #pragma unroll
-        for (int u = 0; u <= 8; u++) {
-            if (u < 6) bv[(u + 2) % 3] = acts(u + 2);
-            if (u == 0 || u == 4)
-                wv = Q5 ? dequant_q5(row.nd[u >> 2], row.qh[u >> 2] >> (2 * g), row.s, row.n, nm)
-                        : dequant_nib(row.nd[u >> 2], row.s, row.n, nm);
-            if (u < 8) D[u & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bv[u % 3], wv, z, 0, 0, 0);
+        for (int u = 0; u <= 2 * NT; u++) {
+            if (u < 2 * NT - 2) bv[(u + 2) % 3] = acts(u + 2);
+            if (u == 0 || u == NT)
+                wv = Q5 ? dequant_q5(row.nd[u / NT], row.qh[u / NT] >> (2 * g), row.s, row.n, nm)
+                        : dequant_nib(row.nd[u / NT], row.s, row.n, nm);
+            if (u < 2 * NT) D[u & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bv[u % 3], wv, z, 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
             if (u > 0) {
-                const int kk = (u - 1) >> 2, tt = (u - 1) & 3;
+                const int kk = (u - 1) / NT, tt = (u - 1) % NT;
 #pragma unroll
                 for (int i = 0; i < 4; i++)
                     accF[kk][tt][i] = fmaf(D[(u - 1) & 1][i], dxs[4 * tt + i], accF[kk][tt][i]);
@@ -682,8 +687,9 @@ static bool lanes_lds(const void* kern, size_t lds) {
 template <bool Q5>
 static int launch_q4k_lanes(const PfArgs& a, hipStream_t s) {
     constexpr size_t lds = 2 * sizeof(LnStage<Q5>);
-    static const bool ok = lanes_lds((const void*)prefill_q4k_lanes_kernel<Q5>, lds);
-    return launch_lanes<lds>(prefill_q4k_lanes_kernel<Q5>, ok, a, s);
+    static const bool ok = lanes_lds((const void*)prefill_q4k_lanes_kernel<Q5, 4>, lds) &&
+                           lanes_lds((const void*)prefill_q4k_lanes_kernel<Q5, 2>, lds);
+    return launch_lanes<lds>(a.p <= kHalfTok ? prefill_q4k_lanes_kernel<Q5, 2> : prefill_q4k_lanes_kernel<Q5, 4>, ok, a, s);
 }
 
 int launch_q5k_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,
@@ -765,6 +771,7 @@ __device__ __forceinline__ h8v q6_highs(uint32_t qh, h2v S, int g, const Q6Masks
     return h8v{a0[0], a0[1], a1[0], a1[1], a2[0], a2[1], a3[0], a3[1]};
 }
 
+template <int NT>
 __global__ __launch_bounds__(1024) void prefill_q6k_lanes_kernel(PfArgs a, TlMap mp) {
     extern __shared__ __attribute__((aligned(16))) uint8_t dyn[];
     Q6Stage* const st = (Q6Stage*)dyn;
@@ -846,7 +853,7 @@ __global__ __launch_bounds__(1024) void prefill_q6k_lanes_kernel(PfArgs a, TlMap
             f16v P = __builtin_amdgcn_mfma_f32_16x16x1f32(x0, sk, z16, 0, 0, 0);  // VMULPS
             P = __builtin_amdgcn_mfma_f32_16x16x1f32(x8, sk8, P, 0, 0, 0);        // VFMADD231PS
 #pragma unroll
-            for (int tt = 0; tt < 4; tt++) {
+            for (int tt = 0; tt < NT; tt++) {
 #pragma unroll
                 for (int i = 0; i < 4; i++) accM[kk][tt][i] = fmaf(d, P[4 * tt + i], accM[kk][tt][i]);
                 pin4(accM[kk][tt]);
@@ -857,14 +864,14 @@ __global__ __launch_bounds__(1024) void prefill_q6k_lanes_kernel(PfArgs a, TlMap
         // step u = (kk, tt); the next step's activations are read ahead
         const f4v z = {0.0f, 0.0f, 0.0f, 0.0f};
         auto acts = [&](int u) __attribute__((always_inline)) {
-            return *(const h8v*)(S.b16 + (((u & 3) * 8 + kp + 4 * (u >> 2)) * 4 + g) * 256 + c * 16);
+            return *(const h8v*)(S.b16 + ((u % NT * 8 + kp + 4 * (u / NT)) * 4 + g) * 256 + c * 16);
         };
         h8v bv[2], wl, wh;
         bv[0] = acts(0);
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const int kk = u >> 2, tt = u & 3;
-            if (u < 7) bv[(u + 1) & 1] = acts(u + 1);
+        for (int u = 0; u < 2 * NT; u++) {
+            const int kk = u / NT, tt = u % NT;
+            if (u < 2 * NT - 1) bv[(u + 1) & 1] = acts(u + 1);
             if (tt == 0) {
                 const uint2 ql = *(const uint2*)&R.q[16 * kk + c][8 * (g >> 1)];
                 const uint32_t qh = *(const uint32_t*)&R.q[32 + 16 * kk + c][8 * (kp & 1) + 4 * (g >> 1)];
@@ -883,7 +890,7 @@ __global__ __launch_bounds__(1024) void prefill_q6k_lanes_kernel(PfArgs a, TlMap
             __builtin_amdgcn_sched_barrier(0);
             // the wave's last read of its raw rows has returned: refill their
             // slot two blocks ahead
-            if (u == 4) copy_raw(b + 2, S);
+            if (u == NT) copy_raw(b + 2, S);
         }
         wait_vmem_le<3>();  // block b + 1 has landed (all but the raw copies of b + 2)
         wait_lgkm0();
@@ -920,8 +927,9 @@ int launch_q6k_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const 
                     kTiledMinP);
     PfArgs a{d_w, rb, rows, blocks, act, p, out, out_stride};
     constexpr size_t lds = 2 * sizeof(Q6Stage);
-    static const bool ok = lanes_lds((const void*)prefill_q6k_lanes_kernel, lds);
-    GLLM_TRY((launch_lanes<lds>(prefill_q6k_lanes_kernel, ok, a, s)));
+    static const bool ok = lanes_lds((const void*)prefill_q6k_lanes_kernel<4>, lds) &&
+                           lanes_lds((const void*)prefill_q6k_lanes_kernel<2>, lds);
+    GLLM_TRY((launch_lanes<lds>(p <= kHalfTok ? prefill_q6k_lanes_kernel<2> : prefill_q6k_lanes_kernel<4>, ok, a, s)));
     GLLM_HIP(hipGetLastError());
     return GLLM_OK;
 }
@@ -954,6 +962,7 @@ struct Q80Stage {
 };
 typedef _Float16 h4v __attribute__((ext_vector_type(4)));
 
+template <int NT>
 __global__ __launch_bounds__(1024) void prefill_q8_0_lanes_kernel(PfArgs a, TlMap mp) {
     extern __shared__ __attribute__((aligned(16))) uint8_t dyn[];
     Q80Stage* const st = (Q80Stage*)dyn;
@@ -1025,15 +1034,15 @@ __global__ __launch_bounds__(1024) void prefill_q8_0_lanes_kernel(PfArgs a, TlMa
         for (int q = 0; q < 8; q++) d[q] = factor_f16(dh[q >> 1] >> (16 * (q & 1)));
         // step u = (kk, tt): token 16 tt + 4g + i, weight row 16 rq + c
         auto acts = [&](int u) __attribute__((always_inline)) {
-            return *(const h8v*)(S.b16 + (((u & 3) * 8 + kp + 4 * (u >> 2)) * 4 + g) * 256 + c * 16);
+            return *(const h8v*)(S.b16 + ((u % NT * 8 + kp + 4 * (u / NT)) * 4 + g) * 256 + c * 16);
         };
         h8v bv[2];
         h4v we, wo;
         bv[0] = acts(0);
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const int kk = u >> 2, tt = u & 3;
-            if (u < 7) bv[(u + 1) & 1] = acts(u + 1);
+        for (int u = 0; u < 2 * NT; u++) {
+            const int kk = u / NT, tt = u % NT;
+            if (u < 2 * NT - 1) bv[(u + 1) & 1] = acts(u + 1);
             if (tt == 0) {
                 const uint2 v = *(const uint2*)&R.q[32 * kk + 16 * (g >> 1) + c][8 * (g & 1)];
                 we = halves(v.x);
@@ -1058,7 +1067,7 @@ __global__ __launch_bounds__(1024) void prefill_q8_0_lanes_kernel(PfArgs a, TlMa
             __builtin_amdgcn_sched_barrier(0);
             // the wave's last read of its raw rows has returned: refill their
             // slot two groups ahead
-            if (u == 4) copy_raw(b + 2, S);
+            if (u == NT) copy_raw(b + 2, S);
         }
         wait_vmem_le<2>();  // group b + 1 has landed (all but the raw copies of b + 2)
         wait_lgkm0();
@@ -1090,8 +1099,9 @@ int launch_q8_0_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const
         return fail(GLLM_EINVAL, "prefill: Q8_0 tiles need > %d tokens and < 4 GiB operands", kTiledMinP);
     PfArgs a{d_w, rb, rows, blocks, act, p, out, out_stride};
     constexpr size_t lds = 2 * sizeof(Q80Stage);
-    static const bool ok = lanes_lds((const void*)prefill_q8_0_lanes_kernel, lds);
-    GLLM_TRY((launch_lanes<lds>(prefill_q8_0_lanes_kernel, ok, a, s)));
+    static const bool ok = lanes_lds((const void*)prefill_q8_0_lanes_kernel<4>, lds) &&
+                           lanes_lds((const void*)prefill_q8_0_lanes_kernel<2>, lds);
+    GLLM_TRY((launch_lanes<lds>(p <= kHalfTok ? prefill_q8_0_lanes_kernel<2> : prefill_q8_0_lanes_kernel<4>, ok, a, s)));
     GLLM_HIP(hipGetLastError());
     return GLLM_OK;
 }

@@ -96,6 +96,19 @@ def test_prefill_q4_0_tile_edges(hip, rows, cols, p):
     assert_bits(w.matvec_batch(xs), amd64(data, xs, rows, cols, ref.Q4_0), f"{rows}x{cols} p={p}")
 
 
+@pytest.mark.parametrize("qtype", [ref.Q4_K, ref.Q5_K, ref.Q6_K, ref.Q8_0, ref.Q4_0])
+@pytest.mark.parametrize("p", [32, 33, 96, 97])
+def test_prefill_half_token_tiles(hip, qtype, p):
+    """32 tokens run two of the 64-token tile's four token tiles, 33 all; the
+    same counts behind a full tile."""
+    rows, cols = 70, 2048
+    data = (quant_matrix(qtype, rows, cols, 960 + p)[0] if qtype in (ref.Q4_K, ref.Q6_K, ref.Q8_0)
+            else random_rows(qtype, rows, cols, 960 + p))
+    w = hip.Weight.from_host(data, qtype, rows, cols)
+    xs = normal(961 + p, (p, cols))
+    assert_bits(w.matvec_batch(xs), amd64(data, xs, rows, cols, qtype), f"type {qtype} p={p}")
+
+
 @pytest.mark.parametrize("qtype", [ref.Q4_K, ref.Q6_K])
 @pytest.mark.parametrize("rows,cols,p", [(1, 6144, 2), (17, 2048, 5), (40, 6144, 8), (33, 4096, 9), (16, 2048, 16),
                                          (8200, 2048, 7), (8200, 2048, 13), (20, 8192, 4)])
