@@ -458,20 +458,22 @@ __device__ inline void silu_q8_block(const float* gate, const float* up, int b, 
 // they are issued before the weight prefetch and retire first (in order), so
 // its vmcnt waits for the weight registers stay exact, and the kernel waits
 // for the copies itself (vmcnt <= number of weight loads) before s_barrier.
-// M0 holds the wave's LDS destination; lane i writes M0 + 16*i (4*i).
+// M0 holds the wave's LDS destination; lane i writes M0 + 16*i (4*i).  A scalar
+// write of M0 needs one wait state before a load that goes to LDS, which the
+// compiler cannot add inside an asm string: the s_nop.
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }
 
 __device__ __forceinline__ void lds_copy16(const void* gsrc, uint32_t lds_dst) {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off"
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
                  :
                  : "v"(gsrc), "s"(lds_dst)
                  : "memory", "m0");
 }
 
 __device__ __forceinline__ void lds_copy4(const void* gsrc, uint32_t lds_dst) {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off"
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
                  :
                  : "v"(gsrc), "s"(lds_dst)
                  : "memory", "m0");

@@ -375,15 +375,16 @@ struct LnStage {
 };
 
 // Direct global -> LDS copies addressed by a wave-uniform base and a 32-bit
-// per-lane byte offset (the saddr form), so a copy costs one VGPR.
+// per-lane byte offset (the saddr form), so a copy costs one VGPR.  The s_nop
+// is the wait state between the M0 write and the load, as in lds_copy16.
 __device__ __forceinline__ void lds_copy16_s(const void* sbase, uint32_t voff, uint32_t lds_dst) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                  :
                  : "v"(voff), "s"(sbase), "s"(lds_dst)
                  : "memory", "m0");
 }
 __device__ __forceinline__ void lds_copy4_s(const void* sbase, uint32_t voff, uint32_t lds_dst) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1"
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
                  :
                  : "v"(voff), "s"(sbase), "s"(lds_dst)
                  : "memory", "m0");
