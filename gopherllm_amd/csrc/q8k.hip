@@ -97,7 +97,9 @@ __global__ __launch_bounds__(256) void q8k_prep_kernel(const float* __restrict__
     if (amax != 0.0f && amax == amax) {
         scale = amax / 127.0f;
         const float inv = 127.0f / amax;
-        q = (int)rintf(v * inv);
+        // int8 before anything is made of it: 127 / amax overflows for the
+        // smallest amax, and the f16 copies below hold what q8perm holds
+        q = (int8_t)(int)rintf(v * inv);
     }
     if (plain_q8) {
         plain_q8[(size_t)t * cols + (size_t)b * 256 + e] = (int8_t)q;

@@ -142,6 +142,28 @@ def test_prefill_degenerate_blocks(hip):
     assert_bits(got, amd64(data, xs, rows, cols), "degenerate activations")
 
 
+@pytest.mark.parametrize("qtype", [ref.Q4_K, ref.Q5_K, ref.Q6_K, ref.Q8_0, ref.Q4_0])
+@pytest.mark.parametrize("p", [3, 8, 16, 17, 40])
+def test_tiny_activations(hip, qtype, p):
+    """Activations so small that d * xscale and the sums are subnormal, against
+    the oracle; and smaller still, where 127 / amax overflows (the int8 codes
+    then are what the conversion of an infinity gives), against the one-token
+    kernels."""
+    rows, cols = 70, 6144
+    data = (quant_matrix(qtype, rows, cols, 970)[0] if qtype in (ref.Q4_K, ref.Q6_K, ref.Q8_0)
+            else random_rows(qtype, rows, cols, 970))
+    w = hip.Weight.from_host(data, qtype, rows, cols)
+    xs = normal(971 + p, (p, cols), 5e-37)
+    assert 0 < np.abs(xs).max() / 127 * 0.02 < np.finfo(np.float32).tiny
+    got = w.matvec_batch(xs)
+    assert np.any(got != 0)
+    assert_bits(got, amd64(data, xs, rows, cols, qtype), f"type {qtype} p={p}")
+    xs = normal(972 + p, (p, cols), 1e-38)
+    one = np.stack([w.matvec_batch(x[None])[0] for x in xs])
+    assert np.isfinite(one).all()
+    assert_bits(w.matvec_batch(xs), one, f"type {qtype} p={p} vs one token")
+
+
 def test_prefill_extremes_closed_form(hip):
     """TestAuditQ4KDotExtremes (q4k_q8_amd64_audit_test.go:18-52) batched: every
     code byte 0xff, d = dmin = 1, x = +-1 -> q8 = +-127, sc = m = 63, nibbles 15;
