@@ -260,10 +260,8 @@ static int ensure_buffers(gllm_hip_model* m, int p) {
     if (m->h_tokens) (void)hipHostFree(m->h_tokens);
     GLLM_HIP(hipMalloc(&m->d_tokens, (size_t)(p + 4) * 4));
     GLLM_HIP(hipHostMalloc(&m->h_tokens, (size_t)(p + 4) * 4, hipHostMallocDefault));
-    // every projection input's own size: the attention output may be wider than
-    // the FFN's, and rows past kSmallCols carry no records, so a narrower input
-    // may need more
-    const size_t an = std::max({act_bytes(c.dim, p), act_bytes(c.hidden, p), act_bytes(c.n_heads * c.head_dim, p)});
+    // the widest projection input: the attention output may be wider than the FFN's
+    const size_t an = act_bytes(std::max({c.dim, c.hidden, c.n_heads * c.head_dim}), p);
     if (m->act) (void)hipFree(m->act);
     GLLM_HIP(hipMalloc(&m->act, an));
     m->act_n = an;

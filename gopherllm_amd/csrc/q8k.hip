@@ -7,10 +7,15 @@
 //                        applies ScaleF32(xs, 32) where it reads them)
 // bit for bit, and writes q8 in the lane-permuted layout the row kernels read
 // (q8perm_offset in gllm_common.h).
+#include <algorithm>
+
 #include "gllm_common.h"
 
 namespace gllm {
 
+// Monotone in cols and in p: a buffer sized for its widest use serves every
+// narrower one.  Small batches past kSmallCols carry no records, but may not
+// need less than the widest that does.
 size_t act_bytes(int cols, int p) {
     size_t n = (size_t)cols * p;                   // q8perm
     n += (size_t)(cols / 256) * p * 4;             // xscale
@@ -24,6 +29,8 @@ size_t act_bytes(int cols, int p) {
     } else if (p > 1 && cols <= kSmallCols) {
         n = (n + 255) & ~(size_t)255;
         n += (size_t)(cols / 256) * 4 * small_rec(small_pt(p));  // rec
+    } else if (p > 1) {
+        return std::max(n + 256, act_bytes(kSmallCols, p));
     }
     return n + 256;
 }

@@ -203,7 +203,9 @@ int gllm_hip_matvec_dev_noalloc(gllm_hip_weight* w, const float* d_xs, int p, fl
  * matrices (acquireQ8 + fillQ4KXSums/fillQ6KXSums16, kernels_amd64.go:246,
  * then dotQ4KRowsQ8 / dotQ6KRowsQ8 / dotQ8_0RowsQ8, kernels_amd64.go:268-285,
  * 611-619).  d_act is a caller-owned device buffer of
- * gllm_hip_act_bytes(cols, p) bytes holding the quantised activations. */
+ * gllm_hip_act_bytes(cols, p) bytes holding the quantised activations; the
+ * size never falls as cols or p grows, so one buffer for the largest serves
+ * all. */
 size_t gllm_hip_act_bytes(int cols, int p);
 int gllm_hip_q8k_prepare_dev(const float* d_xs, int cols, int p, void* d_act, void* stream);
 int gllm_hip_matvec_q8_dev(gllm_hip_weight* w, const void* d_act, int p, float* d_outs,

@@ -48,6 +48,20 @@ def test_no_gpu_reports_unavailable_without_crashing():
     assert _lib.last_error()
 
 
+def test_act_bytes_never_falls():
+    """One activation buffer, sized for the widest input and most rows, serves
+    every smaller call, and the no-allocation call's 4 MiB hold what they did."""
+    from gopherllm_amd import act_bytes
+    widths = [256, 512, 4096, 32768, 65280, 65536, 65792, 66048, 70144, 98304, 131072, 190208]
+    rows = list(range(1, 20)) + [32, 33, 512]
+    size = {(c, p): act_bytes(c, p) for c in widths for p in rows}
+    for a, b in zip(widths, widths[1:]):
+        assert all(size[a, p] <= size[b, p] for p in rows), (a, b)
+    for a, b in zip(rows, rows[1:]):
+        assert all(size[c, a] <= size[c, b] for c in widths), (a, b)
+    assert all(size[c, 16] <= 4 << 20 for c in widths if c <= 98304)
+
+
 def test_product_does_not_import_the_oracle():
     pkg = os.path.join(ROOT, "gopherllm_amd")
     for dirpath, _, files in os.walk(pkg):
