@@ -1433,17 +1433,11 @@ static bool vdec_usable(int kvmul, int span_max) {
     if (kvmul != 1 && kvmul != 2 && kvmul != 4) return false;
     const size_t bytes = vdec_lds_bytes(kvmul, span_max);
     if (bytes <= 65536) return true;
-    static const bool big_ok = [] {
-        const int cap = 160 * 1024;
-        return hipFuncSetAttribute((const void*)attn_values_dec_kernel<4>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, cap) == hipSuccess &&
-               hipFuncSetAttribute((const void*)attn_values_dec_kernel<2>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, cap) == hipSuccess &&
-               hipFuncSetAttribute((const void*)attn_values_dec_kernel<1>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, cap) == hipSuccess;
-    }();
-    if (!big_ok) (void)hipGetLastError();
-    return big_ok && bytes <= 160 * 1024;
+    const size_t cap = 160 * 1024;
+    const void* kern = kvmul == 4   ? (const void*)attn_values_dec_kernel<4>
+                       : kvmul == 2 ? (const void*)attn_values_dec_kernel<2>
+                                    : (const void*)attn_values_dec_kernel<1>;
+    return bytes <= cap && lds_opt_in(kern, cap);
 }
 
 // Several tokens on the matrix cores (attn_prefill.hip) instead of a
@@ -1542,34 +1536,20 @@ int attend_exact(const gllm_hip_kv* kv, int l, const float* d_q, int n_heads, in
                 hipLaunchKernelGGL(attn_values_dec_kernel<1>, grid, dim3(kVDecThreads), lds, s, sc,
                                    kv->v[l], kv->kv_dim_v, start, span0, span_max, d_out, d_end);
         } else if (p == 1 && span_max <= kLongSpan) {
-            static const bool lds_ok = [] {
-                // dynamic LDS beyond 64 KB for long rows
-                return hipFuncSetAttribute((const void*)attn_values_long_kernel,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)long_lds_bytes(kLongSpan)) == hipSuccess;
-            }();
-            if (!lds_ok) {
-                (void)hipGetLastError();
-                if (long_lds_bytes(span_max) > 65536)
-                    return fail(GLLM_EDEVICE, "attend: %zu bytes of LDS not available",
-                                long_lds_bytes(span_max));
-            }
+            // dynamic LDS beyond 64 KB for long rows
+            if (!lds_opt_in((const void*)attn_values_long_kernel, long_lds_bytes(kLongSpan)) &&
+                long_lds_bytes(span_max) > 65536)
+                return fail(GLLM_EDEVICE, "attend: %zu bytes of LDS not available",
+                            long_lds_bytes(span_max));
             hipLaunchKernelGGL(attn_values_long_kernel, dim3(n_heads * 4), dim3(kLongThreads),
                                long_lds_bytes(span_max), s, sc, cmax, kv->v[l], kv->kv_dim_v,
                                kvmul, start, span0, span_max, d_out, d_end);
         } else if (p == 1) {
-            static const bool lds_ok = [] {
-                // dynamic LDS beyond 64 KB for long rows
-                return hipFuncSetAttribute((const void*)attn_softmax_values_kernel<4>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)smax_lds_bytes<4>(kSmaxSpan1)) == hipSuccess;
-            }();
-            if (!lds_ok) {
-                (void)hipGetLastError();
-                if (smax_lds_bytes<4>(span_max) > 65536)
-                    return fail(GLLM_EDEVICE, "attend: %zu bytes of LDS not available",
-                                smax_lds_bytes<4>(span_max));
-            }
+            // dynamic LDS beyond 64 KB for long rows
+            if (!lds_opt_in((const void*)attn_softmax_values_kernel<4>, smax_lds_bytes<4>(kSmaxSpan1)) &&
+                smax_lds_bytes<4>(span_max) > 65536)
+                return fail(GLLM_EDEVICE, "attend: %zu bytes of LDS not available",
+                            smax_lds_bytes<4>(span_max));
             hipLaunchKernelGGL(attn_softmax_values_kernel<4>, dim3(n_heads * 4, p), dim3(256),
                                smax_lds_bytes<4>(span_max), s, sc, kv->v[l], kv->kv_dim_v, kvmul,
                                start, span0, span_max, d_out, d_end);

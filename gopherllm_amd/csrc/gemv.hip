@@ -1964,22 +1964,8 @@ static void (*fmt_kernel(int g))(GemvJob) {
 }
 
 // Dynamic LDS of the staged batch activations: up to the 160 KB a gfx950
-// workgroup may use, after a one-time opt-in per kernel.
+// workgroup may use, after an opt-in per kernel and device.
 constexpr size_t kStagedActMax = 160 * 1024 - 64;
-static bool lds_opt_in(const void* kern) {
-    static std::mutex mu;
-    static std::vector<const void*> done;
-    std::lock_guard<std::mutex> lock(mu);
-    for (const void* d : done)
-        if (d == kern) return true;
-    if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kStagedActMax) !=
-        hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    done.push_back(kern);
-    return true;
-}
 
 // The Q6_K, Q8_0 and other-format row kernel for this type, batch tile NT
 // and G; FUSE selects the variant that quantises x itself; shallow: the
@@ -2040,7 +2026,7 @@ static int launch_q4k_bp_inst(GemvJob& j, const int* rows, hipStream_t s) {
                                        : gemv_q4k_bp_kernel<B, NS, NTH, RP, 2, P>;
         else if (j.xf) kern = gemv_q4k_bp_kernel<B, NS, NTH, RP, 1, P>;
     }
-    if (lds > 64 * 1024 && !lds_opt_in((const void*)kern))
+    if (lds > 64 * 1024 && !lds_opt_in((const void*)kern, kStagedActMax))
         return fail(GLLM_EDEVICE, "gemv: %zu B of LDS refused", lds);
     hipLaunchKernelGGL(kern, dim3(wg), dim3(NTH), lds, s, j);
     GLLM_HIP(hipGetLastError());
@@ -2084,7 +2070,7 @@ template <int B, int R, int NS, int NLD, int D>
 static int launch_q4k_ws_inst(GemvJob& j, const int* rows, hipStream_t s) {
     constexpr size_t lds = Q4KWsLayout<B, R>::bytes;
     auto kern = gemv_q4k_ws_kernel<B, R, NS, NLD, D>;
-    if (lds > 64 * 1024 && !lds_opt_in((const void*)kern))
+    if (lds > 64 * 1024 && !lds_opt_in((const void*)kern, kStagedActMax))
         return fail(GLLM_EDEVICE, "gemv: %zu B of LDS refused", lds);
     hipLaunchKernelGGL(kern, dim3((rows[0] + R - 1) / R), dim3(R * 8 * NS + NLD * 64), lds, s,
                        j.w[0], j.xf, j.out[0], rows[0], (int)j.rb);
@@ -2148,7 +2134,7 @@ int launch_gemv_nt(GemvJob& j, int type, int grid, const int* rows, hipStream_t 
     j.sa = 0;
     if (NT > 1 && (type == GLLM_TYPE_Q6_K || type == GLLM_TYPE_Q8_0)) {
         lds = staged_act_bytes(j.ntok, j.cols, type == GLLM_TYPE_Q6_K);
-        if (lds <= kStagedActMax && lds_opt_in((const void*)kern)) {
+        if (lds <= kStagedActMax && lds_opt_in((const void*)kern, kStagedActMax)) {
             j.sa = 1;
         } else {
             lds = 0;

@@ -35,6 +35,9 @@ int check(hipError_t e, const char* what);
 hipStream_t thread_stream();
 // Compute units of the current device (cached per device).
 int device_cus();
+// Allows `kern` to be launched with up to `bytes` of dynamic LDS on the current
+// device (asked for once per device); false if the device refuses.
+bool lds_opt_in(const void* kern, size_t bytes);
 // Growable device scratch of the calling thread for work on `stream` (slot
 // 0..11).  Null, with the error set, when it cannot grow: allocation failed,
 // or the stream is being captured into a graph.

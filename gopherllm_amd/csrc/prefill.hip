@@ -672,25 +672,18 @@ __global__ __launch_bounds__(1024) void prefill_q4k_lanes_kernel(PfArgs a, TlMap
 
 // One workgroup of 1024 threads per 64 x 64 tile.
 template <size_t LDS>
-static int launch_lanes(void (*kern)(PfArgs, TlMap), bool lds_ok, const PfArgs& a, hipStream_t s) {
+static int launch_lanes(void (*kern)(PfArgs, TlMap), const PfArgs& a, hipStream_t s) {
     static_assert(LDS >= 65536 && LDS <= 160 * 1024, "the stages, and the exchange over them");
-    if (!lds_ok) return fail(GLLM_EDEVICE, "prefill: %zu bytes of LDS were refused", LDS);
+    if (!lds_opt_in((const void*)kern, LDS)) return fail(GLLM_EDEVICE, "prefill: %zu bytes of LDS were refused", LDS);
     const TlMap mp = tl_map(a.rows, a.p);
     hipLaunchKernelGGL(kern, dim3(8 * mp.tg_size * mp.rg_size), dim3(1024), LDS, s, a, mp);
     return GLLM_OK;
-}
-static bool lanes_lds(const void* kern, size_t lds) {
-    if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess) return true;
-    (void)hipGetLastError();
-    return false;
 }
 
 template <bool Q5>
 static int launch_q4k_lanes(const PfArgs& a, hipStream_t s) {
     constexpr size_t lds = 2 * sizeof(LnStage<Q5>);
-    static const bool ok = lanes_lds((const void*)prefill_q4k_lanes_kernel<Q5, 4>, lds) &&
-                           lanes_lds((const void*)prefill_q4k_lanes_kernel<Q5, 2>, lds);
-    return launch_lanes<lds>(a.p <= kHalfTok ? prefill_q4k_lanes_kernel<Q5, 2> : prefill_q4k_lanes_kernel<Q5, 4>, ok, a, s);
+    return launch_lanes<lds>(a.p <= kHalfTok ? prefill_q4k_lanes_kernel<Q5, 2> : prefill_q4k_lanes_kernel<Q5, 4>, a, s);
 }
 
 int launch_q5k_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,
@@ -928,9 +921,7 @@ int launch_q6k_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const 
                     kTiledMinP);
     PfArgs a{d_w, rb, rows, blocks, act, p, out, out_stride};
     constexpr size_t lds = 2 * sizeof(Q6Stage);
-    static const bool ok = lanes_lds((const void*)prefill_q6k_lanes_kernel<4>, lds) &&
-                           lanes_lds((const void*)prefill_q6k_lanes_kernel<2>, lds);
-    GLLM_TRY((launch_lanes<lds>(p <= kHalfTok ? prefill_q6k_lanes_kernel<2> : prefill_q6k_lanes_kernel<4>, ok, a, s)));
+    GLLM_TRY((launch_lanes<lds>(p <= kHalfTok ? prefill_q6k_lanes_kernel<2> : prefill_q6k_lanes_kernel<4>, a, s)));
     GLLM_HIP(hipGetLastError());
     return GLLM_OK;
 }
@@ -1100,9 +1091,7 @@ int launch_q8_0_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const
         return fail(GLLM_EINVAL, "prefill: Q8_0 tiles need > %d tokens and < 4 GiB operands", kTiledMinP);
     PfArgs a{d_w, rb, rows, blocks, act, p, out, out_stride};
     constexpr size_t lds = 2 * sizeof(Q80Stage);
-    static const bool ok = lanes_lds((const void*)prefill_q8_0_lanes_kernel<4>, lds) &&
-                           lanes_lds((const void*)prefill_q8_0_lanes_kernel<2>, lds);
-    GLLM_TRY((launch_lanes<lds>(p <= kHalfTok ? prefill_q8_0_lanes_kernel<2> : prefill_q8_0_lanes_kernel<4>, ok, a, s)));
+    GLLM_TRY((launch_lanes<lds>(p <= kHalfTok ? prefill_q8_0_lanes_kernel<2> : prefill_q8_0_lanes_kernel<4>, a, s)));
     GLLM_HIP(hipGetLastError());
     return GLLM_OK;
 }
@@ -1267,8 +1256,7 @@ int launch_q4_0_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const
         return fail(GLLM_EINVAL, "prefill: Q4_0 tiles need > %d tokens and < 4 GiB", kTiledMinP);
     PfArgs a{d_w, rb, rows, blocks, act, p, out, out_stride};
     constexpr size_t lds = 2 * sizeof(Q40Stage);
-    static const bool ok = lanes_lds((const void*)prefill_q4_0_lanes_kernel, lds);
-    GLLM_TRY((launch_lanes<lds>(prefill_q4_0_lanes_kernel, ok, a, s)));
+    GLLM_TRY((launch_lanes<lds>(prefill_q4_0_lanes_kernel, a, s)));
     GLLM_HIP(hipGetLastError());
     return GLLM_OK;
 }

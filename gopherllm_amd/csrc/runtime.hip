@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "gllm_common.h"
+#include "lds_optin.h"
 
 namespace gllm {
 
@@ -94,6 +95,15 @@ int device_cus() {
         cus[d] = n;
     }
     return cus[d];
+}
+
+bool lds_opt_in(const void* kern, size_t bytes) {
+    static LdsOptIn opt;
+    return opt.allow(current_device(), kern, bytes, [](const void* k, size_t n) {
+        if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)n) == hipSuccess) return true;
+        (void)hipGetLastError();
+        return false;
+    });
 }
 
 hipStream_t thread_stream() {
