@@ -2226,10 +2226,19 @@ int run_gemv(int n, gllm_hip_weight* const* ws, const ActQ8& act, int p, float* 
     if (wg == 0) return GLLM_OK;
     auto all = [&](auto fits) { return std::all_of(ws, ws + n, fits); };
     if (all([&](auto* w) { return small_batch_fits(act, p, w); })) {
-        for (int i = 0; i < n; i++)
-            GLLM_TRY(launch_small_lanes(w0->type == GLLM_TYPE_Q6_K, ws[i]->d_data, ws[i]->row_bytes, ws[i]->rows,
-                                        ws[i]->blocks, act, p, outs[i], j.out_stride[i], s));
-        return GLLM_OK;
+        SmallJob sj{};
+        for (int i = 0; i < n; i++) {
+            sj.w[i] = j.w[i];
+            sj.out[i] = j.out[i];
+            sj.rows[i] = j.rows[i];
+            sj.out_stride[i] = j.out_stride[i];
+        }
+        sj.n = n;
+        sj.blocks = j.blocks;
+        sj.p = p;
+        sj.rb = j.rb;
+        sj.rec = act.rec;
+        return launch_small_lanes(w0->type == GLLM_TYPE_Q6_K, sj, s);
     }
     if (w0->type == GLLM_TYPE_Q4_K && p >= kMfmaMinTok) {
         // batched prefill: matrix-core products, same bits as the row kernel

@@ -102,10 +102,18 @@ int launch_q5k_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const 
 // Batched Q4_0 x Q8_K on the matrix cores, same contract and needs.
 int launch_q4_0_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,
                       float* out, int out_stride, hipStream_t s);
-// 2 to kTiledMinP rows of Q4_K (q6: Q6_K, blocks % 8 == 0) x Q8_K, same
-// contract; needs act.rec and rows * rb < 4 GiB.
-int launch_small_lanes(bool q6, const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,
-                       float* out, int out_stride, hipStream_t s);
+// 2 to kTiledMinP rows of up to three weights of one type and width, Q4_K (q6:
+// Q6_K, blocks % 8 == 0) x Q8_K, same contract; needs the records and
+// rows * rb < 4 GiB.  wg_begin is the launcher's.
+struct SmallJob {
+    const uint8_t* w[3];
+    float* out[3];
+    int rows[3], out_stride[3], wg_begin[3];
+    int n, blocks, p;
+    size_t rb;
+    const uint8_t* rec;
+};
+int launch_small_lanes(bool q6, SmallJob j, hipStream_t s);
 // Batched Q8_0 x Q8_K on the matrix cores, same contract; needs the f16 tiles
 // (p > kTiledMinP) and operands under 4 GiB.
 int launch_q8_0_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,

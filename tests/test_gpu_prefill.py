@@ -34,6 +34,16 @@ def assert_bits(got, want, what):
         f"{got[tuple(bad[0])]} vs {want[tuple(bad[0])]}"
 
 
+def matvec_group(hip, ws, xs):
+    """One call for weights that share their input."""
+    import torch
+    x = torch.from_numpy(xs).cuda()
+    outs = [torch.full((len(xs), w.rows), -1.0, device="cuda") for w in ws]
+    hip.matvec_multi_dev(ws, x, outs)
+    torch.cuda.synchronize()
+    return [o.cpu().numpy() for o in outs]
+
+
 @pytest.mark.parametrize("rows,cols,p", [(300, 1024, 16), (300, 1024, 33), (64, 256, 100),
                                          (1000, 4096, 64), (70, 14336, 40)])
 def test_prefill_bit_exact_small(hip, rows, cols, p):
@@ -123,6 +133,19 @@ def test_small_batch_edges(hip, qtype, rows, cols, p):
     xs = normal(931 + p, (p, cols))
     xs[p // 2, :256] = 0.0
     assert_bits(w.matvec_batch(xs), amd64(data, xs, rows, cols, qtype), f"{rows}x{cols} p={p}")
+
+
+@pytest.mark.parametrize("qtype", [ref.Q4_K, ref.Q6_K])
+@pytest.mark.parametrize("rows,cols,p", [((33, 16, 1), 6144, 5), ((4100, 1040), 2048, 8), ((4097, 1024, 3100), 2048, 6),
+                                         ((17, 40, 48), 6144, 13), ((16, 500), 8192, 4)])
+def test_small_batch_groups(hip, qtype, rows, cols, p):
+    """Two and three weights in one grid: short last row tiles, a weight of one
+    row, enough workgroups for either split of the lane pairs."""
+    xs = normal(991 + p, (p, cols))
+    data = [quant_matrix(qtype, r, cols, 990 + i)[0] for i, r in enumerate(rows)]
+    got = matvec_group(hip, [hip.Weight.from_host(d, qtype, r, cols) for d, r in zip(data, rows)], xs)
+    for i, (d, r) in enumerate(zip(data, rows)):
+        assert_bits(got[i], amd64(d, xs, r, cols, qtype), f"weight {i} of {rows} x {cols} p={p}")
 
 
 def test_prefill_degenerate_blocks(hip):
