@@ -1890,11 +1890,17 @@ static Q4KShape q4k_shape(int total_rows, int blocks) {
     return best;
 }
 
+// The launch has an unrolled kernel with its activations staged in LDS (the
+// generic kernel otherwise).
+static bool q4k_compiled(int nt, const Q4KShape& sh, int blocks) {
+    return q4k_stage_bytes(nt, blocks * 256) <= kMaxStage && q4k_has_nl(blocks / sh.g) && sh.threads >= 256;
+}
+
 template <int NT, int G>
 int launch_q4k(GemvJob& j, const int* rows, int n, const Q4KShape& sh, hipStream_t s) {
     const int nl = j.blocks / G;
     const size_t stage = q4k_stage_bytes(NT, j.cols);
-    const bool compiled = stage <= kMaxStage && q4k_has_nl(nl) && sh.threads >= 256;
+    const bool compiled = q4k_compiled(NT, sh, j.blocks);
     if (j.xf && (NT != 1 || !compiled || j.cols > kFuseCols))
         return fail(GLLM_EINVAL, "gemv: fused quantisation needs batch 1 and a compiled shape");
     // the generic kernel keeps 256-thread workgroups of 32 / G rows
@@ -2171,16 +2177,56 @@ static bool q6k_tiled_fits(const ActQ8& act, int p, const gllm_hip_weight* w) {
            (size_t)w->rows * w->row_bytes < ((size_t)1 << 32);
 }
 
-// The small-batch matrix-core kernel applies (launch_small_lanes).  Its cost
-// hardly depends on the tokens, the row kernels' does: at 14336 x 4096 Q4_K
-// takes 13.2 / 16.2 us at 2 / 4 tokens on the row kernels and 15.8 / 16.3 here
-// (at 4096 columns they walk a row in few steps; 4096 x 14336 at 2 tokens
-// takes 25.1 there and 18.3 here); Q6_K 4096 x 14336 takes 24.5 / 29.4 / 33.1
-// at 2 / 3 / 4 and 14336 x 4096 18.2 / 21.2 / 24.1, here 26.5 and 23.8.
-static bool small_batch_fits(const ActQ8& act, int p, const gllm_hip_weight* w) {
-    if (!act.rec || p < 2 || (size_t)w->rows * w->row_bytes >= ((size_t)1 << 32)) return false;
-    if (w->type == GLLM_TYPE_Q4_K) return p > 4 || w->cols > 4096;
-    return w->type == GLLM_TYPE_Q6_K && w->blocks % 8 == 0 && p >= 4;
+// 2 to 16 rows: true when launch_small_lanes takes these weights (one type and
+// width, one grid) and is the fastest of the kernels that could.  It streams
+// few rows best and hardly depends on the tokens.  The row kernels pay per
+// token, but a row count that their compiled shapes split well runs near the
+// memory rate; the 64 x 16 tiles (launch_q4k_mfma) win on many rows from 8
+// tokens on.  Lines from a scan of 512 .. 57344 rows x 1024 .. 28672 columns with
+// the weights rotating through 320 MB and the quantiser launch included
+// (us: this kernel / the other):
+//   Q4_K up to 4 tokens, up to 4096 columns: 14336 x 4096 at 2 15.8 / 13.2, at 4
+//     16.3 / 16.2
+//   compiled rows (8192 columns): 1024 rows at 2 12.4 / 13.9, 4096 13.3 / 12.6;
+//     at 3 4096 13.1 / 14.1, 6144 19.7 / 19.0; at 4 6144 19.8 / 21.7, 8192 21.8
+//     / 19.3, 28672 52 / 45
+//   other rows: 4096 x 5120 at 2 10.2 / 27.4, 28672 x 5120 43.4 / 40.3, at 3 42.7
+//     / 48.1; 57344 x 5120 at 4 73.3 / 71.3, x 14336 186 / 176 at 2 and 187 / 235
+//     at 3
+//   5 to 7 tokens: 14336 x 4096 19.1 / 19.3, 28672 x 4096 33.8 / 27.7 at 5, 33.7 /
+//     30.3 at 6, 33.5 / 33.0 at 7 (x 1024 14.8 / 13.8)
+//   8 tokens: 14336 x 4096 19.0 / 21.7, 28672 x 4096 33.7 / 31.4, x 8192 51.9 / 52.6,
+//     57344 x 14336 (no cache holds it) 188 / 177
+//   9 to 16: 8192 x 4096 14.9 / 25.7, 14336 x 4096 24.8 / 22.0, x 14336 54.1 / 57.8,
+//     28672 x 14336 90.8 / 82.8
+//   Q6_K at 4: 512 x 14336 26.3 / 24.7, 1024 x 8192 17.8 / 17.3, 4096 x 4096 12.2 /
+//     15.8; at 3 14336 x 4096 23.8 / 21.2
+static bool small_batch_fits(int n, gllm_hip_weight* const* ws, int p) {
+    const gllm_hip_weight* w0 = ws[0];
+    if (p < 2 || p > kTiledMinP || w0->cols > kSmallCols) return false;
+    int total = 0, fewest = w0->rows;
+    size_t bytes = 0;
+    for (int i = 0; i < n; i++) {
+        const size_t b = (size_t)ws[i]->rows * ws[i]->row_bytes;
+        if (b >= ((size_t)1 << 32)) return false;
+        total += ws[i]->rows;
+        fewest = std::min(fewest, ws[i]->rows);
+        bytes += b;
+    }
+    const int blocks = w0->blocks;
+    if (w0->type == GLLM_TYPE_Q6_K) return blocks % 8 == 0 && (p > 4 || (p == 4 && total > 1024));
+    if (w0->type != GLLM_TYPE_Q4_K) return false;
+    if (p < kMfmaMinTok) {
+        const bool compiled = q4k_compiled(p <= 4 ? 4 : 8, q4k_shape(total, blocks), blocks);
+        if (p > 4) return !compiled || total < 24576 || (p == 7 && blocks > 4);
+        if (w0->cols <= 4096) return false;
+        if (compiled) return total < (p == 2 ? 4096 : p == 3 ? 6144 : 8192);
+        if (p == 2) return total < (blocks < 56 ? 24576 : 49152);
+        return blocks >= 56 || total < 49152;
+    }
+    if (p == 8) return n > 1 || total < 20480 || (blocks > 20 && bytes < ((size_t)300 << 20));
+    // the 64-row tiles of every weight cover two thirds of the CUs
+    return (fewest + 63) / 64 < 2 * device_cus() / 3 || (blocks >= 56 && fewest < 20480);
 }
 
 int run_gemv(int n, gllm_hip_weight* const* ws, const ActQ8& act, int p, float* const* outs,
@@ -2225,7 +2271,7 @@ int run_gemv(int n, gllm_hip_weight* const* ws, const ActQ8& act, int p, float* 
     j.wg_begin[n] = wg;
     if (wg == 0) return GLLM_OK;
     auto all = [&](auto fits) { return std::all_of(ws, ws + n, fits); };
-    if (all([&](auto* w) { return small_batch_fits(act, p, w); })) {
+    if (act.rec && small_batch_fits(n, ws, p)) {
         SmallJob sj{};
         for (int i = 0; i < n; i++) {
             sj.w[i] = j.w[i];
@@ -2317,8 +2363,13 @@ int gemv_f32(int n, gllm_hip_weight* const* ws, const float* d_xs, int p, float*
         } else {
             if (!quantised) {
                 act_carve(act_buf, cols, p, &act);
-                // records only for a weight that reads them
-                if (std::none_of(ws + i, ws + n, [&](auto* w) { return small_batch_fits(act, p, w); })) act.rec = nullptr;
+                // records only for a run of weights that reads them
+                bool records = false;
+                for (int a = i, b; a < n; a = b) {
+                    for (b = a + 1; b < n && ws[b]->type == ws[a]->type;) b++;
+                    records = records || small_batch_fits(b - a, ws + a, p);
+                }
+                if (!records) act.rec = nullptr;
                 GLLM_TRY(launch_q8k_prep(d_xs, cols, p, act, s));
                 quantised = true;
             }
@@ -2436,7 +2487,7 @@ int gemv_silu_f32(gllm_hip_weight* w, const float* gate, const float* up, int p,
     }
     ActQ8 act;
     act_carve(act_buf, w->cols, p, &act);
-    if (!small_batch_fits(act, p, w)) act.rec = nullptr;
+    if (!small_batch_fits(1, ws, p)) act.rec = nullptr;
     GLLM_TRY(launch_q8k_prep_silu(gate, up, w->cols, p, act, s));
     return run_gemv(1, ws, act, p, outs, nullptr, s, nullptr);
 }

@@ -148,6 +148,19 @@ def test_small_batch_groups(hip, qtype, rows, cols, p):
         assert_bits(got[i], amd64(d, xs, r, cols, qtype), f"weight {i} of {rows} x {cols} p={p}")
 
 
+@pytest.mark.parametrize("rows,cols,p", [(10816, 512, 12), (10817, 768, 9), (10830, 2304, 15), (20480, 256, 8),
+                                         (20479, 256, 8), (24576, 1024, 6), (24576, 1024, 7), (4100, 8192, 2),
+                                         (4090, 8192, 2), (6144, 8192, 3), (8192, 2048, 16)])
+def test_small_batch_routes(hip, rows, cols, p):
+    """Both sides of the lines between the small-batch kernel, the row kernels
+    and the 64 x 16 tiles (one block or an odd count, short last row tiles,
+    fewer than 16 tokens)."""
+    data = np.tile(quant_matrix(ref.Q4_K, 50, cols, 995)[0], -(-rows // 50))[:rows * (cols // 256) * 144]
+    w = hip.Weight.from_host(data, ref.Q4_K, rows, cols)
+    xs = normal(996 + p, (p, cols))
+    assert_bits(w.matvec_batch(xs), amd64(data, xs, rows, cols), f"{rows}x{cols} p={p}")
+
+
 def test_prefill_degenerate_blocks(hip):
     """All-zero tokens, zero 256-blocks inside a token, a lone large value and
     NaN-free extremes (q8kQuantize's scale-0 blocks, quant_q8k_portable.go:36-62)."""
