@@ -2171,10 +2171,12 @@ struct NormIn {
     ActQ8 sq_act;
 };
 
-// The batched Q6_K matrix-core kernel applies (launch_q6k_tiled).
-static bool q6k_tiled_fits(const ActQ8& act, int p, const gllm_hip_weight* w) {
-    return p > kTiledMinP && act.b16t && w->blocks % 8 == 0 &&
-           (size_t)w->rows * w->row_bytes < ((size_t)1 << 32);
+// The matrix-core kernels of more than kTiledMinP rows apply to every weight of
+// the group: 32-bit offsets into a weight and, Q6_K, 16-byte aligned blocks.
+static bool lanes_fit(int n, gllm_hip_weight* const* ws, const ActQ8& act, int p) {
+    return p > kTiledMinP && act.b16t && std::all_of(ws, ws + n, [](auto* w) {
+        return (size_t)w->rows * w->row_bytes < ((size_t)1 << 32) && (w->type != GLLM_TYPE_Q6_K || w->blocks % 8 == 0);
+    });
 }
 
 // 2 to 16 rows: true when launch_small_lanes takes these weights (one type and
@@ -2270,7 +2272,6 @@ int run_gemv(int n, gllm_hip_weight* const* ws, const ActQ8& act, int p, float* 
     }
     j.wg_begin[n] = wg;
     if (wg == 0) return GLLM_OK;
-    auto all = [&](auto fits) { return std::all_of(ws, ws + n, fits); };
     if (act.rec && small_batch_fits(n, ws, p)) {
         SmallJob sj{};
         for (int i = 0; i < n; i++) {
@@ -2293,25 +2294,15 @@ int run_gemv(int n, gllm_hip_weight* const* ws, const ActQ8& act, int p, float* 
                                      act, p, outs[i], j.out_stride[i], s));
         return GLLM_OK;
     }
-    if (w0->type == GLLM_TYPE_Q8_0 && p > kTiledMinP && (size_t)w0->rows * w0->row_bytes < ((size_t)1 << 32) &&
-        (size_t)p * w0->cols < ((size_t)1 << 32)) {
+    const auto lanes = w0->type == GLLM_TYPE_Q8_0   ? launch_q8_0_tiled
+                       : w0->type == GLLM_TYPE_Q6_K ? launch_q6k_tiled
+                       : w0->type == GLLM_TYPE_Q5_K ? launch_q5k_tiled
+                       : w0->type == GLLM_TYPE_Q4_0 ? launch_q4_0_tiled
+                                                    : nullptr;
+    if (lanes && lanes_fit(n, ws, act, p)) {
         for (int i = 0; i < n; i++)
-            GLLM_TRY(launch_q8_0_tiled(ws[i]->d_data, ws[i]->row_bytes, ws[i]->rows, ws[i]->blocks,
-                                       act, p, outs[i], j.out_stride[i], s));
-        return GLLM_OK;
-    }
-    if ((w0->type == GLLM_TYPE_Q5_K || w0->type == GLLM_TYPE_Q4_0) && p > kTiledMinP &&
-        all([](auto* w) { return (size_t)w->rows * w->row_bytes < ((size_t)1 << 32); })) {
-        const auto launch = w0->type == GLLM_TYPE_Q5_K ? launch_q5k_tiled : launch_q4_0_tiled;
-        for (int i = 0; i < n; i++)
-            GLLM_TRY(launch(ws[i]->d_data, ws[i]->row_bytes, ws[i]->rows, ws[i]->blocks, act, p, outs[i],
-                            j.out_stride[i], s));
-        return GLLM_OK;
-    }
-    if (w0->type == GLLM_TYPE_Q6_K && q6k_tiled_fits(act, p, w0)) {
-        for (int i = 0; i < n; i++)
-            GLLM_TRY(launch_q6k_tiled(ws[i]->d_data, ws[i]->row_bytes, ws[i]->rows, ws[i]->blocks,
-                                      act, p, outs[i], j.out_stride[i], s));
+            GLLM_TRY(lanes(ws[i]->d_data, ws[i]->row_bytes, ws[i]->rows, ws[i]->blocks, act, p, outs[i],
+                           j.out_stride[i], s));
         return GLLM_OK;
     }
     for (int t0 = 0; t0 < p; t0 += kMaxTok) {

@@ -114,8 +114,7 @@ struct SmallJob {
     const uint8_t* rec;
 };
 int launch_small_lanes(bool q6, SmallJob j, hipStream_t s);
-// Batched Q8_0 x Q8_K on the matrix cores, same contract; needs the f16 tiles
-// (p > kTiledMinP) and operands under 4 GiB.
+// Batched Q8_0 x Q8_K on the matrix cores, same contract and needs.
 int launch_q8_0_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,
                       float* out, int out_stride, hipStream_t s);
 // Same, for the activation siluMulF32(gate, up) computed on the fly.

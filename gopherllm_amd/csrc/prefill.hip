@@ -1087,8 +1087,8 @@ __global__ __launch_bounds__(1024) void prefill_q8_0_lanes_kernel(PfArgs a, TlMa
 int launch_q8_0_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,
                       float* out, int out_stride, hipStream_t s) {
     if (rows <= 0 || blocks <= 0 || p <= 0) return GLLM_OK;
-    if (p <= kTiledMinP || (size_t)rows * rb >= ((size_t)1 << 32) || (size_t)p * blocks * 256 >= ((size_t)1 << 32))
-        return fail(GLLM_EINVAL, "prefill: Q8_0 tiles need > %d tokens and < 4 GiB operands", kTiledMinP);
+    if (!act.b16t || p <= kTiledMinP || (size_t)rows * rb >= ((size_t)1 << 32))
+        return fail(GLLM_EINVAL, "prefill: Q8_0 tiles need > %d tokens and < 4 GiB", kTiledMinP);
     PfArgs a{d_w, rb, rows, blocks, act, p, out, out_stride};
     constexpr size_t lds = 2 * sizeof(Q80Stage);
     GLLM_TRY((launch_lanes<lds>(p <= kHalfTok ? prefill_q8_0_lanes_kernel<2> : prefill_q8_0_lanes_kernel<4>, a, s)));

@@ -161,6 +161,32 @@ def test_small_batch_routes(hip, rows, cols, p):
     assert_bits(w.matvec_batch(xs), amd64(data, xs, rows, cols), f"{rows}x{cols} p={p}")
 
 
+@pytest.mark.parametrize("qtype,p", [(ref.Q8_0, 17), (ref.Q6_K, 17), (ref.Q5_K, 17), (ref.Q4_0, 17), (ref.Q4_K, 9)])
+def test_group_with_a_weight_past_4_gib(hip, qtype, p):
+    """The kernels with 32-bit offsets look at every weight of a group: 64 rows
+    beside the same rows repeated past 4 GiB."""
+    import torch
+    cols = 4096
+    data = (quant_matrix(qtype, 64, cols, 997)[0] if qtype in (ref.Q4_K, ref.Q6_K, ref.Q8_0)
+            else random_rows(qtype, 64, cols, 997))
+    times = (1 << 32) // len(data) + 1
+    raw = torch.from_numpy(data).cuda().repeat(times)
+    assert raw.numel() > 1 << 32
+    ws = [hip.Weight.from_host(data, qtype, 64, cols), hip.Weight.from_device(raw, qtype, 64 * times, cols)]
+    del raw
+    xs = normal(998, (p, cols))
+    x = torch.from_numpy(xs).cuda()
+    outs = [torch.full((p, w.rows), -1.0, device="cuda") for w in ws]
+    print(f"type {qtype}, weights of 64 and {64 * times} rows", flush=True)
+    hip.matvec_multi_dev(ws, x, outs)
+    torch.cuda.synchronize()
+    want = torch.from_numpy(amd64(data, xs, 64, cols, qtype)).cuda()
+    assert torch.equal(outs[0].view(torch.int32), want.view(torch.int32))
+    assert (outs[1].view(torch.int32).view(p, times, 64) == want.view(torch.int32)[:, None]).all()
+    del ws, outs
+    torch.cuda.empty_cache()
+
+
 def test_prefill_degenerate_blocks(hip):
     """All-zero tokens, zero 256-blocks inside a token, a lone large value and
     NaN-free extremes (q8kQuantize's scale-0 blocks, quant_q8k_portable.go:36-62)."""
