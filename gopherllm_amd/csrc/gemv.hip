@@ -2172,10 +2172,13 @@ struct NormIn {
 };
 
 // The matrix-core kernels of more than kTiledMinP rows apply to every weight of
-// the group: 32-bit offsets into a weight and, Q6_K, 16-byte aligned blocks.
+// the group: 32-bit offsets into a weight and, Q6_K, 16-byte aligned blocks and
+// 32-bit offsets into xs16 too.
 static bool lanes_fit(int n, gllm_hip_weight* const* ws, const ActQ8& act, int p) {
-    return p > kTiledMinP && act.b16t && std::all_of(ws, ws + n, [](auto* w) {
-        return (size_t)w->rows * w->row_bytes < ((size_t)1 << 32) && (w->type != GLLM_TYPE_Q6_K || w->blocks % 8 == 0);
+    const size_t max32 = (size_t)1 << 32;
+    return p > kTiledMinP && act.b16t && std::all_of(ws, ws + n, [&](auto* w) {
+        return (size_t)w->rows * w->row_bytes < max32 &&
+               (w->type != GLLM_TYPE_Q6_K || (w->blocks % 8 == 0 && (size_t)p * w->blocks * 64 < max32));
     });
 }
 

@@ -916,8 +916,9 @@ __global__ __launch_bounds__(1024) void prefill_q6k_lanes_kernel(PfArgs a, TlMap
 int launch_q6k_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,
                      float* out, int out_stride, hipStream_t s) {
     if (rows <= 0 || blocks <= 0 || p <= 0) return GLLM_OK;
-    if (!act.b16t || p <= kTiledMinP || blocks % 8 || (size_t)rows * rb >= ((size_t)1 << 32))
-        return fail(GLLM_EINVAL, "prefill: Q6_K tiles need > %d tokens, blocks %% 8 == 0, < 4 GiB",
+    if (!act.b16t || p <= kTiledMinP || blocks % 8 || (size_t)rows * rb >= ((size_t)1 << 32) ||
+        (size_t)p * blocks * 64 >= ((size_t)1 << 32))
+        return fail(GLLM_EINVAL, "prefill: Q6_K tiles need > %d tokens, blocks %% 8 == 0, < 4 GiB of weight and of sums",
                     kTiledMinP);
     PfArgs a{d_w, rb, rows, blocks, act, p, out, out_stride};
     constexpr size_t lds = 2 * sizeof(Q6Stage);
