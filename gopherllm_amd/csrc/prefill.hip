@@ -25,18 +25,18 @@
 // 8s + 4 + i (high nibble, sub-block 2s + 1).  MFMA lane L supplies
 // kappa = 8(L/16) .. 8(L/16) + 7 of both operands, i.e. one weight dword.
 //
-// Three kinds of kernel follow: prefill_q4k_mfma_kernel (8 to 16 tokens of
-// weights or columns past what the others address), the *_lanes_kernels (more
-// than 16 tokens, every format below on its own chains) and
-// small_lanes_kernel (2 to 16 tokens).
+// Three kinds of kernel follow: prefill_q4k_mfma_kernel (8 to 16 tokens, where
+// the rows fill the GPU or the activations carry no records), the *_lanes_kernels
+// (more than 16 tokens, every format below on its own chains) and
+// small_lanes_kernel (2 to 16 tokens).  The last two take the activations as
+// the A operand and the weights as B.
 //
-// prefill_q4k_mfma_kernel: a workgroup is RW x TW waves over 16 RW weight
-// rows x 16 TW tokens; wave w owns the 16x16 tile of rows 16 (w % RW) .. + 15
-// and tokens 16 (w / RW) .. + 15.  Per block the workgroup stages the tokens'
-// q8 (as f16), xsums and xscales and the rows' decoded scales/mins and nibble
-// bytes in LDS (double-buffered, loaded one block ahead).
-#include <cstdlib>
-
+// prefill_q4k_mfma_kernel: a workgroup is four waves over 64 weight rows x 16
+// tokens; wave w owns the 16x16 tile of rows 16 w .. + 15.  Per block the
+// workgroup stages the tokens' q8 (as f16), xsums and xscales and the rows'
+// decoded scales/mins and nibble bytes in LDS (double-buffered, loaded one
+// block ahead).  It wins over small_lanes_kernel with many rows, see
+// small_batch_fits for both sides.
 #include "gllm_common.h"
 
 namespace gllm {
@@ -48,23 +48,22 @@ typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 constexpr int kPfBStride = 528;  // bytes per token row of the f16 q8 tile: 512 + 16 (no bank conflicts)
 constexpr int kPfWStride = 36;   // dwords per row of the staged weight nibbles: 32 + 4
 
-// One block's staged operands for a workgroup of RW 16-row groups x TW
-// 16-token columns.
-template <int RW, int TW>
+constexpr int kPfRows = 64, kPfTok = 16, kPfThreads = 256;  // of a workgroup
+
+// One block's staged operands of a workgroup.
 struct PfStage {
-    static constexpr int kRows = 16 * RW, kTok = 16 * TW;
-    uint8_t b16[kTok * kPfBStride];
-    float xsum[8][kTok];        // [lane k][token]
-    float xsc[kTok];
-    uint32_t sch[8][kRows];     // [sub-block j][row] half2(sc_j, sc_j)
-    uint32_t scn[8][kRows];     // [sub-block j][row] half2(-1024 sc_j, -1024 sc_j)
-    float m[8][kRows];          // [lane k][row]
-    float d[kRows];
-    float dmin[kRows];
+    uint8_t b16[kPfTok * kPfBStride];
+    float xsum[8][kPfTok];        // [lane k][token]
+    float xsc[kPfTok];
+    uint32_t sch[8][kPfRows];     // [sub-block j][row] half2(sc_j, sc_j)
+    uint32_t scn[8][kPfRows];     // [sub-block j][row] half2(-1024 sc_j, -1024 sc_j)
+    float m[8][kPfRows];          // [lane k][row]
+    float d[kPfRows];
+    float dmin[kPfRows];
     // nibble dwords per row as [group s][lane k] (lane (g, c) of a wave reads
     // its 8 dwords as 32 contiguous bytes); 36-dword rows keep the 16 rows'
     // 16-byte reads on distinct banks
-    uint32_t wa[kRows][kPfWStride];
+    uint32_t wa[kPfRows][kPfWStride];
 };
 
 // four signed bytes -> two half2 words holding the same integers
@@ -114,86 +113,73 @@ struct PfArgs {
     int out_stride;
 };
 
-// Staging registers of one block for T = 64 RW TW threads, mapped so that
-// every LDS store of a wave hits distinct banks:
-//   q8: unit u = (token u/16, part u%16), units tid, tid + T, ...: q8 bytes
-//       8 part .. + 7 and 128 + 8 part .. + 7, written as f16 at 16 part and
-//       256 + 16 part of the token's row;
-//   threads 0 .. 2 kTok - 1 one xsum quad, threads 0 .. kTok - 1 one xscale;
-//   unit u = (sub-block j = u / kRows, row u % kRows): the row's block header
-//   and the 16 nibble bytes of lane k = j.
-template <int RW, int TW>
+// Staging registers of one block, mapped so that every LDS store of a wave hits
+// distinct banks:
+//   q8: thread = (token tid / 16, part tid % 16): q8 bytes 8 part .. + 7 and
+//       128 + 8 part .. + 7, written as f16 at 16 part and 256 + 16 part of the
+//       token's row;
+//   threads 0 .. 2 kPfTok - 1 one xsum quad, threads 0 .. kPfTok - 1 one xscale;
+//   unit u = (sub-block j = u / kPfRows, row u % kPfRows), units tid and tid +
+//   kPfThreads: the row's block header and the 16 nibble bytes of lane k = j.
 struct PfRegs {
-    static constexpr int T = 64 * RW * TW;
-    static constexpr int NQ = 16 * 16 * TW / T;  // q8 units per thread
-    static constexpr int NH = 8 * 16 * RW / T;   // header units per thread
-    uint32_t q[NQ][4];
+    static constexpr int NH = 8 * kPfRows / kPfThreads;  // header units per thread
+    uint32_t q[4];
     f4v xs;
     float xc;
     u4v h[NH];
     u4v w[NH];
 };
 
-template <int RW, int TW>
 __device__ __forceinline__ void pf_load(const PfArgs& a, int row0, int tok0, int b,
-                                        PfRegs<RW, TW>& r) {
-    using R = PfRegs<RW, TW>;
-    constexpr int kRows = 16 * RW, kTok = 16 * TW;
+                                        PfRegs& r) {
     const int tid = threadIdx.x;
     const int cols = a.blocks * 256;
-#pragma unroll
-    for (int i = 0; i < R::NQ; i++) {
-        const int u = tid + R::T * i;
-        const int t = min(tok0 + (u >> 4), a.p - 1);
-        const int8_t* src = a.act.q8perm + (size_t)t * cols + (size_t)b * 256 + 8 * (u & 15);
+    {
+        const int t = min(tok0 + (tid >> 4), a.p - 1);
+        const int8_t* src = a.act.q8perm + (size_t)t * cols + (size_t)b * 256 + 8 * (tid & 15);
         const uint2 lo = *(const uint2*)src, hi = *(const uint2*)(src + 128);
-        r.q[i][0] = lo.x; r.q[i][1] = lo.y; r.q[i][2] = hi.x; r.q[i][3] = hi.y;
+        r.q[0] = lo.x; r.q[1] = lo.y; r.q[2] = hi.x; r.q[3] = hi.y;
     }
-    if (tid < 2 * kTok) {
+    if (tid < 2 * kPfTok) {
         const int t = min(tok0 + (tid >> 1), a.p - 1);
         r.xs = *(const f4v*)(a.act.xs32 + (size_t)t * (cols / 32) + b * 8 + 4 * (tid & 1));
     }
-    if (tid < kTok) r.xc = a.act.xscale[(size_t)min(tok0 + tid, a.p - 1) * a.blocks + b];
+    if (tid < kPfTok) r.xc = a.act.xscale[(size_t)min(tok0 + tid, a.p - 1) * a.blocks + b];
 #pragma unroll
-    for (int i = 0; i < R::NH; i++) {
-        const int u = tid + R::T * i;
-        const int row = min(row0 + u % kRows, a.rows - 1);
+    for (int i = 0; i < PfRegs::NH; i++) {
+        const int u = tid + kPfThreads * i;
+        const int row = min(row0 + u % kPfRows, a.rows - 1);
         const uint8_t* rp = a.w + (size_t)row * a.rb;
         r.h[i] = *(const u4v*)(rp + q4k_hdr_off(b));
-        r.w[i] = *(const u4v*)(rp + q4k_nib_off(a.blocks, b) + 16 * (u / kRows));
+        r.w[i] = *(const u4v*)(rp + q4k_nib_off(a.blocks, b) + 16 * (u / kPfRows));
     }
 }
 
-template <int RW, int TW>
-__device__ __forceinline__ void pf_store(const PfRegs<RW, TW>& r, PfStage<RW, TW>& st) {
-    using R = PfRegs<RW, TW>;
-    constexpr int kRows = 16 * RW, kTok = 16 * TW;
+__device__ __forceinline__ void pf_store(const PfRegs& r, PfStage& st) {
     const int tid = threadIdx.x;
-#pragma unroll
-    for (int i = 0; i < R::NQ; i++) {
-        const int u = tid + R::T * i;
+    {
         uint32_t v[8];
-        i8x4_to_h(r.q[i][0], v[0], v[1]);
-        i8x4_to_h(r.q[i][1], v[2], v[3]);
-        i8x4_to_h(r.q[i][2], v[4], v[5]);
-        i8x4_to_h(r.q[i][3], v[6], v[7]);
-        uint8_t* row = st.b16 + (u >> 4) * kPfBStride + 16 * (u & 15);
+        i8x4_to_h(r.q[0], v[0], v[1]);
+        i8x4_to_h(r.q[1], v[2], v[3]);
+        i8x4_to_h(r.q[2], v[4], v[5]);
+        i8x4_to_h(r.q[3], v[6], v[7]);
+        uint8_t* row = st.b16 + (tid >> 4) * kPfBStride + 16 * (tid & 15);
         *(u4v*)row = u4v{v[0], v[1], v[2], v[3]};
         *(u4v*)(row + 256) = u4v{v[4], v[5], v[6], v[7]};
     }
-    if (tid < 2 * kTok) {
+    if (tid < 2 * kPfTok) {
         const int t = tid >> 1, k0 = 4 * (tid & 1);
         st.xsum[k0][t] = r.xs.x;
         st.xsum[k0 + 1][t] = r.xs.y;
         st.xsum[k0 + 2][t] = r.xs.z;
         st.xsum[k0 + 3][t] = r.xs.w;
     }
-    if (tid < kTok) st.xsc[tid] = r.xc;
+    if (tid < kPfTok) st.xsc[tid] = r.xc;
 #pragma unroll
-    for (int i = 0; i < R::NH; i++) {
+    for (int i = 0; i < PfRegs::NH; i++) {
         // getScaleMinK4 (simd.go:1672-1677) for sub-block j
-        const int u = tid + R::T * i;
-        const int row = u % kRows, j = u / kRows;
+        const int u = tid + kPfThreads * i;
+        const int row = u % kPfRows, j = u / kPfRows;
         const uint32_t s03 = r.h[i].y, s47 = r.h[i].z, s811 = r.h[i].w;
         uint32_t sc, mn;
         if (j < 4) {
@@ -222,20 +208,14 @@ __device__ __forceinline__ void pf_store(const PfRegs<RW, TW>& r, PfStage<RW, TW
     }
 }
 
-template <int RW, int TW>
-// (two waves per SIMD for multi-wave workgroups; a one-wave workgroup, one
-// per CU, may use the whole register file for its deeper staging)
-__global__ __launch_bounds__(64 * RW * TW) __attribute__((amdgpu_waves_per_eu(RW * TW > 1 ? 2 : 1)))
+__global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void prefill_q4k_mfma_kernel(PfArgs a) {
-    using Stage = PfStage<RW, TW>;
-    __shared__ __align__(16) Stage stage[2];
+    __shared__ __align__(16) PfStage stage[2];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int g = lane >> 4, c = lane & 15;
-    const int rw = wave % RW, tw = wave / RW;  // 16-row group, 16-token column
-    const int row0 = blockIdx.x * Stage::kRows, tok0 = blockIdx.y * Stage::kTok;
-    // D layout: rows 4g + i of the wave's 16, token c of its column
-    const int lr = 16 * rw + 4 * g;
-    const int lt = 16 * tw + c;
+    const int row0 = blockIdx.x * kPfRows, tok0 = blockIdx.y * kPfTok;
+    // D layout: rows 4g + i of the wave's 16, token c
+    const int lr = 16 * wave + 4 * g;
 
     float accF[4][8], accM[4][8];
 #pragma unroll
@@ -244,29 +224,29 @@ void prefill_q4k_mfma_kernel(PfArgs a) {
         for (int k = 0; k < 8; k++) accF[i][k] = accM[i][k] = 0.0f;
 
     // one block's products from a staged LDS tile
-    auto block = [&](const Stage& st) __attribute__((always_inline)) {
+    auto block = [&](const PfStage& st) __attribute__((always_inline)) {
         // this lane's A row (MFMA row c of the wave's 16): its 8 nibble dwords
-        const u4v wq0 = *(const u4v*)&st.wa[16 * rw + c][8 * g];
-        const u4v wq1 = *(const u4v*)&st.wa[16 * rw + c][8 * g + 4];
+        const u4v wq0 = *(const u4v*)&st.wa[16 * wave + c][8 * g];
+        const u4v wq1 = *(const u4v*)&st.wa[16 * wave + c][8 * g + 4];
         const uint32_t wq[8] = {wq0.x, wq0.y, wq0.z, wq0.w, wq1.x, wq1.y, wq1.z, wq1.w};
-        const uint32_t sh_lo = st.sch[2 * g][16 * rw + c], sn_lo = st.scn[2 * g][16 * rw + c];
-        const uint32_t sh_hi = st.sch[2 * g + 1][16 * rw + c], sn_hi = st.scn[2 * g + 1][16 * rw + c];
+        const uint32_t sh_lo = st.sch[2 * g][16 * wave + c], sn_lo = st.scn[2 * g][16 * wave + c];
+        const uint32_t sh_hi = st.sch[2 * g + 1][16 * wave + c], sn_hi = st.scn[2 * g + 1][16 * wave + c];
         // F chain factors d * xscale per D row
         const f4v dv = *(const f4v*)&st.d[lr];
         const f4v dm = *(const f4v*)&st.dmin[lr];
-        const float xc = st.xsc[lt];
+        const float xc = st.xsc[c];
         float dxs[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) dxs[i] = dv[i] * xc;
 #pragma unroll
         for (int k = 0; k < 8; k++) {
             const h8v av = dequant_a(wq[k], sh_lo, sn_lo, sh_hi, sn_hi);
-            const h8v bv = *(const h8v*)(st.b16 + lt * kPfBStride + 64 * k + 16 * g);
+            const h8v bv = *(const h8v*)(st.b16 + c * kPfBStride + 64 * k + 16 * g);
             const f4v z = {0.0f, 0.0f, 0.0f, 0.0f};
             const f4v dI = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bv, z, 0, 0, 0);
             // M chain operands: mins of the lane's 4 D rows, xsum of its token
             const f4v mk = *(const f4v*)&st.m[k][lr];
-            const float xk = st.xsum[k][lt];
+            const float xk = st.xsum[k][c];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 accF[i][k] = fmaf(dI[i], dxs[i], accF[i][k]);
@@ -282,7 +262,7 @@ void prefill_q4k_mfma_kernel(PfArgs a) {
     // under a branch the compiler's vmcnt wait for the older set would also
     // wait for the newer one and cancel the prefetch.
     const int nb = a.blocks;
-    PfRegs<RW, TW> r0, r1;
+    PfRegs r0, r1;
     pf_load(a, row0, tok0, 0, r0);
     pf_store(r0, stage[0]);
     pf_load(a, row0, tok0, min(1, nb - 1), r1);
@@ -300,7 +280,7 @@ void prefill_q4k_mfma_kernel(PfArgs a) {
         __syncthreads();
     }
     // tree8 of the reference's horizontal sum, then the (row, token) store
-    const int t = tok0 + lt;
+    const int t = tok0 + c;
     if (t < a.p) {
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -315,10 +295,9 @@ void prefill_q4k_mfma_kernel(PfArgs a) {
     }
 }
 
-template <int RW, int TW>
 static void launch_pf(const PfArgs& a, hipStream_t s) {
-    dim3 grid((a.rows + 16 * RW - 1) / (16 * RW), (a.p + 16 * TW - 1) / (16 * TW));
-    hipLaunchKernelGGL((prefill_q4k_mfma_kernel<RW, TW>), grid, dim3(64 * RW * TW), 0, s, a);
+    dim3 grid((a.rows + kPfRows - 1) / kPfRows, (a.p + kPfTok - 1) / kPfTok);
+    hipLaunchKernelGGL(prefill_q4k_mfma_kernel, grid, dim3(kPfThreads), 0, s, a);
 }
 
 // --- more than 16 activation rows: one pair of AVX2 lanes per wave ---------
@@ -1529,11 +1508,9 @@ int launch_small_lanes(bool q6, SmallJob j, hipStream_t s) {
     return GLLM_OK;
 }
 
-// Kernel choice for Q4_K from 8 rows on, after run_gemv's small batches
-// (launch_small_lanes): 64 x 64 tiles split by AVX2 lane above 16 rows, and 64
-// rows x 16 tokens (prefill_q4k_mfma_kernel) for batches without records, that
-// is past kSmallCols columns or 4 GiB of weight.  The other kernels address a
-// weight with 32-bit offsets.
+// Q4_K from 8 rows on, after run_gemv's small batches (launch_small_lanes): 64 x
+// 64 tiles split by AVX2 lane above 16 rows, which address a weight with 32-bit
+// offsets, and 64 rows x 16 tokens (prefill_q4k_mfma_kernel) below.
 int launch_q4k_mfma(const uint8_t* d_w, size_t rb, int rows, int blocks, const ActQ8& act, int p,
                     float* out, int out_stride, hipStream_t s) {
     if (rows <= 0 || blocks <= 0 || p <= 0) return GLLM_OK;
@@ -1544,9 +1521,7 @@ int launch_q4k_mfma(const uint8_t* d_w, size_t rb, int rows, int blocks, const A
             return fail(GLLM_EINVAL, "prefill: %d rows of %zu B need f16 tiles and < 4 GiB", rows, rb);
         GLLM_TRY(launch_q4k_lanes<false>(a, s));
     } else {
-        if ((rows + 63) / 64 < 2 * device_cus() / 3 && !fits)
-            return fail(GLLM_EINVAL, "prefill: weights of %zu B past 4 GiB", (size_t)rows * rb);
-        launch_pf<4, 1>(a, s);
+        launch_pf(a, s);  // 64-bit offsets
     }
     GLLM_HIP(hipGetLastError());
     return GLLM_OK;

@@ -161,6 +161,39 @@ def test_small_batch_routes(hip, rows, cols, p):
     assert_bits(w.matvec_batch(xs), amd64(data, xs, rows, cols), f"{rows}x{cols} p={p}")
 
 
+@pytest.mark.parametrize("p", [5, 8, 11, 16])
+def test_small_batch_past_the_records(hip, p):
+    """65792 columns carry no records: the row kernels and the 64 x 16 tiles,
+    257 blocks, one row past a tile."""
+    rows, cols = 65, 65792
+    data, _ = quant_matrix(ref.Q4_K, rows, cols, 980)
+    w = hip.Weight.from_host(data, ref.Q4_K, rows, cols)
+    xs = normal(981 + p, (p, cols))
+    assert_bits(w.matvec_batch(xs), amd64(data, xs, rows, cols), f"{rows}x{cols} p={p}")
+
+
+def test_small_batch_few_rows_past_4_gib(hip):
+    """8192 rows of 512 KB: a weight of 4 GiB with too few rows for the 64 x 16
+    tiles to cover the GPU still runs on them."""
+    import torch
+    rows, cols, p = 32, 256 * 3641, 9
+    data, _ = quant_matrix(ref.Q4_K, rows, cols, 982)
+    times = 8192 // rows
+    raw = torch.from_numpy(data).cuda().repeat(times)
+    assert raw.numel() > 1 << 32
+    w = hip.Weight.from_device(raw, ref.Q4_K, 8192, cols)
+    del raw
+    xs = normal(983, (p, cols))
+    out = torch.full((p, 8192), -1.0, device="cuda")
+    print(f"8192 x {cols}, {p} tokens", flush=True)
+    w.matvec_dev(torch.from_numpy(xs).cuda(), out)
+    torch.cuda.synchronize()
+    want = torch.from_numpy(amd64(data, xs, rows, cols)).cuda()
+    assert (out.view(torch.int32).view(p, times, rows) == want.view(torch.int32)[:, None]).all()
+    del w
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("qtype,p", [(ref.Q8_0, 17), (ref.Q6_K, 17), (ref.Q5_K, 17), (ref.Q4_0, 17), (ref.Q4_K, 9)])
 def test_group_with_a_weight_past_4_gib(hip, qtype, p):
     """The kernels with 32-bit offsets look at every weight of a group: 64 rows
