@@ -25,7 +25,7 @@
 
 namespace gllm {
 int gemv_f32(int n, gllm_hip_weight* const* ws, const float* d_xs, int p, float* const* outs,
-             const int* strides, void* act_buf, hipStream_t s);
+             const int* strides, void* act_buf, hipStream_t s, size_t act_cap = SIZE_MAX);
 int gemv_group(int n, gllm_hip_weight* const* ws, const float* d_x, float* const* outs,
                const int* strides, void* act_buf, hipStream_t s);
 int group_routing(int n, gllm_hip_weight* const* ws, int* fl);

@@ -2203,12 +2203,12 @@ static bool lanes_fit(int n, gllm_hip_weight* const* ws, const ActQ8& act, int p
 //   8 tokens: 14336 x 4096 19.0 / 21.7, 28672 x 4096 33.7 / 31.4, x 8192 51.9 / 52.6,
 //     57344 x 14336 (no cache holds it) 188 / 177
 //   9 to 16: 8192 x 4096 14.9 / 25.7, 14336 x 4096 24.8 / 22.0, x 14336 54.1 / 57.8,
-//     28672 x 14336 90.8 / 82.8
+//     28672 x 14336 90.8 / 82.8, 11000 x 66048 (408 MB) 274 / 250
 //   Q6_K at 4: 512 x 14336 26.3 / 24.7, 1024 x 8192 17.8 / 17.3, 4096 x 4096 12.2 /
 //     15.8; at 3 14336 x 4096 23.8 / 21.2
 static bool small_batch_fits(int n, gllm_hip_weight* const* ws, int p) {
     const gllm_hip_weight* w0 = ws[0];
-    if (p < 2 || p > kTiledMinP || w0->cols > kSmallCols) return false;
+    if (p < 2 || p > kTiledMinP) return false;
     int total = 0, fewest = w0->rows;
     size_t bytes = 0;
     for (int i = 0; i < n; i++) {
@@ -2229,9 +2229,10 @@ static bool small_batch_fits(int n, gllm_hip_weight* const* ws, int p) {
         if (p == 2) return total < (blocks < 56 ? 24576 : 49152);
         return blocks >= 56 || total < 49152;
     }
-    if (p == 8) return n > 1 || total < 20480 || (blocks > 20 && bytes < ((size_t)300 << 20));
+    const bool cached = bytes < ((size_t)300 << 20);
+    if (p == 8) return n > 1 || total < 20480 || (blocks > 20 && cached);
     // the 64-row tiles of every weight cover two thirds of the CUs
-    return (fewest + 63) / 64 < 2 * device_cus() / 3 || (blocks >= 56 && fewest < 20480);
+    return (fewest + 63) / 64 < 2 * device_cus() / 3 || (blocks >= 56 && fewest < 20480 && cached);
 }
 
 int run_gemv(int n, gllm_hip_weight* const* ws, const ActQ8& act, int p, float* const* outs,
@@ -2337,12 +2338,13 @@ bool fused_quant(int n, gllm_hip_weight* const* ws) {
 // consecutive weights of one type is one row-kernel launch (the run's
 // kernel quantises x itself at batch 1 when its shape allows), and every run
 // that reads pre-quantised activations shares one q8kQuantize + xsums into
-// `act` (act_bytes(cols, p) bytes of device scratch).  Runs of different
+// `act` (act_bytes(cols, p) bytes of device scratch, or act_cap < act_bytes
+// that hold act_plain_bytes: no records then).  Runs of different
 // types are what the reference's mixed groups compute: one int8 row dot per
 // projection (tryMatvecAttentionInto, model.go:3156-3190;
 // matvecBatchQ8Fused, kernels_portable_tunables.go:304-408).
 int gemv_f32(int n, gllm_hip_weight* const* ws, const float* d_xs, int p, float* const* outs,
-             const int* strides, void* act_buf, hipStream_t s) {
+             const int* strides, void* act_buf, hipStream_t s, size_t act_cap = SIZE_MAX) {
     const int cols = ws[0]->cols;
     ActQ8 act{};
     bool quantised = false;
@@ -2363,7 +2365,7 @@ int gemv_f32(int n, gllm_hip_weight* const* ws, const float* d_xs, int p, float*
                     for (b = a + 1; b < n && ws[b]->type == ws[a]->type;) b++;
                     records = records || small_batch_fits(b - a, ws + a, p);
                 }
-                if (!records) act.rec = nullptr;
+                if (!records || act_bytes(cols, p) > act_cap) act.rec = nullptr;
                 GLLM_TRY(launch_q8k_prep(d_xs, cols, p, act, s));
                 quantised = true;
             }

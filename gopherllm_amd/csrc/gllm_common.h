@@ -66,14 +66,13 @@ struct ActQ8 {
     uint16_t* b16t;
     float* xs32t;    // xs32 of the same batches as [block][tile][lane k][token c]
     int tiles;       // ceil(p / 16) when b16t is set
-    // Batches of 2 .. kTiledMinP rows of up to kSmallCols columns carry what
-    // one wave of the small-batch kernels reads of a block as one record of
-    // small_rec(p) bytes instead, [block][lane pair k, k + 4]; see SmallRec.
+    // Batches of 2 .. kTiledMinP rows carry what one wave of the small-batch
+    // kernel reads of a block as one record of small_rec(small_pt(p)) bytes
+    // instead, [block][lane pair k, k + 4].  Null where nothing reads them.
     uint8_t* rec;
     int cols, p;
 };
 constexpr int kTiledMinP = 16;
-constexpr int kSmallCols = 65536;  // keeps act_bytes of the small batches under 4 MiB
 __host__ __device__ __forceinline__ int small_pt(int p) { return p <= 8 ? 8 : 16; }
 // A record for pt (8 or 16) tokens, zero past p, q8 as f16 in b16t's order:
 //   f16 b16[2 lanes][4 groups g][pt][8]; f32 xs32[2 lanes][pt]; f32 xscale[pt];
@@ -85,6 +84,7 @@ __host__ __device__ __forceinline__ int b16_slot(int kappa) {
     return (kappa & 4) | ((kappa & 1) << 1) | ((kappa >> 1) & 1);
 }
 size_t act_bytes(int cols, int p);
+size_t act_plain_bytes(int cols, int p);  // without the records
 void act_carve(void* base, int cols, int p, ActQ8* a);
 int launch_q8k_prep(const float* d_x, int cols, int p, const ActQ8& a, hipStream_t s);
 // Batched Q4_K x Q8_K on the matrix cores (bit-identical to the row kernel):

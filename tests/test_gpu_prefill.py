@@ -162,9 +162,8 @@ def test_small_batch_routes(hip, rows, cols, p):
 
 
 @pytest.mark.parametrize("p", [5, 8, 11, 16])
-def test_small_batch_past_the_records(hip, p):
-    """65792 columns carry no records: the row kernels and the 64 x 16 tiles,
-    257 blocks, one row past a tile."""
+def test_small_batch_wide_rows(hip, p):
+    """257 blocks and one row past the row tiles, both token widths."""
     rows, cols = 65, 65792
     data, _ = quant_matrix(ref.Q4_K, rows, cols, 980)
     w = hip.Weight.from_host(data, ref.Q4_K, rows, cols)

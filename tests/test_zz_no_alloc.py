@@ -69,6 +69,25 @@ def test_noalloc_refuses_beyond_its_maximum(hip):
     assert (out.cpu().numpy() == 7.0).all()
 
 
+@pytest.mark.parametrize("cols,p", [(70144, 16), (180224, 9), (376832, 8), (1000192, 2)])
+def test_noalloc_wide_rows(hip, cols, p):
+    """Activations near 4 MiB, with the small-batch records beside them and, for
+    two rows of a million columns, without room for the records."""
+    import torch
+    L = hip._lib.load()
+    rows = 20
+    data, _ = quant_matrix(ref.Q4_K, rows, cols, 940)
+    w = hip.Weight.from_host(data, hip.TYPE_Q4_K, rows, cols)
+    assert hip.act_bytes(cols, p) > 4 << 20
+    x = torch.from_numpy(normal(941, (p, cols))).cuda()
+    a, b = (torch.full((p, rows), v, device="cuda") for v in (-1.0, -2.0))
+    print(f"noalloc {rows}x{cols} p={p}", flush=True)
+    assert _call(L, "gllm_hip_matvec_dev", w, x, p, a, rows) == 0, hip._lib.last_error()
+    assert _call(L, "gllm_hip_matvec_dev_noalloc", w, x, p, b, rows) == 0, hip._lib.last_error()
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(b.cpu().numpy()), bits(a.cpu().numpy()))
+
+
 def test_noalloc_captured_on_a_fresh_stream(hip):
     """The call needs no earlier call on its stream before capture (it takes
     no scratch from the stream's pool): capture it on a new stream, replay
