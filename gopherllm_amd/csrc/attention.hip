@@ -1457,7 +1457,7 @@ static bool prefill_path(const gllm_hip_kv* kv, int p, int kvmul, int hd, int sp
 // Device floats that attend_exact works in for at most p tokens over spans of
 // at most span_max.
 size_t attend_exact_floats(const gllm_hip_kv* kv, int p, int n_heads, int n_kv, int hd, int span_max) {
-    const bool tiles = attend_prefill_fits(hd, kv->kv_dim_k, kv->kv_dim_v);
+    const bool tiles = p > 1 && attend_prefill_fits(hd, kv->kv_dim_k, kv->kv_dim_v);
     const size_t rows = tiles ? std::min(p, 15) : p;  // tokens that may take the other kernels
     const size_t n = rows * n_heads * (span_max + 1) + (size_t)n_heads * ((span_max + 31) / 32) + 64;
     return tiles ? std::max(n, attend_prefill_floats(p, n_heads, n_kv, span_max)) : n;

@@ -362,12 +362,29 @@ def test_prompt_longer_than_one_prefill_chunk(hip):
         assert np.array_equal(v, c2.vcache(l, max_len)[:used]), l
 
 
+def test_new_decoder_has_no_prompt_scores(hip):
+    """A decoder that has seen no prompt keeps one token's scores, n_heads x
+    max_len floats, not the 16 query rows per kv head of a prompt tile."""
+    import torch
+    from gopherllm_amd.decoder import LlamaDecoder
+    heads, hd, max_len = 16, 64, 65536
+    m = tiny_llama(seed=17, n_layers=1, dim=256, hidden=512, n_heads=heads, n_kv_heads=heads, head_dim=hd, vocab=1200)
+    torch.cuda.synchronize()
+    LlamaDecoder.from_host_model(m, 64)  # the library's own first allocations
+    before = torch.cuda.mem_get_info()[0]
+    gpu = LlamaDecoder.from_host_model(m, max_len)
+    used = before - torch.cuda.mem_get_info()[0]
+    kv, rope, scores = 2 * max_len * heads * hd * 2, 2 * max_len * hd // 2 * 4, heads * max_len * 4
+    print(f"{used >> 20} MiB, of them {(kv + rope + scores) >> 20} of cache, RoPE rows and scores", flush=True)
+    assert used < kv + rope + scores + (32 << 20)
+    del gpu
+
+
 def test_prefill_crossing_position_6144(hip):
     """A 300-token prefill at positions 6000..6299 over a cache whose rows
     0..5999 hold the same random f16 K/V on both sides: its later tokens span
-    more than 6144 positions, where prefill attention takes the generic
-    scores / softmax / values kernels (in the model's scores buffer).  The
-    logits, the token, the new KV rows and 4 decode steps after it equal the
+    more than 6144 positions (the prompt attention at head_dim 64, in the
+    model's scores buffer).  The logits, the token, the new KV rows and 4 decode steps after it equal the
     oracle's."""
     from gopherllm_amd.decoder import LlamaDecoder
     m = tiny_llama(seed=15, n_layers=1, dim=256, hidden=512, n_heads=4, n_kv_heads=1, head_dim=64,
@@ -404,8 +421,8 @@ def test_prefill_crossing_position_6144(hip):
 def test_prefill_mixed_types_take_the_batched_tiles(hip):
     """Q4_K_M-style mix at widths whose rows hold a multiple of 8 blocks
     (dim 2048, hidden 4096): the prefill's Q6_K attn_v / ffn_down run the
-    matrix-core tiles and a Q8_0 ffn_down the vector-unit tiles (prompt of
-    90 tokens: ragged 64-token tiles), then greedy steps; logits, hidden
+    matrix-core tiles and so does a Q8_0 ffn_down (prompt of 90 tokens:
+    ragged 64-token tiles), then greedy steps; logits, hidden
     states and tokens equal the oracle's."""
     from gopherllm_amd.decoder import LlamaDecoder
 
