@@ -1470,10 +1470,11 @@ bool attend_exact_graphable(const gllm_hip_kv* kv, int n_heads, int n_kv, int hd
            span_cap <= kSmaxSpan1;
 }
 
-// scratch: attend_exact_floats(p, ...) floats of device memory, or null for
-// the calling thread's scratch.  d_end (with p == 1): the end position is read
-// on the device and span_cap bounds the span, so the launches do not depend
-// on the position (a captured decode step replays for every position).
+// scratch: attend_exact_floats(p, ...) floats of device memory, or, for one
+// token, null for the calling thread's scratch.  d_end (with p == 1): the end
+// position is read on the device and span_cap bounds the span, so the launches
+// do not depend on the position (a captured decode step replays for every
+// position).
 int attend_exact(const gllm_hip_kv* kv, int l, const float* d_q, int n_heads, int n_kv, int hd,
                  int start, int end0, int p, float scale, float* d_out, hipStream_t s,
                  float* scratch, const int* d_end, int span_cap, const float* rope_sin,
@@ -1492,11 +1493,9 @@ int attend_exact(const gllm_hip_kv* kv, int l, const float* d_q, int n_heads, in
         return fail(GLLM_EINVAL, "attend: RoPE folding needs one token and its raw k / v rows");
     const AttnRope rope{rope_sin, rope_cos, d_knew, d_vnew, kv->k[l], kv->v[l], rope_cur};
     if (prefill_path(kv, p, kvmul, hd, span_max)) {
-        float* sc = scratch ? scratch
-                            : (float*)thread_scratch(5, attend_prefill_floats(p, n_heads, n_kv, span_max) * 4, s);
-        if (!sc) return scratch_error();
+        if (!scratch) return fail(GLLM_EINVAL, "attend: several tokens work in the caller's scratch");
         return attend_prefill(d_q, kv->k[l] + (size_t)start * kv->kv_dim_k, kv->v[l] + (size_t)start * kv->kv_dim_v,
-                              kv->kv_dim_k, n_heads, n_kv, hd, span0, p, scale, sc, d_out, s);
+                              kv->kv_dim_k, n_heads, n_kv, hd, span0, p, scale, scratch, d_out, s);
     }
     if (hd == kFusedHD && kvmul <= 4 && kv->kv_dim_k == kv->kv_dim_v &&
         span_max <= (p == 1 ? kSmaxSpan1 : kSmaxSpan)) {

@@ -6,8 +6,8 @@
 // maximum; fastExpF32; the denominator and every output element summed in
 // position order.  Each of these chains is a K loop of a float32 matrix
 // product, and v_mfma_f32_16x16x4 evaluates exactly such a chain: four fmas
-// in the order k = 0 .. 3, each rounded (denormals, infinities and zero signs
-// included), so whole 16 x 16 tiles of scores and outputs run on the matrix
+// in the order k = 0 .. 3, each rounded (subnormals, infinities and zero signs
+// included; the probe library's test compares them), so whole 16 x 16 tiles of scores and outputs run on the matrix
 // cores with the reference's bits.  Per kv head the query rows of a chunk are
 // numbered R = token * kvmul + head; a query tile is 16 of them, so one pass
 // over K and V serves 16 rows where a workgroup per (head, token) read them
@@ -30,10 +30,11 @@
 //
 // A 512-token prompt through two 8B-shaped layers at positions 0 / 3500 went
 // from 2433 / 7434 us to 1885 / 2872 us; in a 3000-token prompt the scores and
-// values launches take 82 and 154 us on average.  The scores launch runs at
-// half the f32 matrix rate; the values launch is bound by the exponentials
-// (about 30 VALU operations each, which the f32 MFMA does not overlap) and
-// the products together.
+// values launches take 81 and 153 us on average.  No cycle of an f32 MFMA runs
+// under VALU work here (the coexecution counter stays at 0), so the two add up:
+// 57 percent of the SIMDs' busy cycles MFMA and 32 VALU in the scores launch, 30
+// and 35 in the values launch, whose waves also wait for one another at each
+// step's barrier.
 #include <algorithm>
 
 #include "attn_exp.h"

@@ -328,10 +328,10 @@ static void launch_pf(const PfArgs& a, hipStream_t s) {
 // and ran all eight lanes of a 16 x 32 tile in a wave (two waves per SIMD,
 // LDS traffic 370 KB per block), 195 us with eight waves of 32 rows x 64
 // tokens (two per SIMD), 202 us with eight waves of 16 rows x 128 tokens, 175
-// us like this.  What is left is issue: per wave and block 64 chain steps, 40
-// VALU operations of dequantisation and 11 matrix instructions, which hardly
-// overlap the VALU on this part (a 16x16x32 f16 MFMA and four fmas take 30
-// cycles at four waves per SIMD, the MFMA alone 20).
+// us like this.  What is left is issue: per wave and block 128 VALU instructions,
+// 64 of them chain steps, and 11 matrix instructions of 16 (f16) and 32 cycles
+// (f32); by the counters the SIMDs' busy cycles are 61 percent VALU and 26
+// percent MFMA, a quarter of the latter under VALU work.
 // Up to kHalfTok tokens the products and chains run on two of the four token
 // tiles only (NT = 2).  17 tokens, four / two tiles: 4096 x 14336 Q4_K 78 / 64 us,
 // Q5_K 91 / 77, Q6_K 120 / 96, Q8_0 138 / 86.  As a branch inside one kernel it
@@ -697,8 +697,9 @@ int launch_q5k_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const 
 // With the quantiser launch, 4096 x 14336 x 333 (1.5 rounds of workgroups) and
 // 14336 x 4096 x 512: 473 and 490 us for 64 x 64 tiles that ran all eight
 // lanes in a wave and built the A operands twice, 245 and 260 us like this.
-// Bound by issue: per wave and block 96 chain steps, about 70 operations of
-// dequantisation and 21 matrix instructions.
+// Bound by issue: of the SIMDs' busy cycles 64 percent VALU (190 instructions per
+// wave and block, 96 of them chain steps) and 35 percent MFMA (21), a fifth of
+// the latter under VALU work.
 struct Q6Raw {
     uint8_t q[64][16];   // [16 part + row c]: lane kp's ql, lane kp + 4's ql, the 16 bytes with their qh
     uint8_t sc[16][16];  // [row c]
@@ -923,6 +924,8 @@ int launch_q6k_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const 
 // instruction each.
 // With the quantiser launch, 14336 x 4096 x 512: 718 us for 64 x 64 tiles on
 // the vector units (25 VALU operations per lane product), 305 us like this.
+// Bound by the VALU, 93 percent of the SIMDs' busy cycles; two thirds of the
+// matrix instructions' cycles run under it.
 struct Q80Raw {
     uint8_t q[64][16];  // [32 (k / 4) + 16 half + row c]
     uint8_t d[16][16];  // [row c]: eight f16 scales
@@ -1249,9 +1252,10 @@ int launch_q4_0_tiled(const uint8_t* d_w, size_t rb, int rows, int blocks, const
 // activations (small_rec: f16 operands and sums).  No wave waits for another
 // before the final tree, so there is no barrier in the loop.
 // KP: four waves take 16-byte pieces of each 128-byte weight line at
-// different times; with many rows that is what bounds the launch (the L1 does
-// not hold the lines between them), so two pairs per wave are faster there,
-// and one pair per wave where rows are few and waves scarce.
+// different times, two waves of two pairs each fetch it less often: at 14336 x
+// 4096 and 8 tokens a launch makes 745 thousand L2 reads in 14.4 us, with one pair
+// per wave 857 thousand in 16.0 us.  Where rows are few and waves scarce one
+// pair per wave is faster.
 // Up to 8 tokens (PT = 8) both lanes share one MFMA tile: D rows 0-7 hold lane
 // kp's eight tokens and rows 8-15 lane kp + 4's, two MFMAs accumulating into
 // it with the other lane's A rows zero (read from a zeroed LDS row; every sum

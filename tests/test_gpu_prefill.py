@@ -370,8 +370,8 @@ def test_prefill_q6k_configs2_shapes(hip, rows, cols):
 @pytest.mark.parametrize("rows,cols,p", [(300, 1024, 17), (64, 256, 100), (1000, 4096, 64),
                                          (70, 14336, 40), (130, 2048, 33)])
 def test_prefill_q8_0_bit_exact_small(hip, rows, cols, p):
-    """Q8_0 batches of more than 16 tokens (64 x 64 tiles on the vector
-    units): ragged row and token tiles against the amd64-order oracle."""
+    """Q8_0 batches of more than 16 tokens: ragged row and token tiles against
+    the amd64-order oracle."""
     data, _ = quant_matrix(ref.Q8_0, rows, cols, 700 + p + rows)
     w = hip.Weight.from_host(data, ref.Q8_0, rows, cols)
     xs = normal(701 + p, (p, cols))
