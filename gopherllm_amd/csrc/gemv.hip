@@ -2762,7 +2762,8 @@ int gllm_hip_matvec_q8_dev(gllm_hip_weight* w, const void* d_act, int p, float* 
     return run_gemv(1, ws, act, p, outs, strides, (hipStream_t)stream, nullptr);
 }
 
-// Host-pointer forms: stage through pinned memory on the thread's stream.
+// Host-pointer forms: copies from and to the caller's memory on the thread's
+// stream, which is waited for before the return.
 static int matvec_host(int n, gllm_hip_weight* const* ws, const float* x, int p, float* const* outs) {
     for (int i = 0; i < n; i++) GLLM_TRY(validate_weight(ws[i]));
     if (!x || p <= 0) return fail(GLLM_EINVAL, "matvec: bad input");

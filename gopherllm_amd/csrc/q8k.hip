@@ -64,14 +64,18 @@ void act_carve(void* base, int cols, int p, ActQ8* a) {
 // plain == true writes q8 in element order (the debug entry point) instead of
 // the lane-permuted order.  With `up` set, the activation is
 // siluMulF32(x, up) (the FFN's SwiGLU), evaluated here instead of in a launch
-// of its own.
+// of its own.  KIND: an instance for each batch class, so that none pays for
+// what the others write (512 rows of 14336 at 21.9 us, 23.2 with one kernel for
+// all).
+enum { kPrepRows, kPrepTiles, kPrepRecords };  // q8perm and sums alone, with b16t / xs32t, with rec
+template <int KIND>
 __global__ __launch_bounds__(256) void q8k_prep_kernel(const float* __restrict__ x, int cols,
                                                        ActQ8 a, int8_t* __restrict__ plain_q8,
                                                        float* __restrict__ plain_scale,
                                                        const float* __restrict__ up) {
     const int b = blockIdx.x, t = blockIdx.y, e = threadIdx.x;
     const int nb = cols / 256;
-    if (a.b16t && t >= a.p) {  // padding tokens of the last f16 tile (uniform per workgroup)
+    if (KIND == kPrepTiles && t >= a.p) {  // padding tokens of the last f16 tile (uniform per workgroup)
         const int kappa = q8perm_offset(e);
         a.b16t[((size_t)b * a.tiles + (t >> 4)) * 4096 + ((kappa >> 3) * 16 + (t & 15)) * 8 +
                b16_slot(kappa)] = 0;
@@ -79,7 +83,7 @@ __global__ __launch_bounds__(256) void q8k_prep_kernel(const float* __restrict__
         return;
     }
     const int pt = small_pt(a.p);
-    if (a.rec && t >= a.p) {  // padding tokens of the records (uniform per workgroup)
+    if (KIND == kPrepRecords && t >= a.p) {  // padding tokens of the records (uniform per workgroup)
         const int kappa = q8perm_offset(e), k = kappa >> 5;
         uint8_t* r = a.rec + ((size_t)b * 4 + (k & 3)) * small_rec(pt);
         ((uint16_t*)r)[(((k >> 2) * 4 + ((kappa >> 3) & 3)) * pt + t) * 8 + b16_slot(kappa)] = 0;
@@ -113,7 +117,7 @@ __global__ __launch_bounds__(256) void q8k_prep_kernel(const float* __restrict__
     }
     const int kappa = q8perm_offset(e);
     a.q8perm[(size_t)t * cols + (size_t)b * 256 + kappa] = (int8_t)q;
-    if (a.b16t) {
+    if constexpr (KIND == kPrepTiles) {
         // kappa = 32 k + 8 g + i -> ((k 4 + g) 16 + c) 8 + b16_slot(i) of the tile block
         a.b16t[((size_t)b * a.tiles + (t >> 4)) * 4096 + ((kappa >> 3) * 16 + (t & 15)) * 8 +
                b16_slot(kappa)] = __builtin_bit_cast(uint16_t, (_Float16)(float)q);
@@ -122,7 +126,7 @@ __global__ __launch_bounds__(256) void q8k_prep_kernel(const float* __restrict__
     auto rec_f = [&](int k, int row) -> float& {
         return ((float*)(a.rec + ((size_t)b * 4 + k) * small_rec(pt) + pt * 128))[row * pt + t];
     };
-    if (a.rec) {
+    if constexpr (KIND == kPrepRecords) {
         const int k = kappa >> 5;
         uint8_t* r = a.rec + ((size_t)b * 4 + (k & 3)) * small_rec(pt);
         ((uint16_t*)r)[(((k >> 2) * 4 + ((kappa >> 3) & 3)) * pt + t) * 8 + b16_slot(kappa)] =
@@ -139,8 +143,8 @@ __global__ __launch_bounds__(256) void q8k_prep_kernel(const float* __restrict__
         const float a0 = s[0] + s[4], a1 = s[1] + s[5], a2 = s[2] + s[6], a3 = s[3] + s[7];
         const float xs = (a0 + a1) + (a2 + a3);
         a.xs32[(size_t)t * (cols / 32) + b * 8 + e] = xs;
-        if (a.xs32t) a.xs32t[(((size_t)b * a.tiles + (t >> 4)) * 8 + e) * 16 + (t & 15)] = xs;
-        if (a.rec) rec_f(e & 3, e >> 2) = xs;
+        if constexpr (KIND == kPrepTiles) a.xs32t[(((size_t)b * a.tiles + (t >> 4)) * 8 + e) * 16 + (t & 15)] = xs;
+        if constexpr (KIND == kPrepRecords) rec_f(e & 3, e >> 2) = xs;
     } else if (e >= 64 && e < 80) {
         // sumF32Groups16: v_k = x[k] + x[8+k], then the same tree, then x32
         const int gi = e - 64;
@@ -151,27 +155,28 @@ __global__ __launch_bounds__(256) void q8k_prep_kernel(const float* __restrict__
         const float a0 = s[0] + s[4], a1 = s[1] + s[5], a2 = s[2] + s[6], a3 = s[3] + s[7];
         const float xs = (a0 + a1) + (a2 + a3);
         a.xs16[(size_t)t * (cols / 16) + b * 16 + gi] = xs;
-        if (a.rec) rec_f(gi & 3, 3 + (gi >> 2)) = xs;
+        if constexpr (KIND == kPrepRecords) rec_f(gi & 3, 3 + (gi >> 2)) = xs;
     }
 }
 
-int launch_q8k_prep(const float* d_x, int cols, int p, const ActQ8& a, hipStream_t s) {
+static int launch_prep(const float* d_x, const float* d_up, int cols, int p, const ActQ8& a, hipStream_t s) {
     if (cols <= 0 || cols % 256 || p <= 0) return fail(GLLM_EINVAL, "q8k: cols %d p %d", cols, p);
+    const auto kern = a.b16t  ? q8k_prep_kernel<kPrepTiles>
+                      : a.rec ? q8k_prep_kernel<kPrepRecords>
+                              : q8k_prep_kernel<kPrepRows>;
     dim3 grid(cols / 256, a.b16t ? 16 * a.tiles : a.rec ? small_pt(p) : p);
-    hipLaunchKernelGGL(q8k_prep_kernel, grid, dim3(256), 0, s, d_x, cols, a, (int8_t*)nullptr,
-                       (float*)nullptr, (const float*)nullptr);
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, d_x, cols, a, (int8_t*)nullptr, (float*)nullptr, d_up);
     GLLM_HIP(hipGetLastError());
     return GLLM_OK;
+}
+
+int launch_q8k_prep(const float* d_x, int cols, int p, const ActQ8& a, hipStream_t s) {
+    return launch_prep(d_x, nullptr, cols, p, a, s);
 }
 
 int launch_q8k_prep_silu(const float* d_gate, const float* d_up, int cols, int p, const ActQ8& a,
                          hipStream_t s) {
-    if (cols <= 0 || cols % 256 || p <= 0) return fail(GLLM_EINVAL, "q8k: cols %d p %d", cols, p);
-    dim3 grid(cols / 256, a.b16t ? 16 * a.tiles : a.rec ? small_pt(p) : p);
-    hipLaunchKernelGGL(q8k_prep_kernel, grid, dim3(256), 0, s, d_gate, cols, a, (int8_t*)nullptr,
-                       (float*)nullptr, d_up);
-    GLLM_HIP(hipGetLastError());
-    return GLLM_OK;
+    return launch_prep(d_gate, d_up, cols, p, a, s);
 }
 
 }  // namespace gllm
@@ -184,7 +189,7 @@ extern "C" int gllm_hip_q8k_quantize_dev(const float* d_x, int cols, int p, int8
         return fail(GLLM_EINVAL, "gllm_hip_q8k_quantize_dev: bad arguments");
     ActQ8 a{};
     dim3 grid(cols / 256, p);
-    hipLaunchKernelGGL(q8k_prep_kernel, grid, dim3(256), 0, (hipStream_t)stream, d_x, cols, a,
+    hipLaunchKernelGGL(q8k_prep_kernel<kPrepRows>, grid, dim3(256), 0, (hipStream_t)stream, d_x, cols, a,
                        d_q8, d_scales, (const float*)nullptr);
     GLLM_HIP(hipGetLastError());
     return GLLM_OK;
