@@ -48,7 +48,7 @@ struct GemvJob {
     int blocks;
     int cols;
     size_t rb;
-    ActQ8 act;        // pre-quantised activations (unfused kernels)
+    RowAct act;       // pre-quantised activations (unfused kernels)
     const float* xf;  // f32 activations when the kernel quantises them itself
     int rows_per_wg;  // rows per workgroup: blockDim.x / (8 * G)
     int tok0;         // first activation row of this launch
@@ -65,7 +65,7 @@ struct GemvJob {
     // 256-row blocks in sq_cnt; the last of a block's 2 * 256 / rows_per_wg
     // workgroups quantises siluMulF32(out[0], out[1]) of the block into sq_act
     int* sq_cnt;
-    ActQ8 sq_act;
+    RowAct sq_act;
     // greedy argmax epilogue (batch-1 Q6_K, one weight): keys[gridDim.x]
     // and the repeat-penalty window
     ArgmaxOut am;
@@ -2168,7 +2168,7 @@ struct NormIn {
     float* xout;
     float eps;
     int* sq_cnt;
-    ActQ8 sq_act;
+    RowAct sq_act;
 };
 
 // The matrix-core kernels of more than kTiledMinP rows apply to every weight of
@@ -2428,7 +2428,7 @@ bool norm_fusable(int n, gllm_hip_weight* const* ws) {
 int gemv_norm_f32(int n, gllm_hip_weight* const* ws, const float* x, const float* res,
                   const float* nw, float eps, float* xout, float* const* outs, hipStream_t s) {
     if (!norm_fusable(n, ws)) return fail(GLLM_EUNSUP, "gemv: no RMSNorm prologue for this group");
-    const NormIn ni{nw, res, xout, eps, nullptr, ActQ8{}};
+    const NormIn ni{nw, res, xout, eps, nullptr, RowAct{}};
     ActQ8 none{};
     return run_gemv(n, ws, none, 1, outs, nullptr, s, x, &ni);
 }

@@ -51,12 +51,15 @@ int self_check();
 // Per-thread pinned host staging buffer.
 void* thread_pinned(int slot, size_t bytes);
 
-// Activation buffers produced by the Q8K quantiser for p rows of cols floats.
-struct ActQ8 {
+// Activation buffers produced by the Q8K quantiser for p rows of cols floats:
+// what the row kernels read (and carry in their arguments).
+struct RowAct {
     int8_t* q8perm;  // [p][cols] lane-permuted int8 (see q8perm_offset)
     float* xscale;   // [p][cols/256]
     float* xs32;     // [p][cols/32]   per-32 sums (amd64 order)
     float* xs16;     // [p][cols/16]   per-16 sums (amd64 order; Q6_K scales them by 32)
+};
+struct ActQ8 : RowAct {
     // Batches of more than kTiledMinP rows also get the q8 values as f16 in
     // the matrix-core operand layout of the batched kernels:
     // [block][16-token tile][lane k][group g][token c][8 halves], the eight
@@ -411,11 +414,10 @@ __device__ __forceinline__ float silu_mul(float g, float up) {
 // wmax: 4 floats of LDS).  SYS: read gate / up with system-scope loads
 // (written by other workgroups of the same launch).
 template <bool SYS = false>
-__device__ inline void silu_q8_block(const float* gate, const float* up, int b, const ActQ8& a,
+__device__ inline void silu_q8_block(const float* gate, const float* up, int b, const RowAct& a,
                                      float* sx, float* wmax) {
     const int e = threadIdx.x;
     const bool on = e < 256;
-    const int nb = a.cols / 256;
     float v = 0.0f;
     if (on) {
         const size_t idx = (size_t)b * 256 + e;
@@ -460,7 +462,6 @@ __device__ inline void silu_q8_block(const float* gate, const float* up, int b, 
         const float a0 = s8[0] + s8[4], a1 = s8[1] + s8[5], a2 = s8[2] + s8[6], a3 = s8[3] + s8[7];
         a.xs16[(size_t)b * 16 + gi] = (a0 + a1) + (a2 + a3);
     }
-    (void)nb;
 }
 
 // Direct global->LDS copies issued from inline assembly.  The compiler does
