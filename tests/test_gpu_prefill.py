@@ -171,11 +171,13 @@ def test_small_batch_wide_rows(hip, p):
     assert_bits(w.matvec_batch(xs), amd64(data, xs, rows, cols), f"{rows}x{cols} p={p}")
 
 
-def test_small_batch_few_rows_past_4_gib(hip):
+@pytest.mark.parametrize("p", [6, 9])
+def test_small_batch_few_rows_past_4_gib(hip, p):
     """8192 rows of 512 KB: a weight of 4 GiB with too few rows for the 64 x 16
-    tiles to cover the GPU still runs on them."""
+    tiles to cover the GPU still runs on them, and on the row kernel below 8
+    tokens."""
     import torch
-    rows, cols, p = 32, 256 * 3641, 9
+    rows, cols = 32, 256 * 3641
     data, _ = quant_matrix(ref.Q4_K, rows, cols, 982)
     times = 8192 // rows
     raw = torch.from_numpy(data).cuda().repeat(times)
